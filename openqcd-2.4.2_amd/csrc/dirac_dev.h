@@ -9,6 +9,24 @@
 
 namespace oqh {
 
+// Work-groups are dispatched round-robin over the 8 XCDs of the chip, each
+// with its own L2.  The tile of work-group b: with C > 0 each XCD takes runs
+// of C consecutive tiles (C = 1 is the plain dispatch order), with C = 0 one
+// contiguous range of tiles.  Consecutive tiles are neighbours within a
+// thread block of the site order, so a run shares its face lines in one L2.
+__device__ inline int xcd_tile(int b, int nb, int C)
+{
+   if (C == 0)
+   {
+      int q = nb >> 3, r = nb & 7, j = b & 7;
+      return j * q + min(j, r) + (b >> 3);
+   }
+   const int span = 8 * C;
+   if (C <= 1 || b >= nb / span * span) return b;
+   const int g = b / span, rr = b % span;
+   return g * span + (rr & 7) * C + (rr >> 3);
+}
+
 template <typename C> __device__ inline void load_spinor(const C *f, int y, C *s)
 {
    const C *p = f + (size_t)(y >> 6) * (12 * SB) + (y & (SB - 1));

@@ -7,17 +7,13 @@
 //
 // The reference visits the points x and planes (mu,nu) and adds the
 // traceless antihermitian part of each plaquette, started at each of its
-// four links, to the force on that link.  Here one lane per link gathers the
-// six plaquettes that contain its link (two per plane), computing every term
-// with the same products and the same association as the reference:
+// four links, to the force on that link.  Here one lane per link sums the six
+// staples of its link and projects once (k_flow),
 //
-//   plaquette at b in plane (mu,nu):  U0=U(b,mu) U1=U(b+mu,nu) U2=U(b,nu)
-//   U3=U(b+nu,mu);  F(U0) += P(U0 (U1 U3^+) U2^+),  F(U2) -= the same,
-//   F(U1) += P((U1 U3^+)(U2^+ U0)),  F(U3) -= P((U2^+ U0)(U1 U3^+))
+//   F(U) = P(U S),  P(w) = (w - w^+)/2 - tr(w - w^+)/6
 //
-// with P(w) = (w - w^+)/2 - tr(w - w^+)/6 expressed in the 8 real components
-// of su3_alg_dble.  Only the order in which the six terms of a link are added
-// differs from the reference, so forces agree to rounding.  Open boundary
+// in the 8 real components of su3_alg_dble; forces agree with the reference's
+// sum over plaquettes to rounding.  Open boundary
 // conditions (type 0): time-like plaquettes at x0 = N0-1 are omitted and the
 // space-like plaquettes on the boundary slices carry weight 1/2
 // (force0.c:226-274); the update multiplies the step of the space-like links
@@ -28,6 +24,7 @@
 // point in the site-block layout of the gauge field (link l: units 4l..4l+3).
 #include <cfloat>
 #include <cmath>
+#include <utility>
 
 #include "dirac_dev.h"
 #include "ddsum.h"
@@ -41,9 +38,9 @@ struct Su3
    double2 e[9];
 };
 
-// all products are evaluated without contraction, in the order of the
-// reference's macros (include/su3.h:416-463), so that every plaquette term
-// is the reference's value
+// the plaquette sums, the projection and the exponential are evaluated
+// without contraction, in the order of the reference's macros
+// (include/su3.h:416-463)
 #pragma clang fp contract(off)
 
 __device__ inline double2 dot_row(const double2 *a, const double2 *s)
@@ -51,15 +48,6 @@ __device__ inline double2 dot_row(const double2 *a, const double2 *s)
    // sum_k a_k s_k, left to right as _su3_multiply
    double re = a[0].x * s[0].x - a[0].y * s[0].y + a[1].x * s[1].x - a[1].y * s[1].y + a[2].x * s[2].x - a[2].y * s[2].y;
    double im = a[0].x * s[0].y + a[0].y * s[0].x + a[1].x * s[1].y + a[1].y * s[1].x + a[2].x * s[2].y + a[2].y * s[2].x;
-   return make_double2(re, im);
-}
-
-__device__ inline double2 dot_col_dag(const double2 *u, int i, const double2 *s)
-{
-   // (u^+ s)_i, as _su3_inverse_multiply
-   const double2 a0 = u[i], a1 = u[3 + i], a2 = u[6 + i];
-   double re = a0.x * s[0].x + a0.y * s[0].y + a1.x * s[1].x + a1.y * s[1].y + a2.x * s[2].x + a2.y * s[2].y;
-   double im = a0.x * s[0].y - a0.y * s[0].x + a1.x * s[1].y - a1.y * s[1].x + a2.x * s[2].y - a2.y * s[2].x;
    return make_double2(re, im);
 }
 
@@ -71,36 +59,6 @@ __device__ inline Su3 mul(const Su3 &u, const Su3 &v)
    for (int j = 0; j < 3; j++)
    {
       double2 p[3] = {v.e[j], v.e[3 + j], v.e[6 + j]};
-#pragma unroll
-      for (int i = 0; i < 3; i++) w.e[3 * i + j] = dot_row(u.e + 3 * i, p);
-   }
-   return w;
-}
-
-// w = u^+ v
-__device__ inline Su3 dag_mul(const Su3 &u, const Su3 &v)
-{
-   Su3 w;
-#pragma unroll
-   for (int j = 0; j < 3; j++)
-   {
-      double2 p[3] = {v.e[j], v.e[3 + j], v.e[6 + j]};
-#pragma unroll
-      for (int i = 0; i < 3; i++) w.e[3 * i + j] = dot_col_dag(u.e, i, p);
-   }
-   return w;
-}
-
-// w = u v^+
-__device__ inline Su3 mul_dag(const Su3 &u, const Su3 &v)
-{
-   Su3 w;
-#pragma unroll
-   for (int j = 0; j < 3; j++)
-   {
-      double2 p[3];
-#pragma unroll
-      for (int k = 0; k < 3; k++) p[k] = make_double2(v.e[3 * j + k].x, -v.e[3 * j + k].y);
 #pragma unroll
       for (int i = 0; i < 3; i++) w.e[3 * i + j] = dot_row(u.e + 3 * i, p);
    }
@@ -146,8 +104,6 @@ __device__ inline void prod2alg(const Su3 &u, const Su3 &v, double *X)
 struct FArgs
 {
    const double2 *ud;
-   double2 *u_w;     // gauge field written by the update
-   double2 *frc;     // 32 units per odd point
    const int *nbr;   // [8][V], bit 31 flags boundary points
    const int *x0;
    int V, h, N0, bc;
@@ -179,12 +135,6 @@ __device__ inline Su3 link_at(const FArgs &a, int z, int d)
 __device__ inline int up(const FArgs &a, int z, int d) { return a.nbr[(size_t)(2 * d) * a.V + z] & 0x7fffffff; }
 __device__ inline int dn(const FArgs &a, int z, int d) { return a.nbr[(size_t)(2 * d + 1) * a.V + z] & 0x7fffffff; }
 
-__device__ inline void acc8(double *F, const double *X, double r)
-{
-#pragma unroll
-   for (int k = 0; k < 8; k++) F[k] += r * X[k];
-}
-
 // the planes (mu,nu) of force0.c / uidx.c:70 in their orientation
 __device__ inline int plane_n(int a, int b)
 {
@@ -203,94 +153,15 @@ __device__ inline void plane_pq(int n, int &p, int &q)
    q = Q[n];
 }
 
-// weights of a plaquette with base point time t (force0.c:221-274); returns
-// false if the plaquette does not contribute; *w1 tells whether the term of
-// its link U1 is taken
-__device__ inline bool plaq_weight(const FArgs &a, int n, int t, double *r, bool *w1)
+// weight of a plaquette with base point time t (force0.c:221-274); 0 if the
+// plaquette does not contribute
+__device__ inline double plaq_weight(const FArgs &a, int n, int t)
 {
-   *w1 = true;
-   *r = 1.0;
-   if (n < 3)
-   {
-      if (!(t < a.N0 - 1 || a.bc != 0)) return false;
-      *w1 = (t < a.N0 - 1 || a.bc == 3);
-      return true;
-   }
-   if ((t == 0 && a.bc != 3) || (t == a.N0 - 1 && a.bc == 0)) *r = 0.5;
-   return true;
+   if (n < 3) return (t < a.N0 - 1 || a.bc != 0) ? 1.0 : 0.0;
+   return ((t == 0 && a.bc != 3) || (t == a.N0 - 1 && a.bc == 0)) ? 0.5 : 1.0;
 }
 
 }  // namespace
-
-// one lane per link: link (odd point o, slot l); its base point is o for
-// even l and o - mu for odd l
-__global__ __launch_bounds__(256) void k_plaq_frc(FArgs a)
-{
-   int k = blockIdx.x * 256 + threadIdx.x;
-   if (k >= 4 * a.V) return;
-   int j = k >> 3, l = k & 7;
-   int o = a.h + j, mu = l >> 1;
-   int y = (l & 1) ? dn(a, o, mu) : o;
-   double F[8] = {0, 0, 0, 0, 0, 0, 0, 0}, X[8];
-   Su3 Ul = link_at(a, y, mu);
-   for (int nu = 0; nu < 4; nu++)
-   {
-      if (nu == mu) continue;
-      int n = plane_n(mu, nu), p, q;
-      plane_pq(n, p, q);
-      double r;
-      bool w1;
-      if (mu == p)
-      {
-         // (i) base y: the link is U0
-         int b = y;
-         if (plaq_weight(a, n, a.x0[b], &r, &w1))
-         {
-            Su3 U1 = link_at(a, up(a, b, p), q), U2 = link_at(a, b, q), U3 = link_at(a, up(a, b, q), p);
-            Su3 w0 = mul_dag(U1, U3);
-            Su3 w2 = mul_dag(w0, U2);
-            prod2alg(Ul, w2, X);
-            acc8(F, X, r);
-         }
-         // (ii) base y - q: the link is U3
-         b = dn(a, y, q);
-         if (plaq_weight(a, n, a.x0[b], &r, &w1))
-         {
-            Su3 U0 = link_at(a, b, p), U1 = link_at(a, up(a, b, p), q), U2 = link_at(a, b, q);
-            Su3 w0 = mul_dag(U1, Ul);
-            Su3 wb = dag_mul(U2, U0);
-            prod2alg(wb, w0, X);
-            acc8(F, X, -r);
-         }
-      }
-      else
-      {
-         // (iii) base y: the link is U2 (terms with t = 0 of SF bc excluded)
-         int b = y;
-         if (plaq_weight(a, n, a.x0[b], &r, &w1))
-         {
-            Su3 U0 = link_at(a, b, p), U1 = link_at(a, up(a, b, p), q), U3 = link_at(a, up(a, b, q), p);
-            Su3 w0 = mul_dag(U1, U3);
-            Su3 w2 = mul_dag(w0, Ul);
-            prod2alg(U0, w2, X);
-            acc8(F, X, -r);
-         }
-         // (iv) base y - p: the link is U1
-         b = dn(a, y, p);
-         if (plaq_weight(a, n, a.x0[b], &r, &w1) && w1)
-         {
-            Su3 U0 = link_at(a, b, p), U2 = link_at(a, b, q), U3 = link_at(a, up(a, b, q), p);
-            Su3 w0 = mul_dag(Ul, U3);
-            Su3 wb = dag_mul(U2, U0);
-            prod2alg(w0, wb, X);
-            acc8(F, X, r);
-         }
-      }
-   }
-   double2 *f = a.frc + (size_t)(j >> 6) * (32 * SB) + (j & (SB - 1)) + (size_t)(4 * l) * SB;
-#pragma unroll
-   for (int c = 0; c < 4; c++) f[c * SB] = make_double2(F[2 * c], F[2 * c + 1]);
-}
 
 // ---- plaquette sums (uflds/plaq_sum.c:69-175) ----
 
@@ -464,13 +335,143 @@ __device__ inline void exp_update(double eps, const double *X, Su3 &u, const Che
 
 }  // namespace
 
-// one lane per link of the odd points: update rules of wflow.c:96-144
-__global__ __launch_bounds__(256) void k_update_ud(FArgs a, ChexpCoef cc)
+// ---- force and flow step ----
+//
+// One lane per link, the wave's 64 lanes being the 64 odd points of one
+// storage block and the slot l of the link the same for all of them, so that
+// every link of a staple is read as whole lines and no lane takes another
+// branch.  The force on U = U(y,mu) is P(U S) with the sum S of the six
+// staples
+//
+//    U(y+mu,nu) U(y+nu,mu)^+ U(y,nu)^+  and  U(y+mu-nu,nu)^+ U(y-nu,mu)^+ U(y-nu,nu),
+//
+// 13 products of 3x3 matrices instead of the 18 of the separate plaquette
+// terms.  Links are stored with odd points: besides the two links at the
+// link's own point o, each staple pair reads two links at each of the odd
+// points p1 (o + mu + nu or o - mu + nu) and p2 (the same with -nu).
+// In a flow step the new link exp(X) U goes to a second gauge field, which
+// saves writing and reading the force (512 bytes per point and step) and the
+// second launch; the fields change places after the step.
+// What bounds it: the 18 links read per link, 3.8 GB through the caches at
+// 24^4, of which 1.4 GB miss the 4 MB L2 of an XCD (the faces of an 8^4
+// thread block lie scattered over the lines).  A step at 24^4 takes 0.35 ms
+// against 0.79 ms for one kernel with a lane per link in slot order (uneven
+// branches, lines shared by 8 lanes only), which stored the force, and one
+// that applied it.
+
+struct FlowOut
 {
-   int k = blockIdx.x * 256 + threadIdx.x;
-   if (k >= 4 * a.V) return;
-   int j = k >> 3, l = k & 7, o = a.h + j;
-   int t = a.x0[o];
+   double2 *ud;   // new gauge field (flow step) or null (force only)
+   double2 *frc;  // force field or null
+};
+
+namespace {
+
+__device__ inline void load_su3(const double2 *p, Su3 &u)
+{
+#pragma unroll
+   for (int k = 0; k < 9; k++) u.e[k] = p[k * SB];
+}
+
+// S += w V
+__device__ inline void acc_su3(Su3 &S, const Su3 &V, double w)
+{
+#pragma unroll
+   for (int k = 0; k < 9; k++) S.e[k] = make_double2(fma(w, V.e[k].x, S.e[k].x), fma(w, V.e[k].y, S.e[k].y));
+}
+
+// w += a b, w += conj(a) b, w += a conj(b)
+__device__ inline void fma_nn(double2 &w, double2 a, double2 b)
+{
+   w = make_double2(fma(a.x, b.x, fma(-a.y, b.y, w.x)), fma(a.x, b.y, fma(a.y, b.x, w.y)));
+}
+__device__ inline void fma_dn(double2 &w, double2 a, double2 b)
+{
+   w = make_double2(fma(a.x, b.x, fma(a.y, b.y, w.x)), fma(a.x, b.y, fma(-a.y, b.x, w.y)));
+}
+__device__ inline void fma_nd(double2 &w, double2 a, double2 b)
+{
+   w = make_double2(fma(a.x, b.x, fma(a.y, b.y, w.x)), fma(a.y, b.x, fma(-a.x, b.y, w.y)));
+}
+
+// products as FMA chains: u v, u^+ v, u v^+
+template <int KIND> __device__ inline Su3 fmul(const Su3 &u, const Su3 &v)
+{
+   Su3 w;
+#pragma unroll
+   for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+      {
+         double2 z = make_double2(0.0, 0.0);
+#pragma unroll
+         for (int k = 0; k < 3; k++)
+         {
+            if (KIND == 0) fma_nn(z, u.e[3 * i + k], v.e[3 * k + j]);
+            if (KIND == 1) fma_dn(z, u.e[3 * k + i], v.e[3 * k + j]);
+            if (KIND == 2) fma_nd(z, u.e[3 * i + k], v.e[3 * j + k]);
+         }
+         w.e[3 * i + j] = z;
+      }
+   return w;
+}
+
+}  // namespace
+
+template <bool STEP>
+__global__ __launch_bounds__(256) void k_flow(FArgs a, ChexpCoef cc, FlowOut out)
+{
+   // two work-groups (slots 0-3, 4-7) per storage block; consecutive storage
+   // blocks stay on one XCD
+   const int g = xcd_tile(blockIdx.x, gridDim.x, 0);
+   const int l = __builtin_amdgcn_readfirstlane((g & 1) * 4 + (threadIdx.x >> 6));
+   const int j = (g >> 1) * SB + (threadIdx.x & (SB - 1));
+   if (j >= a.h) return;
+   const int mu = l >> 1, o = a.h + j;
+   const bool base_odd = !(l & 1);  // base point y = o, or o - mu
+   const int m = base_odd ? up(a, o, mu) : dn(a, o, mu);  // y + mu, or y
+   const double2 *own = link_ptr(a.ud, j, 0);
+   Su3 S;
+#pragma unroll
+   for (int k = 0; k < 9; k++) S.e[k] = make_double2(0.0, 0.0);
+   const int tb = (a.bc != 3) ? a.x0[base_odd ? o : m] : 0;
+   for (int i = 1; i < 4; i++)
+   {
+      const int nu = (mu + i) & 3;
+      const double2 *p1 = link_ptr(a.ud, up(a, m, nu) - a.h, 0), *p2 = link_ptr(a.ud, dn(a, m, nu) - a.h, 0);
+      double r1 = 1.0, r2 = 1.0;
+      if (a.bc != 3)
+      {
+         // weights of the plaquettes with base points y and y - nu
+         const int n = plane_n(mu, nu);
+         const int td = nu == 0 ? (tb == 0 ? a.N0 - 1 : tb - 1) : tb;
+         r1 = plaq_weight(a, n, tb);
+         r2 = plaq_weight(a, n, td);
+      }
+      // the links of the staples by their slots
+      Su3 A, B, C;
+      load_su3(base_odd ? own + (size_t)(9 * 2 * nu) * SB : p1 + (size_t)(9 * (2 * nu + 1)) * SB, A);  // U(y,nu)
+      load_su3(p1 + (size_t)(9 * (base_odd ? 2 * mu + 1 : 2 * mu)) * SB, B);                          // U(y+nu,mu)
+      load_su3(base_odd ? p1 + (size_t)(9 * (2 * nu + 1)) * SB : own + (size_t)(9 * 2 * nu) * SB, C);  // U(y+mu,nu)
+      acc_su3(S, fmul<2>(C, fmul<0>(A, B)), r1);
+      load_su3(p2 + (size_t)(9 * (base_odd ? 2 * mu + 1 : 2 * mu)) * SB, A);                          // U(y-nu,mu)
+      load_su3(base_odd ? p2 + (size_t)(9 * 2 * nu) * SB : own + (size_t)(9 * (2 * nu + 1)) * SB, B);  // U(y+mu-nu,nu)
+      load_su3(base_odd ? own + (size_t)(9 * (2 * nu + 1)) * SB : p2 + (size_t)(9 * 2 * nu) * SB, C);  // U(y-nu,nu)
+      acc_su3(S, fmul<1>(fmul<0>(A, B), C), r2);
+   }
+   Su3 U;
+   load_su3(own + (size_t)(9 * l) * SB, U);
+   double F[8];
+   prod2alg(U, S, F);
+   if (out.frc)
+   {
+      double2 *f = out.frc + (size_t)(j >> 6) * (32 * SB) + (j & (SB - 1)) + (size_t)(4 * l) * SB;
+#pragma unroll
+      for (int c = 0; c < 4; c++) f[c * SB] = make_double2(F[2 * c], F[2 * c + 1]);
+   }
+   if (!STEP) return;
+   // update rules of wflow.c:96-144
+   const int t = a.x0[o];
    double e = a.eps;
    bool upd = true;
    if (t == 0)
@@ -487,23 +488,10 @@ __global__ __launch_bounds__(256) void k_update_ud(FArgs a, ChexpCoef cc)
       else if (l >= 2 && a.bc == 0)
          e = 2.0 * a.eps;
    }
-   if (!upd) return;
-   const double2 *f = a.frc + (size_t)(j >> 6) * (32 * SB) + (j & (SB - 1)) + (size_t)(4 * l) * SB;
-   double X[8];
+   if (upd) exp_update(e, F, U, cc);
+   double2 *un = out.ud + (size_t)(j >> 6) * (72 * SB) + (j & (SB - 1)) + (size_t)(9 * l) * SB;
 #pragma unroll
-   for (int c = 0; c < 4; c++)
-   {
-      double2 v = f[c * SB];
-      X[2 * c] = v.x;
-      X[2 * c + 1] = v.y;
-   }
-   double2 *up = a.u_w + (size_t)(j >> 6) * (72 * SB) + (j & (SB - 1)) + (size_t)(9 * l) * SB;
-   Su3 u;
-#pragma unroll
-   for (int c = 0; c < 9; c++) u.e[c] = up[c * SB];
-   exp_update(e, X, u, cc);
-#pragma unroll
-   for (int c = 0; c < 9; c++) up[c * SB] = u.e[c];
+   for (int c = 0; c < 9; c++) un[c * SB] = U.e[c];
 }
 
 // time-like links at x0 = N0-1 times -1 (periodic bc: antiperiodic quarks)
@@ -536,15 +524,15 @@ static ChexpCoef chexp_coef()
    return cc;
 }
 
-static double2 *d_frc = nullptr;
-static size_t frc_bytes = 0;
+static double2 *d_frc = nullptr;   // force of the last plaq_frc() or flow step
+static double2 *d_ud2 = nullptr;   // second gauge field of the flow steps
+static size_t frc_bytes = 0, ud2_bytes = 0;
 
-static FArgs fargs(bool need_frc = true)
+static FArgs fargs()
 {
    Lib &L = lib();
    FArgs a;
    a.ud = L.d_ud;
-   a.u_w = L.d_ud;
    a.nbr = L.d_nbr;
    a.x0 = L.d_x0;
    a.V = L.g.V;
@@ -552,18 +540,24 @@ static FArgs fargs(bool need_frc = true)
    a.N0 = L.g.L[0];
    a.bc = L.bc;
    a.eps = 0.0;
-   a.frc = nullptr;
-   if (!need_frc) return a;
-   size_t need = units_for(a.h, 32) * sizeof(double2);
-   if (need > frc_bytes)
-   {
-      dev_free(d_frc);
-      d_frc = (double2 *)dev_alloc(need);
-      frc_bytes = d_frc ? need : 0;
-   }
-   a.frc = d_frc;
    return a;
 }
+
+static double2 *flow_buffer(double2 *&p, size_t &have, int nc)
+{
+   Lib &L = lib();
+   const size_t need = units_for(L.g.V / 2, nc) * sizeof(double2);
+   if (need > have)
+   {
+      dev_free(p);
+      p = (double2 *)dev_alloc(need);
+      have = p ? need : 0;
+      if (p) HIP_OK(hipMemsetAsync(p, 0, need, L.stream));
+   }
+   return p;
+}
+
+static unsigned flow_blocks(const FArgs &a) { return 2u * (unsigned)((a.h + SB - 1) / SB); }
 
 static bool flow_ready(const char *where)
 {
@@ -580,8 +574,9 @@ static bool flow_ready(const char *where)
 void release_flow()
 {
    dev_free(d_frc);
-   d_frc = nullptr;
-   frc_bytes = 0;
+   dev_free(d_ud2);
+   d_frc = d_ud2 = nullptr;
+   frc_bytes = ud2_bytes = 0;
 }
 
 }  // namespace oqh
@@ -593,9 +588,9 @@ extern "C" void plaq_frc(void)
    Lib &L = lib();
    if (!flow_ready("plaq_frc [force0.c]")) return;
    FArgs a = fargs();
-   if (!a.frc) return;
-   unsigned nb = (unsigned)((4 * (size_t)a.V + 255) / 256);
-   k_plaq_frc<<<nb, 256, 0, L.stream>>>(a);
+   FlowOut out = {nullptr, flow_buffer(d_frc, frc_bytes, 32)};
+   if (!out.frc) return;
+   k_flow<false><<<flow_blocks(a), 256, 0, L.stream>>>(a, chexp_coef(), out);
    HIP_OK(hipStreamSynchronize(L.stream));
 }
 
@@ -616,14 +611,17 @@ extern "C" void fwd_euler(int n, double eps)
    Lib &L = lib();
    if (!flow_ready("fwd_euler [wflow.c]") || n <= 0) return;
    FArgs a = fargs();
-   if (!a.frc) return;
-   ChexpCoef cc = chexp_coef();
-   unsigned nb = (unsigned)((4 * (size_t)a.V + 255) / 256);
+   double2 *frc = flow_buffer(d_frc, frc_bytes, 32);
+   if (!frc || !flow_buffer(d_ud2, ud2_bytes, 72)) return;
+   const ChexpCoef cc = chexp_coef();
    a.eps = -eps;
    for (int k = 0; k < n; k++)
    {
-      k_plaq_frc<<<nb, 256, 0, L.stream>>>(a);
-      k_update_ud<<<nb, 256, 0, L.stream>>>(a, cc);
+      // the force of the last step stays readable (oqh_export_frc)
+      const FlowOut out = {d_ud2, k == n - 1 ? frc : nullptr};
+      a.ud = L.d_ud;
+      k_flow<true><<<flow_blocks(a), 256, 0, L.stream>>>(a, cc, out);
+      std::swap(L.d_ud, d_ud2);
    }
    HIP_OK(hipStreamSynchronize(L.stream));
    L.ud_version++;
@@ -676,7 +674,7 @@ static double plaq_sum(double wp, const char *where)
    if (!d_part) d_part = (dd *)dev_alloc(sizeof(dd) * (nbmax + 1));
    if (!h_out) HIP_OK(hipHostMalloc((void **)&h_out, sizeof(dd), 0));
    if (!d_part || !h_out) return 0.0;
-   FArgs a = oqh::fargs(false);
+   FArgs a = oqh::fargs();
    int nb = (a.V + 255) / 256;
    nb = nb > nbmax ? nbmax : nb;
    oqh::k_plaq_partial<<<nb, 256, 0, L.stream>>>(a, wp, d_part);
