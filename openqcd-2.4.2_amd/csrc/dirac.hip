@@ -300,6 +300,20 @@ template <typename C> __device__ inline void store_out(C *f, int y, const C *s)
       store_spinor(f, y, s);
 }
 
+// barrier between the lanes of a tile: a tile of 64 lanes is one wavefront,
+// whose LDS accesses are in order; the fence keeps the compiler from moving
+// them
+template <int TP> __device__ inline void tile_sync()
+{
+   if (TP > 64)
+      __syncthreads();
+   else
+   {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+   }
+}
+
 // OWN: the odd lane adds its own hopping term (from the even neighbour, S or
 // global a.s) to acc_o; XCH: the odd lane passes the term of its even
 // neighbour through X, and even lanes gather the terms of neighbours outside
@@ -353,7 +367,7 @@ __device__ inline void tile_phase(const DArgs<T> &a, int t, int e0, bool valid, 
       }
    }
    if (!XCH) return;
-   __syncthreads();
+   tile_sync<TP>();
    // even point e: neighbour z = e -+ mu (odd), the opposite direction
    if (valid)
    {
@@ -388,7 +402,7 @@ __device__ inline void tile_phase(const DArgs<T> &a, int t, int e0, bool valid, 
    // with a single exchange buffer the next phase may overwrite it only
    // after every lane has read it; with two buffers the next phase's barrier
    // gives that order
-   if (XBUF == 1) __syncthreads();
+   if (XBUF == 1) tile_sync<TP>();
 }
 
 // diagonal constant of the SW term at point x (sw_term.c:293-309)
@@ -403,24 +417,23 @@ template <typename T> __device__ inline T sw_const(const DArgs<T> &a, int x)
 }
 
 // (A + i mu) v at point x from the Pauli field or from the S-form
-template <typename T, bool SWS>
+template <typename T, bool SWS, bool NT = OQH_NT_SW>
 __device__ inline void site_term(const DArgs<T> &a, int x, T mu, const typename cplx_of<T>::t *v,
                                  typename cplx_of<T>::t *out)
 {
    if (SWS)
-      sws_site<typename cplx_of<T>::t, OQH_NT_SW>(a.sws, x, sw_const(a, x), mu, v, out);
+      sws_site<typename cplx_of<T>::t, NT>(a.sws, x, sw_const(a, x), mu, v, out);
    else
-      pauli_site<typename cplx_of<T>::t, OQH_NT_SW>(a.sw, x, mu, v, out);
+      pauli_site<typename cplx_of<T>::t, NT>(a.sw, x, mu, v, out);
 }
 
-template <typename T, int TP = TileSize<T>::n, bool REC = false, bool SWS = false>
-__global__ __launch_bounds__(TP) void k_dw_tile(DArgs<T> a)
+// one tile, lane t < TP (a.s_w null: the input is left unchanged on the
+// boundary points; NT: the SW matrices are used once)
+template <typename T, int TP, bool REC, bool SWS, bool NT = OQH_NT_SW>
+__device__ inline void dw_tile(const DArgs<T> &a, int t, int e0, typename cplx_of<T>::t (*S)[TP],
+                               typename cplx_of<T>::t (*X)[6][TP])
 {
    typedef typename cplx_of<T>::t C;
-   __shared__ C S[12][TP];
-   __shared__ C X[XBUF][6][TP];
-   const int t = threadIdx.x;
-   const int e0 = xcd_tile(blockIdx.x, gridDim.x, a.xcdc) * TP;
    const int e = e0 + t, o = a.h + e;
    const bool valid = e < a.h;
    bool eb = false, ob = false;
@@ -457,7 +470,7 @@ __global__ __launch_bounds__(TP) void k_dw_tile(DArgs<T> a)
       for (int c = 0; c < 12; c++) S[c][t] = se[c];
       if (!ob) load_spinor(a.s, o, so);
    }
-   __syncthreads();
+   tile_sync<TP>();
    tile_phase<T, 0, true, TP, true, true, REC>(a, t, e0, valid, nb, S, X[0], so, acc_o, acc_e, a.s);
    tile_phase<T, 0, false, TP, true, true, REC>(a, t, e0, valid, nb, S, X[XBUF - 1], so, acc_o, acc_e, a.s);
    tile_phase<T, 1, true, TP, true, true, REC>(a, t, e0, valid, nb, S, X[0], so, acc_o, acc_e, a.s);
@@ -472,11 +485,11 @@ __global__ __launch_bounds__(TP) void k_dw_tile(DArgs<T> a)
    if (ob)
    {
       zero_spinor(a.r, o);
-      zero_spinor(a.s_w, o);
+      if (a.s_w) zero_spinor(a.s_w, o);
    }
    else
    {
-      site_term<T, SWS>(a, o, a.muo, so, out);
+      site_term<T, SWS, NT>(a, o, a.muo, so, out);
 #pragma unroll
       for (int c = 0; c < 12; c++) out[c] = cadd(out[c], cscale(acc_o[c], a.coef));
       store_out(a.r, o, out);
@@ -484,18 +497,27 @@ __global__ __launch_bounds__(TP) void k_dw_tile(DArgs<T> a)
    if (eb)
    {
       zero_spinor(a.r, e);
-      zero_spinor(a.s_w, e);
+      if (a.s_w) zero_spinor(a.s_w, e);
    }
    else
    {
       C se[12];
 #pragma unroll
       for (int c = 0; c < 12; c++) se[c] = S[c][t];
-      site_term<T, SWS>(a, e, a.mu, se, out);
+      site_term<T, SWS, NT>(a, e, a.mu, se, out);
 #pragma unroll
       for (int c = 0; c < 12; c++) out[c] = cadd(out[c], cscale(acc_e[c], a.coef));
       store_out(a.r, e, out);
    }
+}
+
+template <typename T, int TP = TileSize<T>::n, bool REC = false, bool SWS = false>
+__global__ __launch_bounds__(TP) void k_dw_tile(DArgs<T> a)
+{
+   typedef typename cplx_of<T>::t C;
+   __shared__ C S[12][TP];
+   __shared__ C X[XBUF][6][TP];
+   dw_tile<T, TP, REC, SWS>(a, threadIdx.x, xcd_tile(blockIdx.x, gridDim.x, a.xcdc) * TP, S, X);
 }
 
 // Dwhat / Dwhat_dble in two tile passes (Dw_dble.c:1792-1888):
@@ -613,182 +635,45 @@ __global__ __launch_bounds__(TP) void k_hat2_tile(DArgs<T> a)
 }
 
 // ---------------------------------------------------------------------------
-// Dw / Dw_dble on several fields at once (no reference counterpart): the
-// tile kernel with NR lanes per even-odd pair, one per right-hand side.  The
-// NR lanes of a pair are adjacent in a wavefront and load the same links and
-// Pauli matrices, so each such load is fetched once for all right-hand sides;
-// the spinor staging and exchange are per right-hand side.
+// Dw / Dw_dble on several fields at once (no reference counterpart): tiles of
+// 64 even and 64 odd points, each worked on by one wavefront per field.  The
+// four wavefronts of a work-group take the same tile for four fields and
+// share its links and SW matrices through the L1, the groups of four follow
+// each other on one XCD and share them through its L2.  A wavefront exchanges
+// hopping terms with itself only, so there are no barriers.
+// 12 fields FP64 at 24^4: 0.83 ms against 1.11 ms with 8 lanes per pair of
+// points, 256-lane work-groups and barriers.  Bound by the 4.9 GB that miss
+// the L2 (the neighbours in x2 and x3 lie four to eight lines apart).  Two
+// fields per work-group: 0.85 ms; all tiles of a thread block for four fields
+// before the next four: 0.90 ms; third link rows rebuilt and the S-form of
+// the SW term, as Dw_dble has them: 0.80 ms, but twice the rounding error
+// (3e-16 for 1.3e-16), so the stored links are read.
 // ---------------------------------------------------------------------------
 
-constexpr int NRMAX = 8;
+constexpr int MTP = 64;    // pairs of points per tile
+constexpr int MWV = 4;     // fields per work-group
+constexpr int NRMAX = 16;  // fields per launch
 
-template <typename T> struct MArgs
+template <typename T> struct MFields
 {
    typedef typename cplx_of<T>::t C;
    const C *s[NRMAX];
    C *r[NRMAX];
-   const C *u, *sw;
-   const int *nbr;
-   const unsigned char *bnd;
-   int V, h, n;  // n: number of fields of this launch
-   T mu, muo, coef;
-   int masked;
-   int xcdc;     // tiles per XCD run (xcd_tile; 0: one contiguous range per XCD)
+   int n, ng;  // fields, groups of MWV fields
 };
 
-template <typename T, int MU, bool FWD, int TPP, int NR>
-__device__ inline void multi_phase(const MArgs<T> &a, int t, int p, int k, int e0, bool valid, const int *nb,
-                                   typename cplx_of<T>::t (*S)[TPP * NR], typename cplx_of<T>::t (*X)[TPP * NR],
-                                   const typename cplx_of<T>::t *sk, const typename cplx_of<T>::t *so,
-                                   typename cplx_of<T>::t *acc_o, typename cplx_of<T>::t *acc_e)
+template <typename T> __global__ __launch_bounds__(MWV * 64) void k_dw_multi(DArgs<T> a, MFields<T> f)
 {
    typedef typename cplx_of<T>::t C;
-   const int e = e0 + p;
-   if (valid)
-   {
-      int ny = nb[2 * MU + (FWD ? 0 : 1)];
-      int y = ny & 0x7fffffff;
-      int ly = y - e0;
-      bool yin = (unsigned)ly < (unsigned)TPP;
-      const C *up = link_ptr(a.u, e, FWD ? 2 * MU : 2 * MU + 1);
-      C u[9];
-#pragma unroll
-      for (int q = 0; q < 9; q++) u[q] = up[q * SB];
-      C h0[3], h1[3], c0[3], c1[3];
-      if (!(a.masked && ny < 0))
-      {
-         C sy[12];
-         if (yin)
-         {
-#pragma unroll
-            for (int c = 0; c < 12; c++) sy[c] = S[c][ly * NR + k];
-         }
-         else
-            load_spinor(sk, y, sy);
-         spin_project<C, MU, FWD>(sy, h0, h1);
-         su3_mul<C, !FWD>(u, h0, c0);
-         su3_mul<C, !FWD>(u, h1, c1);
-         spin_expand_add<C, MU, FWD>(c0, c1, acc_o);
-      }
-      if (yin)
-      {
-         spin_project<C, MU, !FWD>(so, h0, h1);
-         su3_mul<C, FWD>(u, h0, c0);
-         su3_mul<C, FWD>(u, h1, c1);
-#pragma unroll
-         for (int c = 0; c < 3; c++)
-         {
-            X[c][ly * NR + k] = c0[c];
-            X[3 + c][ly * NR + k] = c1[c];
-         }
-      }
-   }
-   __syncthreads();
-   if (valid)
-   {
-      int nz = nb[8 + 2 * MU + (FWD ? 1 : 0)];
-      if (!(a.masked && nz < 0))
-      {
-         int z = nz & 0x7fffffff;
-         if ((unsigned)(z - a.h - e0) < (unsigned)TPP)
-         {
-            C c0[3], c1[3];
-#pragma unroll
-            for (int c = 0; c < 3; c++)
-            {
-               c0[c] = X[c][t];
-               c1[c] = X[3 + c][t];
-            }
-            spin_expand_add<C, MU, !FWD>(c0, c1, acc_e);
-         }
-         else
-         {
-            C sz[12];
-            load_spinor(sk, z, sz);
-            hop_one<C, MU, !FWD>(sz, link_ptr(a.u, z - a.h, FWD ? 2 * MU : 2 * MU + 1), acc_e);
-         }
-      }
-   }
-   __syncthreads();
-}
-
-template <typename T, int TPP, int NR>
-__global__ __launch_bounds__(TPP * NR) void k_dw_multi(MArgs<T> a)
-{
-   typedef typename cplx_of<T>::t C;
-   constexpr int NL = TPP * NR;
-   __shared__ C S[12][NL];
-   __shared__ C X[6][NL];
-   const int t = threadIdx.x, p = t / NR, k = t % NR;
-   const int e0 = xcd_tile(blockIdx.x, gridDim.x, a.xcdc) * TPP;
-   const int e = e0 + p, o = a.h + e;
-   const bool valid = e < a.h && k < a.n;
-   const C *sk = a.s[k < a.n ? k : 0];
-   C *rk = a.r[k < a.n ? k : 0];
-   bool eb = false, ob = false;
-   int nb[16];
-   C so[12], acc_o[12], acc_e[12];
-#pragma unroll
-   for (int c = 0; c < 12; c++)
-   {
-      acc_o[c] = cmk<C>(0, 0);
-      acc_e[c] = cmk<C>(0, 0);
-      so[c] = cmk<C>(0, 0);
-   }
-   if (valid)
-   {
-#pragma unroll
-      for (int q = 0; q < 8; q++)
-      {
-         nb[q] = a.nbr[(size_t)q * a.V + o];
-         nb[8 + q] = a.nbr[(size_t)q * a.V + e];
-      }
-      eb = a.masked && a.bnd[e];
-      ob = a.masked && a.bnd[o];
-      C se[12];
-      if (eb)
-      {
-#pragma unroll
-         for (int c = 0; c < 12; c++) se[c] = cmk<C>(0, 0);
-      }
-      else
-         load_spinor(sk, e, se);
-#pragma unroll
-      for (int c = 0; c < 12; c++) S[c][t] = se[c];
-      if (!ob) load_spinor(sk, o, so);
-   }
-   __syncthreads();
-   multi_phase<T, 0, true, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 0, false, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 1, true, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 1, false, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 2, true, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 2, false, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 3, true, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   multi_phase<T, 3, false, TPP, NR>(a, t, p, k, e0, valid, nb, S, X, sk, so, acc_o, acc_e);
-   if (!valid) return;
-   C out[12];
-   if (ob)
-      zero_spinor(rk, o);
-   else
-   {
-      pauli_site<C, OQH_NT_SW>(a.sw, o, a.muo, so, out);
-#pragma unroll
-      for (int c = 0; c < 12; c++) out[c] = cadd(out[c], cscale(acc_o[c], a.coef));
-      store_spinor(rk, o, out);
-   }
-   if (eb)
-      zero_spinor(rk, e);
-   else
-   {
-      C se[12];
-#pragma unroll
-      for (int c = 0; c < 12; c++) se[c] = S[c][t];
-      pauli_site<C, OQH_NT_SW>(a.sw, e, a.mu, se, out);
-#pragma unroll
-      for (int c = 0; c < 12; c++) out[c] = cadd(out[c], cscale(acc_e[c], a.coef));
-      store_spinor(rk, e, out);
-   }
+   __shared__ C S[MWV][12][MTP];
+   __shared__ C X[MWV][XBUF][6][MTP];
+   const int b = xcd_tile(blockIdx.x, gridDim.x, a.xcdc);
+   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int k = (b % f.ng) * MWV + w;
+   if (k >= f.n) return;
+   a.s = f.s[k];
+   a.r = f.r[k];
+   dw_tile<T, MTP, false, false, false>(a, threadIdx.x & 63, (b / f.ng) * MTP, S[w], X[w]);
 }
 
 template <typename T>
@@ -1140,15 +1025,7 @@ extern "C" void Dwhat(float mu, spinor *s, spinor *r) { apply<float>(K_HAT, mu, 
 
 namespace oqh {
 
-template <typename T, int NR> static void launch_multi(const MArgs<T> &a)
-{
-   constexpr int TPP = 256 / NR;
-   unsigned nt = (unsigned)((a.h + TPP - 1) / TPP);
-   if (nt) k_dw_multi<T, TPP, NR><<<nt, 256, 0, lib().stream>>>(a);
-}
-
-// n fields in chunks of up to NRMAX, each with the smallest power of two of
-// lanes per pair that holds it
+// n fields in launches of up to NRMAX
 template <typename T> static void apply_multi(T mu, int n, void **sp, void **rp, const char *where)
 {
    typedef typename cplx_of<T>::t C;
@@ -1160,24 +1037,18 @@ template <typename T> static void apply_multi(T mu, int n, void **sp, void **rp,
       fail(where, "the number of fields must be positive");
       return;
    }
-   MArgs<T> a{};
-   // runs of 32 tiles per XCD (measured at 32^3x64: 0.517 ms per field
-   // against 0.547 with one contiguous range per XCD; 2-128 within 2 %)
-   a.xcdc = 32;
-   a.u = (const C *)(sizeof(T) == 8 ? (const void *)L.d_ud : (const void *)L.d_u);
-   a.sw = (const C *)(sizeof(T) == 8 ? (const void *)L.d_swd : (const void *)L.d_sw);
-   a.nbr = L.d_nbr;
-   a.bnd = L.d_bnd;
-   a.V = L.g.V;
-   a.h = L.g.V / 2;
+   DArgs<T> a = base_args<T>();
    a.mu = mu;
    a.muo = L.eoflg ? (T)0 : mu;
    a.coef = (T)-0.5;
-   a.masked = (L.bc != 3);
+   const unsigned nt = (unsigned)((a.h + MTP - 1) / MTP);
    for (int k0 = 0; k0 < n; k0 += NRMAX)
    {
-      int m = (n - k0 < NRMAX) ? n - k0 : NRMAX;
-      for (int k = 0; k < m; k++)
+      MFields<T> f;
+      f.n = std::min(NRMAX, n - k0);
+      f.ng = (f.n + MWV - 1) / MWV;
+      a.xcdc = 16 * f.ng;  // runs of 16 tiles per XCD (2 tiles: 5 % slower, 32: 1 %)
+      for (int k = 0; k < f.n; k++)
       {
          int o1 = 0, o2 = 0;
          void *s = device_field(sp[k0 + k], prec, &o1), *r = device_field(rp[k0 + k], prec, &o2);
@@ -1191,18 +1062,11 @@ template <typename T> static void apply_multi(T mu, int n, void **sp, void **rp,
             fail(where, "Input and output fields must be different");
             return;
          }
-         a.s[k] = (const C *)s;
-         a.r[k] = (C *)r;
+         f.s[k] = (const C *)s;
+         f.r[k] = (C *)r;
       }
-      a.n = m;
-      if (m == 1)
-         launch_multi<T, 1>(a);
-      else if (m == 2)
-         launch_multi<T, 2>(a);
-      else if (m <= 4)
-         launch_multi<T, 4>(a);
-      else
-         launch_multi<T, 8>(a);
+      const unsigned nb = nt * f.ng;
+      k_dw_multi<T><<<nb, MWV * 64, 0, L.stream>>>(a, f);
    }
 }
 
