@@ -42,7 +42,7 @@
 
 namespace oqh {
 bool sap_prepare(int isolv, const char *where, bool quiet);
-void sap_device(float mu, int isolv, int nmr, float2 *psi, float2 *rho);
+void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho, bool zero, bool want_res);
 bool sap_mixed_mop(float mu, int isolv, int nmr, int ncy, const float2 *rho, float2 *phi, bool want_res);
 }
 
@@ -2239,8 +2239,7 @@ void dfl_mop_dev(const float2 *rho, float2 *phi, float2 *chi)
       Dw(R.mus, (spinor *)phi, (spinor *)chi);
       return;
    }
-   set_s2zero(vt, 2, (spinor *)phi);
-   for (int n = 0; n < R.ncy; n++) sap_device(R.mus, R.isolv, R.nmr, phi, r1);
+   sap_cycles(R.mus, R.isolv, R.nmr, R.ncy, phi, r1, true, true);
    // r1 = rho - D psi0 - D phi_sap, so chi = rho - r1 = D (psi0 + phi_sap)
    assign_s2s(vt, 2, (spinor *)r1, (spinor *)chi);
    diff_s2s(vt, 2, (spinor *)rho, (spinor *)chi);
@@ -2388,8 +2387,7 @@ void gen_cycles(float mus, int ncy, spinor *psi, spinor *r)
    int off = 0;
    float2 *p = (float2 *)device_field(psi, F32, &off), *rr = (float2 *)device_field(r, F32, &off);
    if (L.sap_prec == 1 && sap_mixed_mop(mus, 1, D.nmr, ncy, rr, p, false)) return;
-   set_s2zero(L.g.VT, 2, psi);
-   for (int j = 0; j < ncy; j++) sap_device(mus, 1, D.nmr, p, rr);
+   sap_cycles(mus, 1, D.nmr, ncy, p, rr, true, false);
 }
 
 // one deflated inverse-iteration step of every mode (dfl_smooth_fields):

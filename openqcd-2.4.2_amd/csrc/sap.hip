@@ -65,13 +65,16 @@ struct SapGrid
    bool need64 = false;                  // FP64 block operators in use: keep d_swb64
    __half2 *d_u16 = nullptr;             // FP16 links (FP16 variant of the solver)
    __half2 *d_swb16 = nullptr;           // FP16 block SW field
-   float2 *d_s0gm = nullptr;             // block corrections of 16 sources
+   float2 *d_wf = nullptr;               // face fields of the register kernel (one source)
+   float2 *d_wfm = nullptr;              // those of several sources
+   int wfm_n = 0;                        // number of sources in d_wfm
+   int *d_nbn = nullptr;                 // neighbouring blocks [nb][8] (4^4 blocks)
    double2 *d_swb64 = nullptr;           // FP64 block SW field (FP64 variant)
    int swb64_version = -1;
    double2 *d_h64[3] = {nullptr, nullptr, nullptr};  // FP64 psi, rho, s0g
    double2 *d_scr64 = nullptr;           // FP64 block fields [nbh][3][Ub]
-   __half2 *d_h16[3] = {nullptr, nullptr, nullptr};  // FP16 psi, rho, s0g
-   float *d_hsc[3] = {nullptr, nullptr, nullptr};    // their per-site scales
+   __half2 *d_h16[2] = {nullptr, nullptr};  // FP16 psi, rho
+   float *d_hsc[2] = {nullptr, nullptr};    // their per-site scales
    int u16_epoch = -1, swb16_epoch = -1; // versions they were made from
    int swb_version = 0;                  // incremented by every assign_swb
    std::vector<int> imb;                 // host copy
@@ -93,16 +96,19 @@ template <typename C> struct SArgsT
    size_t Ub;
    C *psi, *rho, *s0g, *scr;
    int n0;             // first block of the colour
-   // FP16 variant: psi, rho and s0g as FP16 spinors with per-site scales
-   __half2 *psi16, *rho16, *s0g16;
-   float *psc, *rsc, *s0sc;
+   // register kernel: face fields of the block corrections and neighbour
+   // blocks ([nb][8])
+   C *wf;
+   const int *nbn;
+   // FP16 variant: psi and rho as FP16 spinors with per-site scales
+   __half2 *psi16, *rho16;
+   float *psc, *rsc;
    int pz;             // psi is zero on entry (not read)
-   int pull;           // add the face terms from the other colour's s0g first
+   int pull;           // add the terms of the other colour's face fields first
    // several right-hand sides in one launch (FP32): nsrc > 0 replaces psi,
-   // rho, s0g by the fields of source blockIdx % nsrc (block kernel) or
-   // blockIdx.y (face kernel)
+   // rho, wf by the fields of source blockIdx % nsrc
    int nsrc;
-   C *pl[16], *rl[16], *sl[16];
+   C *pl[16], *rl[16], *wl[16];
 };
 typedef SArgsT<float2> SArgs;   // FP32 and FP16 variants
 typedef SArgsT<double2> SArgsD; // FP64 variant
@@ -504,21 +510,30 @@ __global__ __launch_bounds__(TPB) void k_sap_blocks(SArgsT<C> a)
 }
 
 // ---------------------------------------------------------------------------
-// the Schwarz sweep with the block held in registers (blocks of 256 points)
+// the Schwarz sweep with the block held in registers (blocks of 4^4 points)
 //
-// Lane x of the work-group owns block point x: its Pauli pair, the links
-// U(x,mu) to its in-block forward neighbours and the values of the block
-// fields s0, s1, s2 at x stay in registers for the whole block solve, so the
-// global memory is read once (links, SW, residual) and written once per
-// block.  A hopping pass exchanges only spinors: each lane puts its input
-// value into LDS (F), adds the forward terms of its neighbours x+mu from F and
-// computes with its own link the backward term of x+mu, which it passes
-// through LDS (X, two colour vectors after the spin projection).  The terms
-// are added in the order of blk_hop (mu = 0..3, forward then backward), so
-// the arithmetic is that of k_sap_blocks.
+// Lane x of the work-group owns block point x: its Pauli pair, its forward
+// links U(x,mu) and the values of the block fields at x stay in registers
+// for the whole block solve, so the global memory is read once (links, SW,
+// residual) and written once per block.  A hopping pass of one parity
+// exchanges only spinors: the lanes of the other parity (separate wavefronts)
+// put their values into LDS (F) and pass the backward terms, formed with
+// their own links, through LDS (X, two colour vectors after the spin
+// projection); the output lanes add the forward terms from F and the
+// backward terms from X.
+//
+// The hopping terms into the blocks of the other colour (Dw_bnd, sap_com of
+// the reference) leave the block solve as Weyl fields on the eight faces:
+// through a forward face the finished term U(x,mu)^+ (1+gamma_mu) s0(x),
+// through a backward face (1-gamma_mu) s0(x), which the receiving point
+// multiplies with its own forward link.  The next block solve of the
+// receiving block adds them to its residual, so that neither the corrections
+// nor the faces' links are gathered point by point.
 // ---------------------------------------------------------------------------
 
 constexpr int RBV = 256;
+constexpr int FPT = 64;              // points of a face
+constexpr int FUN = 8 * 6 * FPT;     // units of the face fields of a block
 
 // complex multiply-accumulate as FMA chains: acc + a b, acc + conj(a) b
 __device__ inline float2 cmac(float2 acc, float2 a, float2 b)
@@ -551,12 +566,30 @@ template <typename S> __device__ inline S from_f2(float2 v);
 template <> __device__ inline float2 from_f2<float2>(float2 v) { return v; }
 template <> __device__ inline __half2 from_f2<__half2>(float2 v) { return __float22half2_rn(v); }
 
+// Block point of a lane.  The order of the points of a 4^4 block is
+// lexicographic within each parity, even points first: lane x < 128 is the
+// even point, x >= 128 the odd point of pair i = x % 128, with
+// i = lex / 2, so the forward neighbour of a point has the pair index
+// i + 32, i + 8, i + 2 or i + (x3 odd) among the points of the other parity.
 template <typename S> struct RegBlock
 {
-   S u[4][9];  // U(x,mu) if x+mu is in the block
-   S m[36];    // Pauli pair at x (units as in the SW field)
-   int fwd[4], bwd[4];
+   S u[4][9];  // U(x,mu)
+   int lex;    // t, x1, x2, x3 in two bits each, from the top
+   bool odd;
    bool bp;    // open-bc boundary point
+   __device__ int coord(int mu) const { return (lex >> (6 - 2 * mu)) & 3; }
+   __device__ int pair() const { return lex >> 1; }
+   __device__ int fwd(int mu) const  // pair index of x + mu (if it is in the block)
+   {
+      return pair() + (mu == 0 ? 32 : (mu == 1 ? 8 : (mu == 2 ? 2 : (lex & 1))));
+   }
+   // index of the point on a face orthogonal to mu as its sender has it: the
+   // transverse coordinates in pairs, the points of even senders first
+   __device__ int face_point(int mu, bool sender_odd) const
+   {
+      const int hi = lex >> (8 - 2 * mu), lo = lex & ((1 << (6 - 2 * mu)) - 1);
+      return (((hi << (6 - 2 * mu)) | lo) >> 1) + (sender_odd ? 32 : 0);
+   }
 };
 
 // out = (A + i mu) v on the two Weyl halves (pauli_half); the half hh = 0
@@ -599,145 +632,65 @@ __device__ inline void pauli_reg(const S *m, float mu, const float2 *v, float2 *
    pauli_reg2(m, stride, m + 18 * stride, stride, mu, v, out);
 }
 
-// OUT: parity of the points whose terms are needed (0 even, 1 odd, 2 all);
-// lane x computes its own forward term if its output is needed and the
-// backward term of x+mu if the output of x+mu is needed, so that for one
-// parity the even and the odd lanes (separate wavefronts) share the work
-template <int MU, int OUT, typename S>
-__device__ inline void rb_hop_mu(const RegBlock<S> &b, bool odd, const float2 *v, float2 *acc, float2 (*F)[RBV],
-                                 float2 (*X)[RBV])
+template <int MU, bool FWD> __device__ inline void weyl_project(const float2 *sp, float2 *h)
 {
-   const int x = threadIdx.x;
-   const int y = b.fwd[MU];
-   const bool own = (OUT == 2) || (OUT == (int)odd);
-   const bool other = (OUT == 2) || (OUT != (int)odd);
-   if (y < RBV)
-   {
-      float2 h0[3], h1[3], c0[3], c1[3], u[9];
-#pragma unroll
-      for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[MU][k]);
-      if (own)
-      {
-         float2 sp[12];
-#pragma unroll
-         for (int c = 0; c < 12; c++) sp[c] = F[c][y];
-         spin_project<float2, MU, true>(sp, h0, h1);
-         su3_mul_f<false>(u, h0, c0);
-         su3_mul_f<false>(u, h1, c1);
-         spin_expand_add<float2, MU, true>(c0, c1, acc);
-      }
-      if (other)
-      {
-         // backward term of y from x through the same link
-         spin_project<float2, MU, false>(v, h0, h1);
-         su3_mul_f<true>(u, h0, c0);
-         su3_mul_f<true>(u, h1, c1);
-#pragma unroll
-         for (int c = 0; c < 3; c++)
-         {
-            X[c][y] = c0[c];
-            X[3 + c][y] = c1[c];
-         }
-      }
-   }
-   __syncthreads();
-   if (own && b.bwd[MU] < RBV)
-   {
-      float2 c0[3], c1[3];
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-      {
-         c0[c] = X[c][x];
-         c1[c] = X[3 + c][x];
-      }
-      spin_expand_add<float2, MU, false>(c0, c1, acc);
-   }
-   __syncthreads();
+   spin_project<float2, MU, FWD>(sp, h, h + 3);
 }
 
-// acc = sum of the hopping terms of the field v over in-block neighbours
-// (at the points of parity OUT); values at boundary points of open bc count
-// as zero (blk_hop skips them).  lb: LDS of 18 * RBV float2.
+// hopping pass into the points of parity OUT: the hopping terms from the
+// in-block neighbours (src of the lanes of the other parity, zero on the
+// boundary points of open bc) are added to w of the lanes of parity OUT,
+// forward terms of mu = 0..3, then backward terms.  src and w may be the same
+// registers.  lb: LDS of 18 * RBV float2.
 template <int OUT, typename S>
-__device__ inline void rb_hop(const RegBlock<S> &b, bool odd, const float2 *vin, float2 *acc, float2 *lb)
+__device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w, float2 *lb)
 {
-   const int x = threadIdx.x;
-   float2 v[12];
-   if (OUT == 2)
-   {
-      float2(*F)[RBV] = (float2(*)[RBV])lb;
-      float2(*X)[RBV] = (float2(*)[RBV])(lb + 12 * RBV);
-#pragma unroll
-      for (int c = 0; c < 12; c++)
-      {
-         v[c] = b.bp ? make_float2(0.0f, 0.0f) : vin[c];
-         F[c][x] = v[c];
-         acc[c] = make_float2(0.0f, 0.0f);
-      }
-      __syncthreads();
-      rb_hop_mu<0, OUT>(b, odd, v, acc, F, X);
-      rb_hop_mu<1, OUT>(b, odd, v, acc, F, X);
-      rb_hop_mu<2, OUT>(b, odd, v, acc, F, X);
-      rb_hop_mu<3, OUT>(b, odd, v, acc, F, X);
-      return;
-   }
-   // one parity: the source lanes (the other parity) store their values
-   // (F, indexed by the point within its parity), compute the backward
-   // terms of all four directions with their own links and pass them on
-   // (X[mu]), while the output lanes compute their forward terms from F;
-   // two barriers per pass.  The output lanes add the forward terms of
-   // mu = 0..3, then the backward ones.
    constexpr int RBH = RBV / 2;
    float2(*F)[RBH] = (float2(*)[RBH])lb;
    float2(*X)[6][RBH] = (float2(*)[6][RBH])(lb + 12 * RBH);
-   const bool own = (OUT == (int)odd);
-#pragma unroll
-   for (int c = 0; c < 12; c++)
+   const bool own = (OUT == (int)b.odd);
+   const int i = b.pair();
+   if (!own)
    {
-      v[c] = b.bp ? make_float2(0.0f, 0.0f) : vin[c];
-      if (!own) F[c][x & (RBH - 1)] = v[c];
-      acc[c] = make_float2(0.0f, 0.0f);
+#pragma unroll
+      for (int c = 0; c < 12; c++) F[c][i] = src[c];
    }
    __syncthreads();
 #pragma unroll
    for (int mu = 0; mu < 4; mu++)
    {
-      const int y = b.fwd[mu];
-      if (y < RBV)
+      const int y = b.fwd(mu);
+      if (b.coord(mu) < 3)
       {
-         float2 h0[3], h1[3], c0[3], c1[3], u[9];
+         float2 h[6], c[6], u[9];
 #pragma unroll
          for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[mu][k]);
          if (own)
          {
             float2 sp[12];
 #pragma unroll
-            for (int c = 0; c < 12; c++) sp[c] = F[c][y & (RBH - 1)];
-            if (mu == 0) { spin_project<float2, 0, true>(sp, h0, h1); }
-            if (mu == 1) { spin_project<float2, 1, true>(sp, h0, h1); }
-            if (mu == 2) { spin_project<float2, 2, true>(sp, h0, h1); }
-            if (mu == 3) { spin_project<float2, 3, true>(sp, h0, h1); }
-            su3_mul_f<false>(u, h0, c0);
-            su3_mul_f<false>(u, h1, c1);
-            if (mu == 0) spin_expand_add<float2, 0, true>(c0, c1, acc);
-            if (mu == 1) spin_expand_add<float2, 1, true>(c0, c1, acc);
-            if (mu == 2) spin_expand_add<float2, 2, true>(c0, c1, acc);
-            if (mu == 3) spin_expand_add<float2, 3, true>(c0, c1, acc);
+            for (int k = 0; k < 12; k++) sp[k] = F[k][y];
+            if (mu == 0) weyl_project<0, true>(sp, h);
+            if (mu == 1) weyl_project<1, true>(sp, h);
+            if (mu == 2) weyl_project<2, true>(sp, h);
+            if (mu == 3) weyl_project<3, true>(sp, h);
+            su3_mul_f<false>(u, h, c);
+            su3_mul_f<false>(u, h + 3, c + 3);
+            if (mu == 0) spin_expand_add<float2, 0, true>(c, c + 3, w);
+            if (mu == 1) spin_expand_add<float2, 1, true>(c, c + 3, w);
+            if (mu == 2) spin_expand_add<float2, 2, true>(c, c + 3, w);
+            if (mu == 3) spin_expand_add<float2, 3, true>(c, c + 3, w);
          }
          else
          {
-            if (mu == 0) spin_project<float2, 0, false>(v, h0, h1);
-            if (mu == 1) spin_project<float2, 1, false>(v, h0, h1);
-            if (mu == 2) spin_project<float2, 2, false>(v, h0, h1);
-            if (mu == 3) spin_project<float2, 3, false>(v, h0, h1);
-            su3_mul_f<true>(u, h0, c0);
-            su3_mul_f<true>(u, h1, c1);
+            if (mu == 0) weyl_project<0, false>(src, h);
+            if (mu == 1) weyl_project<1, false>(src, h);
+            if (mu == 2) weyl_project<2, false>(src, h);
+            if (mu == 3) weyl_project<3, false>(src, h);
+            su3_mul_f<true>(u, h, c);
+            su3_mul_f<true>(u, h + 3, c + 3);
 #pragma unroll
-            for (int c = 0; c < 3; c++)
-            {
-               X[mu][c][y & (RBH - 1)] = c0[c];
-               X[mu][3 + c][y & (RBH - 1)] = c1[c];
-            }
+            for (int k = 0; k < 6; k++) X[mu][k][y] = c[k];
          }
       }
    }
@@ -747,27 +700,48 @@ __device__ inline void rb_hop(const RegBlock<S> &b, bool odd, const float2 *vin,
 #pragma unroll
       for (int mu = 0; mu < 4; mu++)
       {
-         if (b.bwd[mu] < RBV)
+         if (b.coord(mu) > 0)
          {
-            float2 c0[3], c1[3];
+            float2 c[6];
 #pragma unroll
-            for (int c = 0; c < 3; c++)
-            {
-               c0[c] = X[mu][c][x & (RBH - 1)];
-               c1[c] = X[mu][3 + c][x & (RBH - 1)];
-            }
-            if (mu == 0) spin_expand_add<float2, 0, false>(c0, c1, acc);
-            if (mu == 1) spin_expand_add<float2, 1, false>(c0, c1, acc);
-            if (mu == 2) spin_expand_add<float2, 2, false>(c0, c1, acc);
-            if (mu == 3) spin_expand_add<float2, 3, false>(c0, c1, acc);
+            for (int k = 0; k < 6; k++) c[k] = X[mu][k][i];
+            if (mu == 0) spin_expand_add<float2, 0, false>(c, c + 3, w);
+            if (mu == 1) spin_expand_add<float2, 1, false>(c, c + 3, w);
+            if (mu == 2) spin_expand_add<float2, 2, false>(c, c + 3, w);
+            if (mu == 3) spin_expand_add<float2, 3, false>(c, c + 3, w);
          }
       }
    }
 }
 
-// block sums of |s2|^2 and (s2, s1) as in blk_mres_dev, lanes with act
-__device__ inline void rb_sums(bool act, const float2 *s2, const float2 *s1, double &rr, double &zr, double &zi)
+// sum over the 64 lanes of a wavefront, complete in lane 63 (row operations
+// in the vector unit instead of LDS permutes)
+template <int CTRL, int ROWS> __device__ inline double dpp_add(double x)
 {
+   const long long v = __double_as_longlong(x);
+   const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+   const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+   return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+__device__ inline double wave_sum63(double x)
+{
+   x = dpp_add<0xb1, 0xf>(x);   // quad_perm [1,0,3,2]
+   x = dpp_add<0x4e, 0xf>(x);   // quad_perm [2,3,0,1]
+   x = dpp_add<0x141, 0xf>(x);  // row_half_mirror
+   x = dpp_add<0x140, 0xf>(x);  // row_mirror: every lane has its row's sum
+   x = dpp_add<0x142, 0xa>(x);  // row_bcast15: rows 1 and 3 add rows 0 and 2
+   x = dpp_add<0x143, 0xc>(x);  // row_bcast31: rows 2 and 3 add row 1
+   return x;
+}
+
+// block sums of |s2|^2 and (s2, s1) as in blk_mres_dev over the lanes with
+// act (whole wavefronts).  sh may be written again only after another
+// barrier has been passed.
+__device__ inline void rb_sums(bool act, const float2 *s2, const float2 *s1, double (*sh)[4], double &rr, double &zr,
+                               double &zi)
+{
+   const int wv = threadIdx.x >> 6;
    rr = zr = zi = 0.0;
    if (act)
    {
@@ -787,80 +761,128 @@ __device__ inline void rb_sums(bool act, const float2 *s2, const float2 *s1, dou
          zr += (double)pr;
          zi += (double)pi;
       }
+      rr = wave_sum63(rr);
+      zr = wave_sum63(zr);
+      zi = wave_sum63(zi);
    }
-   wg_sum3(rr, zr, zi, RBV);
+   if ((threadIdx.x & 63) == 63)
+   {
+      sh[0][wv] = rr;
+      sh[1][wv] = zr;
+      sh[2][wv] = zi;
+   }
+   __syncthreads();
+   rr = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+   zr = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+   zi = (sh[2][0] + sh[2][1]) + (sh[2][2] + sh[2][3]);
 }
 
-// rho(x) += 1/2 hopping terms into block point x from the corrections s0g
-// of the neighbouring blocks (the other colour), as k_sap_faces applies
-// them, taken here at the start of the block solve
-#ifndef OQH_PULL_GROUP
-#define OQH_PULL_GROUP 2
-#endif
+// face fields: unit c of point p on face f of block n at
+// ((8 n + f) 6 + c) 64 + p; f = 2 mu the forward, 2 mu + 1 the backward face
+__device__ inline size_t face_unit(int n, int f) { return ((size_t)n * 8 + f) * (6 * FPT); }
+
+// acc += hopping terms into the point from outside the block, from the face
+// fields of the neighbouring blocks nbn[0..7] (forward neighbours 2 mu,
+// backward neighbours 2 mu + 1)
 template <typename S>
-__device__ inline void pull_faces(const SArgs &a, const RegBlock<S> &b, const S *ub, int gx, float2 *s1)
+__device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int *nbn, float2 *acc)
 {
-   constexpr bool H = sizeof(S) == 4;
-   const bool odd = gx >= a.h;
-   float2 acc[12], h0[3], h1[3], c0[3], c1[3];
-   zero12(acc);
-   // as in k_sap_faces: one neighbour and one link load per direction,
-   // OQH_PULL_GROUP directions ahead of the arithmetic
-   constexpr int FG = OQH_PULL_GROUP;
-   for (int m0 = 0; m0 < 4; m0 += FG)
+   // all loads first: a point lies on at most one of the faces of a
+   // direction
+   float2 h[4][6];
+#pragma unroll
+   for (int mu = 0; mu < 4; mu++)
    {
-      float2 sp[FG][12], u[FG][9];
-#pragma unroll
-      for (int j = 0; j < FG; j++)
+      const int x = b.coord(mu);
+      if (x == 3 || x == 0)
       {
-         const int MU = m0 + j;
-         const bool fw = b.fwd[MU] == RBV, bw = b.bwd[MU] == RBV;
-         if (fw || bw)
-         {
-            const int y = a.nbr[(size_t)(fw ? 2 * MU : 2 * MU + 1) * a.V + gx] & 0x7fffffff;
-            if (H)
-               load_h16(a.s0g16, a.s0sc, y, sp[j]);
-            else
-               load_spinor((const float2 *)a.s0g, y, sp[j]);
-            const int J = odd ? gx - a.h : y - a.h;
-            const int l = (odd == fw) ? 2 * MU : 2 * MU + 1;
-            const S *up = ub + (J >> 6) * (size_t)(72 * SB) + (J & (SB - 1)) + (size_t)(9 * l) * SB;
+         const size_t f = (x == 3) ? face_unit(nbn[2 * mu], 2 * mu + 1) : face_unit(nbn[2 * mu + 1], 2 * mu);
+         const float2 *p = W + f + b.face_point(mu, !b.odd);
 #pragma unroll
-            for (int q = 0; q < 9; q++) u[j][q] = to_f2(up[q * SB]);
-         }
-      }
-#pragma unroll
-      for (int j = 0; j < FG; j++)
-      {
-         const int MU = m0 + j;
-         const bool fw = b.fwd[MU] == RBV, bw = b.bwd[MU] == RBV;
-#define OQH_PULL_TERM(M)                                                               \
-   if (MU == M)                                                                       \
-   {                                                                                  \
-      if (fw)                                                                         \
-      {                                                                               \
-         spin_project<float2, M, true>(sp[j], h0, h1);                                \
-         su3_mul_f<false>(u[j], h0, c0);                                              \
-         su3_mul_f<false>(u[j], h1, c1);                                              \
-         spin_expand_add<float2, M, true>(c0, c1, acc);                               \
-      }                                                                               \
-      else if (bw)                                                                    \
-      {                                                                               \
-         spin_project<float2, M, false>(sp[j], h0, h1);                               \
-         su3_mul_f<true>(u[j], h0, c0);                                               \
-         su3_mul_f<true>(u[j], h1, c1);                                               \
-         spin_expand_add<float2, M, false>(c0, c1, acc);                              \
-      }                                                                               \
-   }
-         OQH_PULL_TERM(0)
-         OQH_PULL_TERM(1)
-         OQH_PULL_TERM(2)
-         OQH_PULL_TERM(3)
-#undef OQH_PULL_TERM
+         for (int c = 0; c < 6; c++) h[mu][c] = p[c * FPT];
       }
    }
 #pragma unroll
-   for (int c = 0; c < 12; c++) s1[c] = cadd(s1[c], cscale(acc[c], 0.5f));
+   for (int mu = 0; mu < 4; mu++)
+   {
+      const int x = b.coord(mu);
+      if (x == 3)
+      {
+         float2 c[6], u[9];
+#pragma unroll
+         for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[mu][k]);
+         su3_mul_f<false>(u, h[mu], c);
+         su3_mul_f<false>(u, h[mu] + 3, c + 3);
+         if (mu == 0) spin_expand_add<float2, 0, true>(c, c + 3, acc);
+         if (mu == 1) spin_expand_add<float2, 1, true>(c, c + 3, acc);
+         if (mu == 2) spin_expand_add<float2, 2, true>(c, c + 3, acc);
+         if (mu == 3) spin_expand_add<float2, 3, true>(c, c + 3, acc);
+      }
+      else if (x == 0)
+      {
+         if (mu == 0) spin_expand_add<float2, 0, false>(h[mu], h[mu] + 3, acc);
+         if (mu == 1) spin_expand_add<float2, 1, false>(h[mu], h[mu] + 3, acc);
+         if (mu == 2) spin_expand_add<float2, 2, false>(h[mu], h[mu] + 3, acc);
+         if (mu == 3) spin_expand_add<float2, 3, false>(h[mu], h[mu] + 3, acc);
+      }
+   }
+}
+
+// the block's face fields from its correction s0
+template <typename S> __device__ inline void rb_push(const RegBlock<S> &b, const float2 *s0, float2 *W, int n)
+{
+#pragma unroll
+   for (int mu = 0; mu < 4; mu++)
+   {
+      const int x = b.coord(mu);
+      if (x == 3)
+      {
+         float2 h[6], c[6], u[9];
+#pragma unroll
+         for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[mu][k]);
+         if (mu == 0) weyl_project<0, false>(s0, h);
+         if (mu == 1) weyl_project<1, false>(s0, h);
+         if (mu == 2) weyl_project<2, false>(s0, h);
+         if (mu == 3) weyl_project<3, false>(s0, h);
+         su3_mul_f<true>(u, h, c);
+         su3_mul_f<true>(u, h + 3, c + 3);
+         float2 *p = W + face_unit(n, 2 * mu) + b.face_point(mu, b.odd);
+#pragma unroll
+         for (int k = 0; k < 6; k++) p[k * FPT] = c[k];
+      }
+      else if (x == 0)
+      {
+         float2 h[6];
+         if (mu == 0) weyl_project<0, true>(s0, h);
+         if (mu == 1) weyl_project<1, true>(s0, h);
+         if (mu == 2) weyl_project<2, true>(s0, h);
+         if (mu == 3) weyl_project<3, true>(s0, h);
+         float2 *p = W + face_unit(n, 2 * mu + 1) + b.face_point(mu, b.odd);
+#pragma unroll
+         for (int k = 0; k < 6; k++) p[k * FPT] = h[k];
+      }
+   }
+}
+
+// point, links (S: FP32 or FP16) and boundary flag of the lane with point x;
+// OUTER: only the links that leave the block
+template <typename S, bool MASKED, bool OUTER = false>
+__device__ inline void rb_load(const SArgs &a, const S *ub, int x, int gx, RegBlock<S> &b)
+{
+   const int i = x & (RBV / 2 - 1);
+   b.odd = x >= RBV / 2;
+   // the parity of t + x1 + x2 + x3 fixes the last bit of the point
+   b.lex = 2 * i + (((i >> 5) ^ (i >> 3) ^ (i >> 1) ^ (int)b.odd) & 1);
+   b.bp = MASKED && a.bnd[gx];
+#pragma unroll
+   for (int mu = 0; mu < 4; mu++)
+   {
+      if (OUTER && b.coord(mu) < 3) continue;
+      const int J = b.odd ? gx - a.h : (a.nbr[(size_t)(2 * mu) * a.V + gx] & 0x7fffffff) - a.h;
+      const S *up = ub + (size_t)(J >> 6) * (72 * SB) + (J & (SB - 1)) + (size_t)(9 * (b.odd ? 2 * mu : 2 * mu + 1)) * SB;
+#pragma unroll
+      for (int k = 0; k < 9; k++) b.u[mu][k] = up[k * SB];
+   }
 }
 
 #ifndef OQH_SAP_WAVES16
@@ -879,6 +901,17 @@ __device__ inline void pull_faces(const SArgs &a, const RegBlock<S> &b, const S 
 // of each point in LDS and the second in registers (OQH_SAP_MHALF; with
 // both in registers it needs 310 registers and runs one wavefront per SIMD,
 // 1.50 against 0.82 ms per colour at 48^4).
+// With isolv = 1 the two parities work at the same time on A_oo^-1 of the odd
+// and A_ee of the even points, and one set of registers holds the value a
+// point sends or the sum it receives.  A colour at 48^4 takes 0.86 ms and a
+// cycle 2.0 ms; with a gather kernel for the faces (0.39 ms) and the two
+// Pauli products one after the other it was 0.82 and 2.45 ms (FP16 storage at
+// 32^3x64: 0.34 against 0.38 ms per colour).  Bound by both sides: 8200
+// vector instructions per wave take 0.55 ms of issue, the 1150 bytes per
+// point 0.55 ms, and two work-groups per CU overlap them only in part (0.1 ms
+// per further MinRes step).  Swapping the parities' waves in every other
+// work-group, delaying the second work-group of a CU and s_setprio changed
+// nothing.
 // MASKED: open-bc boundary points exist (bc != 3); without them the masking
 // of boundary values is compiled out
 template <int ISOLV, typename S, bool MASKED>
@@ -887,14 +920,15 @@ __attribute__((amdgpu_waves_per_eu(sizeof(S) == 4 ? OQH_SAP_WAVES16 : OQH_SAP_WA
 void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
 {
    __shared__ float2 LB[18 * RBV];  // hopping exchange (rb_hop)
-   // FP16 variant: the Pauli matrices of the block live in LDS, and psi,
-   // rho, s0g are FP16 spinors with per-site scales; FP32 variant with
+   __shared__ double sh[3][4];      // block sums
+   // FP16 variant: the Pauli matrices of the block live in LDS, and psi and
+   // rho are FP16 spinors with per-site scales; FP32 variant with
    // OQH_SAP_MHALF: the first Pauli matrix of each point in LDS, the second
    // in registers
    constexpr bool MLDS = sizeof(S) == 4;
    constexpr bool MHALF = !MLDS && OQH_SAP_MHALF;
-   constexpr bool MALL = MLDS;
-   __shared__ S MS[MALL ? 36 : (MHALF ? 18 : 1)][RBV];
+   constexpr int ML = MLDS ? 36 : (MHALF ? 18 : 0);  // units in LDS
+   __shared__ S MS[ML ? ML : 1][RBV];
    // several sources: consecutive work-groups take the same block for
    // different sources, so its links and SW matrices come from the cache
    const int src = a0.nsrc ? (int)(blockIdx.x % a0.nsrc) : 0;
@@ -904,120 +938,110 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
    {
       a.psi = a0.pl[src];
       a.rho = a0.rl[src];
-      a.s0g = a0.sl[src];
+      a.wf = a0.wl[src];
    }
    const int x = threadIdx.x;
    const int n = a.n0 + bi;
-   const int *imb = a.imb + (size_t)n * RBV;
-   const int gx = imb[x];
-   const bool even = x < a.bh;
-   RegBlock<S> b;
-   b.bp = MASKED && a.bnd[gx];
+   const int gx = a.imb[(size_t)n * RBV + x];
+   const bool even = x < RBV / 2;
    // links and SW matrices: the FP32 fields, or their FP16 copies
    const S *ub = sizeof(S) == sizeof(float2) ? (const S *)a.u : u16;
    const S *swb = sizeof(S) == sizeof(float2) ? (const S *)a.sw : sw16;
-#pragma unroll
-   for (int mu = 0; mu < 4; mu++)
-   {
-      b.fwd[mu] = a.bnb[(2 * mu) * RBV + x];
-      b.bwd[mu] = a.bnb[(2 * mu + 1) * RBV + x];
-      if (b.fwd[mu] < RBV)
-      {
-         const S *up = ub + (blk_link(a, gx, imb[b.fwd[mu]], mu, true) - a.u);
-#pragma unroll
-         for (int k = 0; k < 9; k++) b.u[mu][k] = up[k * SB];
-      }
-   }
+   RegBlock<S> b;
+   rb_load<S, MASKED>(a, ub, x, gx, b);
+   S mreg[ML == 36 ? 1 : 36 - ML];
    {
       const S *m = swb + (size_t)(gx >> 6) * (36 * SB) + (gx & (SB - 1));
 #pragma unroll
       for (int k = 0; k < 36; k++)
       {
-         if (MALL || (MHALF && k < 18))
+         if (k < ML)
             MS[k][x] = m[k * SB];
          else
-            b.m[k] = m[k * SB];
+            mreg[k - ML] = m[k * SB];
       }
    }
-   const S *mp0 = (MALL || MHALF) ? &MS[0][x] : b.m;
-   const int mst0 = (MALL || MHALF) ? RBV : 1;
-   const S *mp1 = MALL ? &MS[18][x] : b.m + 18;
-   const int mst1 = MALL ? RBV : 1;
-   float2 s0[12], s1[12], s2[12], acc[12];
+   const S *mp0 = ML ? &MS[0][x] : mreg;
+   const int mst0 = ML ? RBV : 1;
+   const S *mp1 = ML == 36 ? &MS[18 % (ML ? ML : 1)][x] : mreg + (18 - ML);
+   const int mst1 = ML == 36 ? RBV : 1;
+   const float2 zero = make_float2(0.0f, 0.0f);
+   float2 s0[12], s1[12], w[12];
    if (MLDS)
       load_h16(a.rho16, a.rsc, gx, s1);
    else
       load_spinor((const float2 *)a.rho, gx, s1);
-   // only the FP16 variant pulls the face terms (the FP32 cycles use the
-   // face kernel); the pull is not compiled into the FP32 kernel, whose
-   // registers it would crowd
-   if constexpr (MLDS)
-      if (a.pull) pull_faces<S>(a, b, ub, gx, s1);
+   if (a.pull)
+   {
+      zero12(w);
+      rb_pull(b, a.wf, a.nbn + 8 * (size_t)n, w);
+#pragma unroll
+      for (int c = 0; c < 12; c++) s1[c] = cadd(s1[c], cscale(w[c], 0.5f));
+   }
 #pragma unroll
    for (int c = 0; c < 12; c++)
    {
-      s0[c] = make_float2(0.0f, 0.0f);
-      s2[c] = make_float2(0.0f, 0.0f);
-      if (!ISOLV && b.bp) s1[c] = make_float2(0.0f, 0.0f);
+      s0[c] = zero;
+      if (!ISOLV && b.bp) s1[c] = zero;
    }
 
    if (ISOLV)
    {
       // odd points: s1 = A_oo^-1 s1, then even points: s1 += 1/2 hops
       // (Dwoo_blk, Dweo_blk of sap.c:759-761)
+      zero12(w);
       if (!even)
       {
-         float2 o[12];
-         pauli_reg2(mp0, mst0, mp1, mst1, 0.0f, s1, o);
+         pauli_reg2(mp0, mst0, mp1, mst1, 0.0f, s1, w);
 #pragma unroll
-         for (int c = 0; c < 12; c++) s1[c] = b.bp ? make_float2(0.0f, 0.0f) : o[c];
+         for (int c = 0; c < 12; c++)
+         {
+            if (b.bp) w[c] = zero;
+            s1[c] = w[c];
+         }
       }
-      rb_hop<0>(b, !even, s1, acc, LB);
+      rb_hop<0>(b, w, w, LB);
       if (even)
       {
 #pragma unroll
-         for (int c = 0; c < 12; c++)
-            s1[c] = b.bp ? make_float2(0.0f, 0.0f) : cadd(s1[c], cscale(acc[c], 0.5f));
+         for (int c = 0; c < 12; c++) s1[c] = b.bp ? zero : cadd(s1[c], cscale(w[c], 0.5f));
       }
    }
 
-   // minimal residual steps (blk_solv.c:1117-1186)
+   // minimal residual steps (blk_solv.c:1117-1186): w = D s1
    for (int imr = 0; imr < a.nmr; imr++)
    {
       if (ISOLV)
       {
-         // s2 (odd) = A_oo^-1 (-1/2 hops of s1_e); s2 (even) = A_ee s1 + 1/2 hops of s2_o
-         rb_hop<1>(b, !even, s1, acc, LB);
-         if (!even)
-         {
+         // odd: v = -1/2 hops of s1_e, even: v = s1; w = A_oo^-1 v and
+         // A_ee v at once; even: w += 1/2 hops of w_o
+         zero12(w);
+         rb_hop<1>(b, s1, w, LB);
+         float2 o[12];
 #pragma unroll
-            for (int c = 0; c < 12; c++) acc[c] = cscale(acc[c], -0.5f);
-            pauli_reg2(mp0, mst0, mp1, mst1, 0.0f, acc, s2);
-            if (b.bp)
-            {
+         for (int c = 0; c < 12; c++) w[c] = even ? s1[c] : cscale(w[c], -0.5f);
+         pauli_reg2(mp0, mst0, mp1, mst1, even ? a.mu : 0.0f, w, o);
+         const float f = even ? 2.0f : 1.0f;
 #pragma unroll
-               for (int c = 0; c < 12; c++) s2[c] = make_float2(0.0f, 0.0f);
-            }
-         }
-         rb_hop<0>(b, !even, s2, acc, LB);
-         if (even)
-         {
-            pauli_reg2(mp0, mst0, mp1, mst1, a.mu, s1, s2);
+         for (int c = 0; c < 12; c++) w[c] = (b.bp && !even) ? zero : cscale(o[c], f);
+         rb_hop<0>(b, w, w, LB);
 #pragma unroll
-            for (int c = 0; c < 12; c++)
-               s2[c] = b.bp ? make_float2(0.0f, 0.0f) : cadd(s2[c], cscale(acc[c], 0.5f));
-         }
+         for (int c = 0; c < 12; c++) w[c] = (b.bp && even) ? zero : cscale(w[c], 0.5f);
       }
       else
       {
-         rb_hop<2>(b, !even, s1, acc, LB);
-         pauli_reg2(mp0, mst0, mp1, mst1, even ? a.mu : a.muo, s1, s2);
+float2 o[12];
+         pauli_reg2(mp0, mst0, mp1, mst1, even ? a.mu : a.muo, s1, o);
+         // the accumulators start from -2 A s1, so that w = -1/2 their sum
 #pragma unroll
-         for (int c = 0; c < 12; c++)
-            s2[c] = b.bp ? make_float2(0.0f, 0.0f) : cadd(s2[c], cscale(acc[c], -0.5f));
+         for (int c = 0; c < 12; c++) w[c] = cscale(o[c], -2.0f);
+         rb_hop<1>(b, s1, w, LB);
+         rb_hop<0>(b, s1, w, LB);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = b.bp ? zero : cscale(w[c], -0.5f);
       }
       double rr, zr, zi;
-      rb_sums(ISOLV ? even : true, s2, s1, rr, zr, zi);
+      rb_sums(ISOLV ? even : true, w, s1, sh, rr, zr, zi);
       float r = (float)rr;
       if (r < 2.0f * FLT_MIN) break;
       r = 1.0f / r;
@@ -1028,7 +1052,7 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
          for (int c = 0; c < 12; c++)
          {
             s0[c] = cmac(s0[c], z, s1[c]);
-            s1[c] = cmac(s1[c], mz, s2[c]);
+            s1[c] = cmac(s1[c], mz, w[c]);
          }
       }
    }
@@ -1036,35 +1060,42 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
    if (ISOLV)
    {
       // odd solution s0_o = s1_o - A_oo^-1 (-1/2 hops of s0_e) (Dwoe_blk, Dwoo_blk)
-      rb_hop<1>(b, !even, s0, acc, LB);
+      zero12(w);
+      rb_hop<1>(b, s0, w, LB);
       if (!even)
       {
          float2 o[12];
 #pragma unroll
-         for (int c = 0; c < 12; c++) acc[c] = cscale(acc[c], -0.5f);
-         pauli_reg2(mp0, mst0, mp1, mst1, 0.0f, acc, o);
+         for (int c = 0; c < 12; c++) w[c] = cscale(w[c], -0.5f);
+         pauli_reg2(mp0, mst0, mp1, mst1, 0.0f, w, o);
 #pragma unroll
          for (int c = 0; c < 12; c++)
          {
-            if (b.bp) o[c] = make_float2(0.0f, 0.0f);
+            if (b.bp) o[c] = zero;
             s0[c] = csub(s1[c], o[c]);
          }
       }
    }
 
-   float2 p[12];
+   rb_push(b, s0, a.wf, n);
    if (a.pz)
-      zero12(p);
-   else if (MLDS)
-      load_h16(a.psi16, a.psc, gx, p);
-   else
-      load_spinor((const float2 *)a.psi, gx, p);
+   {
 #pragma unroll
-   for (int c = 0; c < 12; c++) p[c] = cadd(p[c], s0[c]);
-   if (MLDS)
-      store_h16(a.psi16, a.psc, gx, p);
+      for (int c = 0; c < 12; c++) w[c] = s0[c];
+   }
    else
-      store_spinor(a.psi, gx, p);
+   {
+      if (MLDS)
+         load_h16(a.psi16, a.psc, gx, w);
+      else
+         load_spinor((const float2 *)a.psi, gx, w);
+#pragma unroll
+      for (int c = 0; c < 12; c++) w[c] = cadd(w[c], s0[c]);
+   }
+   if (MLDS)
+      store_h16(a.psi16, a.psc, gx, w);
+   else
+      store_spinor(a.psi, gx, w);
    if (ISOLV && !even)
    {
       // odd residual -i mu gamma5 s0 (update_flds1) or 0 (eoflg, update_flds2)
@@ -1077,15 +1108,42 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
       }
    }
    if (MLDS)
-   {
       store_h16(a.rho16, a.rsc, gx, s1);
-      store_h16(a.s0g16, a.s0sc, gx, s0);
-   }
    else
-   {
       store_spinor(a.rho, gx, s1);
-      store_spinor(a.s0g, gx, s0);
+}
+
+// rho += hopping terms from the face fields of the neighbouring blocks for
+// the blocks from n0 on: completes the residual after the last block solves
+template <typename S>
+__global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
+{
+   constexpr bool H = sizeof(S) == 4;
+   const int src = a0.nsrc ? (int)(blockIdx.x % a0.nsrc) : 0;
+   const int bi = a0.nsrc ? (int)(blockIdx.x / a0.nsrc) : (int)blockIdx.x;
+   SArgs a = a0;
+   if (a0.nsrc)
+   {
+      a.rho = a0.rl[src];
+      a.wf = a0.wl[src];
    }
+   const int n = a.n0 + bi;
+   const int gx = a.imb[(size_t)n * RBV + threadIdx.x];
+   RegBlock<S> b;
+   rb_load<S, false, true>(a, H ? u16 : (const S *)a.u, threadIdx.x, gx, b);
+   float2 r[12], acc[12];
+   if (H)
+      load_h16(a.rho16, a.rsc, gx, r);
+   else
+      load_spinor((const float2 *)a.rho, gx, r);
+   zero12(acc);
+   rb_pull(b, a.wf, a.nbn + 8 * (size_t)n, acc);
+#pragma unroll
+   for (int c = 0; c < 12; c++) r[c] = cadd(r[c], cscale(acc[c], 0.5f));
+   if (H)
+      store_h16(a.rho16, a.rsc, gx, r);
+   else
+      store_spinor(a.rho, gx, r);
 }
 
 #ifndef OQH_FACE_GROUP
@@ -1094,18 +1152,9 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
 
 // rho(y) -= hopping terms into y from the block corrections of the
 // neighbouring blocks, for the face points y of the blocks of one colour
-// (S = __half2: FP16 links, FP16 s0g and rho with per-site scales)
-template <typename S>
-__global__ __launch_bounds__(256) void k_sap_faces(SArgs a0, const int *face, const unsigned char *fmask, int nf,
-                                                   const S *u16)
+// (block sizes other than 4^4)
+__global__ __launch_bounds__(256) void k_sap_faces(SArgs a, const int *face, const unsigned char *fmask, int nf)
 {
-   constexpr bool H = sizeof(S) == 4;
-   SArgs a = a0;
-   if (a0.nsrc)
-   {
-      a.rho = a0.rl[blockIdx.y];
-      a.s0g = a0.sl[blockIdx.y];
-   }
    int k = blockIdx.x * 256 + threadIdx.x;
    if (k >= nf) return;
    int y = face[k];
@@ -1113,7 +1162,6 @@ __global__ __launch_bounds__(256) void k_sap_faces(SArgs a0, const int *face, co
    float2 acc[12], h0[3], h1[3], c0[3], c1[3];
    zero12(acc);
    int odd = y >= a.h;
-   const S *ub = H ? u16 : (const S *)a.u;
    // a point of a block of width >= 2 lies on at most one of the faces -mu,
    // +mu: the loads of each direction are issued for all lanes at once (one
    // neighbour and one link per direction and lane), OQH_FACE_GROUP
@@ -1132,16 +1180,13 @@ __global__ __launch_bounds__(256) void k_sap_faces(SArgs a0, const int *face, co
          {
             const int dir = fw ? 2 * MU : 2 * MU + 1;
             const int x = a.nbr[(size_t)dir * a.V + y] & 0x7fffffff;
-            if (H)
-               load_h16(a.s0g16, a.s0sc, x, sp[j]);
-            else
-               load_spinor((const float2 *)a.s0g, x, sp[j]);
+            load_spinor((const float2 *)a.s0g, x, sp[j]);
             // forward: U(y, mu) (odd y) or U(x, mu) stored at the odd x
             const int J = odd ? y - a.h : x - a.h;
             const int l = (odd == fw) ? 2 * MU : 2 * MU + 1;
-            const S *up = ub + (J >> 6) * (size_t)(72 * SB) + (J & (SB - 1)) + (size_t)(9 * l) * SB;
+            const float2 *up = link_ptr(a.u, J, l);
 #pragma unroll
-            for (int q = 0; q < 9; q++) u[j][q] = to_f2(up[q * SB]);
+            for (int q = 0; q < 9; q++) u[j][q] = up[q * SB];
          }
       }
 #pragma unroll
@@ -1175,16 +1220,10 @@ __global__ __launch_bounds__(256) void k_sap_faces(SArgs a0, const int *face, co
       }
    }
    float2 r[12];
-   if (H)
-      load_h16(a.rho16, a.rsc, y, r);
-   else
-      load_spinor((const float2 *)a.rho, y, r);
+   load_spinor((const float2 *)a.rho, y, r);
 #pragma unroll
    for (int c = 0; c < 12; c++) r[c] = cadd(r[c], cscale(acc[c], 0.5f));
-   if (H)
-      store_h16(a.rho16, a.rsc, y, r);
-   else
-      store_spinor(a.rho, y, r);
+   store_spinor(a.rho, y, r);
 }
 
 // ---------------------------------------------------------------------------
@@ -1396,11 +1435,15 @@ static void free_grid()
    for (int c = 0; c < 2; c++) { dev_free(G.d_face[c]); dev_free(G.d_fmask[c]); G.d_face[c] = nullptr; G.d_fmask[c] = nullptr; }
    dev_free(G.d_swb); dev_free(G.d_scr); dev_free(G.d_s0g); dev_free(G.d_bs);
    dev_free(G.d_u16); dev_free(G.d_swb16);
-   for (int k = 0; k < 3; k++) { dev_free(G.d_h16[k]); dev_free(G.d_hsc[k]); dev_free(G.d_h64[k]); }
-   dev_free(G.d_swb64); dev_free(G.d_scr64); dev_free(G.d_s0gm); dev_free(G.d_bsd);
+   for (int k = 0; k < 2; k++) { dev_free(G.d_h16[k]); dev_free(G.d_hsc[k]); }
+   for (int k = 0; k < 3; k++) dev_free(G.d_h64[k]);
+   dev_free(G.d_swb64); dev_free(G.d_scr64); dev_free(G.d_bsd);
+   dev_free(G.d_wf); dev_free(G.d_wfm); dev_free(G.d_nbn);
    dev_free(G.d_ipp); dev_free(G.d_bw);
    G = SapGrid();
 }
+
+static bool reg_kernel() { return OQH_SAP_REG && G.bvol == RBV; }
 
 static bool build_grid(const char *where)
 {
@@ -1543,9 +1586,31 @@ static bool build_grid(const char *where)
       }
    }
    G.d_swb = (float2 *)dev_alloc(units_for(L.g.V, 36) * sizeof(float2));
-   G.d_scr = (float2 *)dev_alloc((size_t)G.nbh * 3 * G.Ub * sizeof(float2));
-   G.d_s0g = (float2 *)dev_alloc(units_for(L.g.V, 12) * sizeof(float2));
-   HIP_OK(hipMemset(G.d_s0g, 0, units_for(L.g.V, 12) * sizeof(float2)));
+   if (reg_kernel())
+   {
+      // neighbouring blocks: the block of a point one step outside
+      std::vector<int> blk(L.g.V), nbn(8 * (size_t)G.nb);
+      for (int n = 0; n < G.nb; n++)
+         for (int i = 0; i < G.bvol; i++) blk[G.imb[(size_t)n * G.bvol + i]] = n;
+      for (int n = 0; n < G.nb; n++)
+         for (int mu = 0; mu < 4; mu++)
+            for (int i = 0; i < G.bvol; i++)
+            {
+               const size_t gx = G.imb[(size_t)n * G.bvol + i];
+               if (bnb[(size_t)(2 * mu) * G.bvol + i] == G.bvol) nbn[8 * (size_t)n + 2 * mu] = blk[L.g.iup[4 * gx + mu]];
+               if (bnb[(size_t)(2 * mu + 1) * G.bvol + i] == G.bvol)
+                  nbn[8 * (size_t)n + 2 * mu + 1] = blk[L.g.idn[4 * gx + mu]];
+            }
+      G.d_nbn = (int *)dev_alloc(sizeof(int) * nbn.size());
+      HIP_OK(hipMemcpy(G.d_nbn, nbn.data(), sizeof(int) * nbn.size(), hipMemcpyHostToDevice));
+      G.d_wf = (float2 *)dev_alloc((size_t)G.nb * FUN * sizeof(float2));
+   }
+   else
+   {
+      G.d_scr = (float2 *)dev_alloc((size_t)G.nbh * 3 * G.Ub * sizeof(float2));
+      G.d_s0g = (float2 *)dev_alloc(units_for(L.g.V, 12) * sizeof(float2));
+      HIP_OK(hipMemset(G.d_s0g, 0, units_for(L.g.V, 12) * sizeof(float2)));
+   }
    G.swb_set = -1;
    G.ready = true;
    return true;
@@ -1607,34 +1672,42 @@ static SArgs sargs(float mu, int nmr)
    a.n0 = 0;
    a.psi16 = G.d_h16[0];
    a.rho16 = G.d_h16[1];
-   a.s0g16 = G.d_h16[2];
    a.psc = G.d_hsc[0];
    a.rsc = G.d_hsc[1];
-   a.s0sc = G.d_hsc[2];
+   a.wf = G.d_wf;
+   a.nbn = G.d_nbn;
    a.pz = 0;
    return a;
 }
 
 static bool half_variant()
 {
-   return OQH_SAP_REG && G.bvol == RBV && lib().sap_prec == 1 && G.d_h16[0] && G.d_h16[1] && G.d_h16[2] && G.d_u16 &&
+   return OQH_SAP_REG && G.bvol == RBV && lib().sap_prec == 1 && G.d_h16[0] && G.d_h16[1] && G.d_u16 &&
           G.d_swb16;
 }
 
-static bool reg_kernel() { return OQH_SAP_REG && G.bvol == RBV; }
-
 // block solves of the blocks of colour ic; the register kernel first adds
-// the face terms from the other colour's corrections if pull is set
+// the terms of the other colour's face fields if pull is set
 static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
 {
    Lib &L = lib();
    SArgs a = a0;
    a.n0 = ic ? G.nbh : 0;
    a.pull = pull;
-   if (a.nsrc)
+   const unsigned nb = (unsigned)(G.nbh * std::max(a.nsrc, 1));
+   if (half_variant() && !a.nsrc)
    {
-      // several sources: the FP32 register kernel only
-      const unsigned nb = (unsigned)(G.nbh * a.nsrc);
+      if (isolv && a.masked)
+         k_sap_reg<1, __half2, true><<<nb, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
+      else if (isolv)
+         k_sap_reg<1, __half2, false><<<nb, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
+      else if (a.masked)
+         k_sap_reg<0, __half2, true><<<nb, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
+      else
+         k_sap_reg<0, __half2, false><<<nb, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
+   }
+   else if (reg_kernel())
+   {
       if (isolv && a.masked)
          k_sap_reg<1, float2, true><<<nb, RBV, 0, L.stream>>>(a, nullptr, nullptr);
       else if (isolv)
@@ -1643,78 +1716,48 @@ static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
          k_sap_reg<0, float2, true><<<nb, RBV, 0, L.stream>>>(a, nullptr, nullptr);
       else
          k_sap_reg<0, float2, false><<<nb, RBV, 0, L.stream>>>(a, nullptr, nullptr);
-      return;
-   }
-   if (half_variant())
-   {
-      if (isolv && a.masked)
-         k_sap_reg<1, __half2, true><<<G.nbh, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
-      else if (isolv)
-         k_sap_reg<1, __half2, false><<<G.nbh, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
-      else if (a.masked)
-         k_sap_reg<0, __half2, true><<<G.nbh, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
-      else
-         k_sap_reg<0, __half2, false><<<G.nbh, RBV, 0, L.stream>>>(a, G.d_u16, G.d_swb16);
-   }
-   else if (reg_kernel())
-   {
-      if (isolv && a.masked)
-         k_sap_reg<1, float2, true><<<G.nbh, RBV, 0, L.stream>>>(a, nullptr, nullptr);
-      else if (isolv)
-         k_sap_reg<1, float2, false><<<G.nbh, RBV, 0, L.stream>>>(a, nullptr, nullptr);
-      else if (a.masked)
-         k_sap_reg<0, float2, true><<<G.nbh, RBV, 0, L.stream>>>(a, nullptr, nullptr);
-      else
-         k_sap_reg<0, float2, false><<<G.nbh, RBV, 0, L.stream>>>(a, nullptr, nullptr);
    }
    else if (G.bvol >= SWG_MAX)
    {
       // large blocks (6^4, 8^4): 1024 threads per block, the few blocks of a
       // small lattice would otherwise leave most of the chip idle
       if (isolv)
-         k_sap_blocks<1, float2, SWG_MAX><<<G.nbh, SWG_MAX, 0, L.stream>>>(a);
+         k_sap_blocks<1, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
       else
-         k_sap_blocks<0, float2, SWG_MAX><<<G.nbh, SWG_MAX, 0, L.stream>>>(a);
+         k_sap_blocks<0, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
    }
    else if (isolv)
-      k_sap_blocks<1><<<G.nbh, SWG, 0, L.stream>>>(a);
+      k_sap_blocks<1><<<nb, SWG, 0, L.stream>>>(a);
    else
-      k_sap_blocks<0><<<G.nbh, SWG, 0, L.stream>>>(a);
+      k_sap_blocks<0><<<nb, SWG, 0, L.stream>>>(a);
 }
 
 // face terms from the corrections of the colour-(1-c) blocks into rho on
-// the faces of the colour-c blocks
+// the faces of the colour-c blocks (block sizes other than 4^4)
 static void sap_push_faces(const SArgs &a, int c)
 {
-   Lib &L = lib();
    if (!G.nface[c]) return;
-   unsigned nbk = (G.nface[c] + 255) / 256;
-   if (a.nsrc)
-   {
-      k_sap_faces<float2><<<dim3(nbk, a.nsrc), 256, 0, L.stream>>>(a, G.d_face[c], G.d_fmask[c], G.nface[c], nullptr);
-      return;
-   }
-   if (half_variant())
-      k_sap_faces<__half2><<<nbk, 256, 0, L.stream>>>(a, G.d_face[c], G.d_fmask[c], G.nface[c], G.d_u16);
-   else
-      k_sap_faces<float2><<<nbk, 256, 0, L.stream>>>(a, G.d_face[c], G.d_fmask[c], G.nface[c], nullptr);
+   k_sap_faces<<<(G.nface[c] + 255) / 256, 256, 0, lib().stream>>>(a, G.d_face[c], G.d_fmask[c], G.nface[c]);
 }
 
 // one Schwarz cycle (sap.c:720-790): colour 0, faces of colour 1, colour 1,
-// faces of colour 0.  With the FP16 register kernel the face terms into a
-// colour are added by its block kernel (pull), so the cycle needs no face
-// kernel except the final one; first: rho is complete on entry (no pull for
-// colour 0); finish: complete rho at the end (faces of colour 0).
+// faces of colour 0.  With the register kernel the face terms into a colour
+// are added by its next block solve; first: rho is complete on entry (none
+// for colour 0); finish: complete rho at the end (faces of colour 0).
 static void sap_cycle(const SArgs &a, int isolv, bool first, bool finish)
 {
-   // the FP32 register kernel keeps the face kernel: pulling the face terms
-   // (scattered loads at the start of every block solve) measured no faster
-   // at two wavefronts per SIMD (2.54 vs 2.49 ms per cycle at 48^4)
-   if (half_variant() && !a.nsrc)
+   if (reg_kernel())
    {
       sap_blocks(a, 0, isolv, !first);
       sap_blocks(a, 1, isolv, 1);
-      if (finish) sap_push_faces(a, 0);
+      if (!finish) return;
+      SArgs c = a;
+      c.n0 = 0;
+      const unsigned nb = (unsigned)(G.nbh * std::max(a.nsrc, 1));
+      if (half_variant() && !a.nsrc)
+         k_sap_complete<__half2><<<nb, RBV, 0, lib().stream>>>(c, G.d_u16);
+      else
+         k_sap_complete<float2><<<nb, RBV, 0, lib().stream>>>(c, nullptr);
    }
    else
    {
@@ -1865,18 +1908,20 @@ bool sap_mop64(double mu, int isolv, int nmr, int ncy, const float2 *rho, float2
    return true;
 }
 
-// one SAP cycle on device fields (no synchronisation); the FP16 variant
-// converts psi and rho to FP16 spinors and back
-void sap_device(float mu, int isolv, int nmr, float2 *psi, float2 *rho)
+// ncy SAP cycles on device fields (no synchronisation); the FP16 variant
+// converts psi and rho to FP16 spinors and back.  zero: the cycles start
+// from psi = 0 (psi need not be set); want_res: rho is needed on return.
+void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho, bool zero, bool want_res)
 {
    Lib &L = lib();
+   const size_t nu = units_for(L.g.V, 12);
+   const unsigned nbu = (unsigned)((nu + 255) / 256);
    if (f64_variant())
    {
-      const size_t nu = units_for(L.g.V, 12);
-      const unsigned nbk = (unsigned)((nu + 255) / 256);
-      k_s32_to_s64<<<nbk, 256, 0, L.stream>>>(psi, G.d_h64[0], nu);
-      k_s32_to_s64<<<nbk, 256, 0, L.stream>>>(rho, G.d_h64[1], nu);
-      sap_cycle64(sargs64(mu, nmr), isolv);
+      if (zero) HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
+      k_s32_to_s64<<<nbu, 256, 0, L.stream>>>(psi, G.d_h64[0], nu);
+      k_s32_to_s64<<<nbu, 256, 0, L.stream>>>(rho, G.d_h64[1], nu);
+      for (int n = 0; n < ncy; n++) sap_cycle64(sargs64(mu, nmr), isolv);
       convert_f64_to_f32(G.d_h64[0], psi, nu, L.stream);
       convert_f64_to_f32(G.d_h64[1], rho, nu, L.stream);
       return;
@@ -1886,29 +1931,40 @@ void sap_device(float mu, int isolv, int nmr, float2 *psi, float2 *rho)
    a.rho = rho;
    const int V = L.g.V;
    const unsigned nbk = (V + 255) / 256;
+   const bool pz = zero && reg_kernel();
+   if (zero && !pz) HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
    if (half_variant())
    {
-      k_s32_to_h16<<<nbk, 256, 0, L.stream>>>(psi, G.d_h16[0], G.d_hsc[0], V);
+      if (!pz) k_s32_to_h16<<<nbk, 256, 0, L.stream>>>(psi, G.d_h16[0], G.d_hsc[0], V);
       k_s32_to_h16<<<nbk, 256, 0, L.stream>>>(rho, G.d_h16[1], G.d_hsc[1], V);
    }
-   sap_cycle(a, isolv, true, true);
+   for (int n = 0; n < ncy; n++)
+   {
+      // the blocks of both colours see psi = 0 in the first cycle
+      a.pz = (n == 0 && pz);
+      sap_cycle(a, isolv, n == 0, n == ncy - 1 && want_res);
+   }
    if (half_variant())
    {
       k_h16_to_s32<<<nbk, 256, 0, L.stream>>>(G.d_h16[0], G.d_hsc[0], psi, V);
-      k_h16_to_s32<<<nbk, 256, 0, L.stream>>>(G.d_h16[1], G.d_hsc[1], rho, V);
+      if (want_res) k_h16_to_s32<<<nbk, 256, 0, L.stream>>>(G.d_h16[1], G.d_hsc[1], rho, V);
    }
 }
 
-// ncy Schwarz cycles (FP32) on n sources at once (n <= 16): psi[k] and
-// rho[k] are full FP32 device fields; each launch takes all sources
+// ncy Schwarz cycles (FP32) from psi = 0 on n sources at once (n <= 16):
+// psi[k] and rho[k] are full FP32 device fields; each launch takes all
+// sources
 bool sap_multi_device(float mu, int isolv, int nmr, int ncy, int n, float2 *const *psi, float2 *const *rho)
 {
-   Lib &L = lib();
    if (n < 1 || n > 16 || !reg_kernel()) return false;
-   if (!G.d_s0gm)
+   const size_t nw = (size_t)G.nb * FUN;
+   if (n > G.wfm_n)
    {
-      G.d_s0gm = (float2 *)dev_alloc(16 * units_for(L.g.V, 12) * sizeof(float2));
-      if (!G.d_s0gm) return false;
+      HIP_OK(hipStreamSynchronize(lib().stream));
+      dev_free(G.d_wfm);
+      G.d_wfm = (float2 *)dev_alloc(n * nw * sizeof(float2));
+      G.wfm_n = G.d_wfm ? n : 0;
+      if (!G.d_wfm) return false;
    }
    SArgs a = sargs(mu, nmr);
    a.nsrc = n;
@@ -1916,9 +1972,13 @@ bool sap_multi_device(float mu, int isolv, int nmr, int ncy, int n, float2 *cons
    {
       a.pl[k] = psi[k];
       a.rl[k] = rho[k];
-      a.sl[k] = G.d_s0gm + (size_t)k * units_for(L.g.V, 12);
+      a.wl[k] = G.d_wfm + (size_t)k * nw;
    }
-   for (int c = 0; c < ncy; c++) sap_cycle(a, isolv, true, true);
+   for (int c = 0; c < ncy; c++)
+   {
+      a.pz = (c == 0);
+      sap_cycle(a, isolv, c == 0, c == ncy - 1);
+   }
    return true;
 }
 
@@ -2040,7 +2100,7 @@ static void ensure_half_fields()
    size_t nu = units_for(L.g.V / 2, 72), ns = units_for(L.g.V, 36);
    if (!G.d_u16) G.d_u16 = (__half2 *)dev_alloc(nu * sizeof(__half2));
    if (!G.d_swb16) G.d_swb16 = (__half2 *)dev_alloc(ns * sizeof(__half2));
-   for (int k = 0; k < 3; k++)
+   for (int k = 0; k < 2; k++)
    {
       if (!G.d_h16[k]) G.d_h16[k] = (__half2 *)dev_alloc(units_for(L.g.V, 12) * sizeof(__half2));
       if (!G.d_hsc[k]) G.d_hsc[k] = (float *)dev_alloc((size_t)L.g.V * sizeof(float));
@@ -2120,7 +2180,7 @@ extern "C" void sap(float mu, int isolv, int nmr, spinor *psi, spinor *eta)
       fail("sap [sap.c]", "the fields must be full fields");
       return;
    }
-   sap_device(mu, isolv, nmr, (float2 *)p.dev, (float2 *)r.dev);
+   sap_cycles(mu, isolv, nmr, 1, (float2 *)p.dev, (float2 *)r.dev, false, true);
    finish(p, F32, V, true);
    finish(r, F32, V, true);
 }
@@ -2595,12 +2655,12 @@ extern "C" double oqh_sap_autotune(int isolv, int nmr, int ncy, int maxvol, int 
       // warm-up cycle
       HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
       k_hash_fill<<<nbk, 256, 0, L.stream>>>(rho, nu, 12345);
-      sap_device((float)0.0f, isolv, nmr, psi, rho);
+      sap_cycles(0.0f, isolv, nmr, 1, psi, rho, false, true);
       HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
       k_hash_fill<<<nbk, 256, 0, L.stream>>>(rho, nu, 12345);
       const double r0 = field_norm(rho, nu, d_part, h_part);
       HIP_OK(hipEventRecord(e0, L.stream));
-      for (int n = 0; n < ncy; n++) sap_device(0.0f, isolv, nmr, psi, rho);
+      sap_cycles(0.0f, isolv, nmr, ncy, psi, rho, false, true);
       HIP_OK(hipEventRecord(e1, L.stream));
       HIP_OK(hipEventSynchronize(e1));
       float ms = 0.0f;

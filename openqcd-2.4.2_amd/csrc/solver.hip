@@ -22,6 +22,7 @@ bool sap_prepare(int isolv, const char *where, bool quiet);
 bool sap_mixed_mop(float mu, int isolv, int nmr, int ncy, const float2 *rho, float2 *phi, bool want_res);
 void sap_mixed_residual(float2 *r);
 bool sap_mop64(double mu, int isolv, int nmr, int ncy, const float2 *rho, float2 *phi, float2 *chi);
+void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho, bool zero, bool want_res);
 bool sap_multi_device(float mu, int isolv, int nmr, int ncy, int n, float2 *const *psi, float2 *const *rho);
 }
 
@@ -245,9 +246,14 @@ static void Mop(int k, spinor *rho, spinor *phi, spinor *chi)
       }
       return;
    }
-   set_s2zero(vt, 2, phi);
    assign_s2s(vt, 2, rho, chi);
-   for (int n = 0; n < L.sap_ncy; n++) sap((float)mud, L.sap_isolv, L.sap_nmr, phi, chi);
+   if (dev)
+      sap_cycles((float)mud, L.sap_isolv, L.sap_nmr, L.sap_ncy, p, c, true, true);
+   else
+   {
+      set_s2zero(vt, 2, phi);
+      for (int n = 0; n < L.sap_ncy; n++) sap((float)mud, L.sap_isolv, L.sap_nmr, phi, chi);
+   }
    if (nn_use && dev)
    {
       // learned correction from the residual the Schwarz cycles leave
@@ -478,10 +484,7 @@ extern "C" void sap_gcr_multi(int n, int nkv, int nmx, int istop, double res, do
       if (act.empty()) break;
       // Mop of every active source: phi = SAP(rho), chi = rho - residual
       for (int s : act)
-      {
-         set_s2zero(vt, 2, S[s].phi[S[s].k]);
          assign_s2s(vt, 2, S[s].rho, S[s].chi[S[s].k]);
-      }
       for (size_t i0 = 0; i0 < act.size(); i0 += 16)
       {
          pl.clear();
