@@ -30,6 +30,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -44,6 +45,14 @@ constexpr int PNS = 128;  // points per work-group
 constexpr int PWG = 256;  // threads per work-group
 constexpr int NLMAX = 8;  // layers
 constexpr int CMAX = 16;  // channels
+constexpr int NBMAX = 16; // pairs of a training batch per launch
+
+// inputs and outputs of the samples of a launch (blockIdx.y)
+struct Batch
+{
+   const void *in[NBMAX];
+   void *out[NBMAX];
+};
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -101,10 +110,11 @@ __device__ inline float2 lnk(__half2 v) { return __half22float2(v); }
 // so every link is loaded once, and one barrier pair serves two directions.
 // accum (out += ...) only with FP32 output.
 template <int CI, int CO, typename TI = float2, typename TO = float2, typename UL = float2>
-__global__ __launch_bounds__(PWG) void k_ptc(const TI *__restrict__ in, TO *__restrict__ out,
-                                             const __bf16 *__restrict__ wp, const UL *__restrict__ u,
+__global__ __launch_bounds__(PWG) void k_ptc(Batch bt, const __bf16 *__restrict__ wp, const UL *__restrict__ u,
                                              const int *__restrict__ nbr, int V, int accum)
 {
+   const TI *__restrict__ in = (const TI *)bt.in[blockIdx.y];
+   TO *__restrict__ out = (TO *)bt.out[blockIdx.y];
    constexpr int KP = kpad(CI);
    constexpr int LD = 2 * KP + 8;  // LDS row stride (bf16): two direction blocks
    static_assert(2 * CO <= 32 && CI % 2 == 0, "channel counts");
@@ -261,20 +271,23 @@ __global__ void k_ptc_pack(const float2 *w, int ci, int co, int adj, __bf16 *wp)
 // sums, as the fused multiply-adds they replace).  The transported channels
 // go to LDS as [K][2 C_in]; each wave owns one 16 x 16 tile of the result (or,
 // with fewer than four tiles, a share of K) and keeps its rows of g, which
-// are the same for all nine directions, in registers.  Bound by the transport
-// loads and the LDS exchange: a pair's gradient at
-// 16^4 (4-12-16-12-4) takes 0.63 ms against 1.63 ms with scalar products of
-// the LDS rows and a sum over the work-groups by one thread per element.
+// are the same for all nine directions, in registers.  Two wavefronts per SIMD
+// (with one, 255 + 4 registers, a layer of 8 samples took 0.84 ms): the loads
+// of one work-group overlap the 96 matrix instructions per direction of the
+// other.  The gradient of 8 pairs at 16^4 (4-12-16-12-4) takes 4.0 ms against
+// 13.0 ms with scalar products of the LDS rows and a sum over the
+// work-groups by one thread per element.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int WG_TILES(int ci, int co) { return ((2 * co + 15) / 16) * ((2 * ci + 15) / 16); }
 constexpr int WG_KSPLIT(int ci, int co) { return 4 / WG_TILES(ci, co); }  // point sets per work-group
 
 template <int CI, int CO>
-__global__ __launch_bounds__(PWG) void k_ptc_wgrad(const float2 *__restrict__ in, const float2 *__restrict__ g,
-                                                   const float2 *__restrict__ u, const int *__restrict__ nbr, int V,
-                                                   float2 *part)
+__global__ __launch_bounds__(PWG) __attribute__((amdgpu_waves_per_eu(2))) void k_ptc_wgrad(Batch bt, const float2 *__restrict__ u,
+                                                   const int *__restrict__ nbr, int V, float2 *part)
 {
+   const float2 *__restrict__ in = (const float2 *)bt.in[blockIdx.y];
+   const float2 *__restrict__ g = (const float2 *)bt.out[blockIdx.y];  // output gradients
    constexpr int NT = (2 * CI + 15) / 16, TILES = WG_TILES(CI, CO), KS = WG_KSPLIT(CI, CO);
    constexpr int CM = CI > CO ? CI : CO;
    // rows of 16-column tiles, padded by one pair against bank conflicts
@@ -308,11 +321,13 @@ __global__ __launch_bounds__(PWG) void k_ptc_wgrad(const float2 *__restrict__ in
       __syncthreads();
    }
    constexpr int CH = CI / 2;
+   int yn = x;  // neighbour of the next direction, one step ahead
    for (int p = 0; p < NDIR; p++)
    {
       if (x < V)
       {
-         const int y = ptc_nbr(nbr, V, x, p);
+         const int y = yn;
+         if (p + 1 < NDIR) yn = ptc_nbr(nbr, V, x, p + 1);
          float2 um[9];
          bool dag = false;
          if (p > 0)
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(PWG) void k_ptc_wgrad(const float2 *__restrict__ in
          const float re1 = __shfl_xor(acc[r + 1], 1), im1 = __shfl_xor(acc[r], 1);
          const int o = 8 * mt + 2 * kk + (r >> 1), i = 8 * nt + (row >> 1);
          if (!(row & 1) && o < CO && i < CI)
-            part[(((size_t)blockIdx.x * KS + ks) * NDIR + p) * CO * CI + o * CI + i] =
+            part[((((size_t)blockIdx.y * gridDim.x + blockIdx.x) * KS + ks) * NDIR + p) * CO * CI + o * CI + i] =
                 make_float2(acc[r] + re1, acc[r + 1] - im1);
       }
       __syncthreads();
@@ -400,9 +415,10 @@ __global__ __launch_bounds__(64 * WSW) void k_ptc_wgrad_sum(const float2 *part, 
    grad[e].y += (float)zi;
 }
 
-// loss terms of one sample: partial sums of |e|^2 and |out - e|^2
-__global__ void k_ptc_loss(const float2 *out, const float2 *e, int n, double *part)
+// loss terms of a sample (blockIdx.y): partial sums of |e|^2 and |out - e|^2
+__global__ void k_ptc_loss(Batch bt, int n, double *part)
 {
+   const float2 *out = (const float2 *)bt.out[blockIdx.y], *e = (const float2 *)bt.in[blockIdx.y];
    __shared__ double sh[2][256];
    double se = 0.0, sd = 0.0;
    for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256)
@@ -426,16 +442,44 @@ __global__ void k_ptc_loss(const float2 *out, const float2 *e, int n, double *pa
    }
    if (threadIdx.x == 0)
    {
-      part[2 * blockIdx.x] = sh[0][0];
-      part[2 * blockIdx.x + 1] = sh[1][0];
+      double *p = part + 2 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x);
+      p[0] = sh[0][0];
+      p[1] = sh[1][0];
    }
 }
 
-// g = c (out - e)
-__global__ void k_ptc_lgrad(const float2 *out, const float2 *e, float c, int n, float2 *g)
+// |e|^2 and |out - e|^2 of a sample (one wave each, fixed order)
+__global__ __launch_bounds__(64) void k_ptc_loss_sum(const double *part, int nb, double *sums)
 {
+   double se = 0.0, sd = 0.0;
+   const double *p = part + 2 * (size_t)blockIdx.x * nb;
+   for (int b = threadIdx.x; b < nb; b += 64)
+   {
+      se += p[2 * b];
+      sd += p[2 * b + 1];
+   }
+   for (int m = 32; m >= 1; m >>= 1)
+   {
+      se += __shfl_xor(se, m);
+      sd += __shfl_xor(sd, m);
+   }
+   if (threadIdx.x == 0)
+   {
+      sums[2 * blockIdx.x] = se;
+      sums[2 * blockIdx.x + 1] = sd;
+   }
+}
+
+// output gradient of the mean loss over npair pairs, g = 2 (out - e) /
+// (npair |e|^2) in place of out (0 for a pair without target)
+__global__ void k_ptc_lgrad(Batch bt, const double *sums, int npair, int n)
+{
+   const float2 *e = (const float2 *)bt.in[blockIdx.y];
+   float2 *g = (float2 *)bt.out[blockIdx.y];
+   const double se = sums[2 * blockIdx.y];
+   const float c = se > 0.0 ? (float)(2.0 / (se * npair)) : 0.0f;
    const int k = blockIdx.x * 256 + threadIdx.x;
-   if (k < n) g[k] = make_float2(c * (out[k].x - e[k].x), c * (out[k].y - e[k].y));
+   if (k < n) g[k] = make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y));
 }
 
 // Adam step on n reals
@@ -473,10 +517,12 @@ struct Net
    bool packed = false;
    int adam_t = 0;
    int V = 0;
+   int nbatch = 0;                 // samples the following fields hold
    float2 *d_act[NLMAX + 1] = {};  // activations of the last forward
-   float2 *d_gb[2] = {};            // backward gradients (ping-pong)
-   float2 *d_part = nullptr;        // weight-gradient partials
-   double *d_lpart = nullptr, *h_lpart = nullptr;
+   float2 *d_out = nullptr;        // its outputs, then the output gradients
+   float2 *d_gb[2] = {};           // backward gradients (ping-pong)
+   float2 *d_part = nullptr;       // weight-gradient partials
+   double *d_lpart = nullptr, *d_lsum = nullptr, *h_lsum = nullptr;  // loss terms
    float2 *d_tmp = nullptr;         // spinor work field of the preconditioner
    bf16x2 *d_inf[2] = {};           // BF16 activations of the preconditioner (ping-pong)
    __half2 *d_u16 = nullptr;        // FP16 links of the preconditioner
@@ -492,9 +538,10 @@ void free_net()
    dev_free(N.d_w); dev_free(N.d_g); dev_free(N.d_m); dev_free(N.d_v);
    for (int l = 0; l < NLMAX; l++) { dev_free(N.d_pf[l]); dev_free(N.d_pa[l]); }
    for (int l = 0; l <= NLMAX; l++) dev_free(N.d_act[l]);
-   dev_free(N.d_gb[0]); dev_free(N.d_gb[1]); dev_free(N.d_part); dev_free(N.d_lpart); dev_free(N.d_tmp);
+   dev_free(N.d_gb[0]); dev_free(N.d_gb[1]); dev_free(N.d_part); dev_free(N.d_lpart); dev_free(N.d_lsum); dev_free(N.d_tmp);
+   dev_free(N.d_out);
    dev_free(N.d_inf[0]); dev_free(N.d_inf[1]); dev_free(N.d_u16);
-   if (N.h_lpart) HIP_OK(hipHostFree(N.h_lpart));
+   if (N.h_lsum) HIP_OK(hipHostFree(N.h_lsum));
    N = Net();
 }
 
@@ -512,64 +559,98 @@ void pack()
    N.packed = true;
 }
 
-// activations sized for the current lattice
-bool ensure_fields()
+// samples that are worked on together: as many as 2 GiB of activations and
+// gradients allow (a batch of 16 at 16^4; one at 32^3x64, whose layers fill
+// the device by themselves)
+int batch_size(int n)
 {
-   Lib &L = lib();
-   if (N.V == L.g.V && N.d_gb[0]) return true;
-   for (int l = 0; l <= NLMAX; l++) { dev_free(N.d_act[l]); N.d_act[l] = nullptr; }
-   for (int k = 0; k < 2; k++) { dev_free(N.d_gb[k]); N.d_gb[k] = nullptr; }
-   for (int k = 0; k < 2; k++) { dev_free(N.d_inf[k]); N.d_inf[k] = nullptr; }
-   dev_free(N.d_part); dev_free(N.d_tmp); dev_free(N.d_u16);
-   N.d_u16 = nullptr;
-   N.u16_epoch = -1;
-   N.V = L.g.V;
-   for (int l = 1; l < N.nl; l++) N.d_act[l] = (float2 *)dev_alloc(units_for(N.V, 3 * CMAX) * sizeof(float2));
-   for (int k = 0; k < 2; k++) N.d_gb[k] = (float2 *)dev_alloc(units_for(N.V, 3 * CMAX) * sizeof(float2));
-   const int nb = (N.V + PNS - 1) / PNS;
-   N.d_part = (float2 *)dev_alloc((size_t)nb * NDIR * CMAX * CMAX * sizeof(float2));
-   N.d_tmp = (float2 *)dev_alloc(units_for(N.V, 12) * sizeof(float2));
-   for (int k = 0; k < 2; k++) N.d_inf[k] = (bf16x2 *)dev_alloc(units_for(N.V, 3 * CMAX) * sizeof(bf16x2));
-   N.d_u16 = (__half2 *)dev_alloc(units_for(N.V / 2, 72) * sizeof(__half2));
-   return N.d_gb[0] && N.d_gb[1] && N.d_part && N.d_tmp && N.d_inf[0] && N.d_inf[1] && N.d_u16;
+   const size_t V = lib().g.V;
+   size_t units = 12;
+   int wmax = 4;
+   for (int l = 1; l < N.nl; l++)
+   {
+      units += 3 * N.w[l];
+      wmax = std::max(wmax, N.w[l]);
+   }
+   units += 2 * 3 * wmax;
+   const size_t bytes = V * units * sizeof(float2);
+   return (int)std::max<size_t>(1, std::min<size_t>(std::min(n, NBMAX), ((size_t)2 << 30) / bytes));
 }
 
-template <int CI, int CO>
-void launch_layer(const float2 *in, float2 *out, const __bf16 *wp, int accum)
+// activations of nb samples for the current lattice
+bool ensure_fields(int nb = 1)
+{
+   Lib &L = lib();
+   if (N.V == L.g.V && N.nbatch >= nb) return true;
+   HIP_OK(hipStreamSynchronize(L.stream));
+   for (int l = 0; l <= NLMAX; l++) { dev_free(N.d_act[l]); N.d_act[l] = nullptr; }
+   for (int k = 0; k < 2; k++) { dev_free(N.d_gb[k]); N.d_gb[k] = nullptr; }
+   dev_free(N.d_part); dev_free(N.d_out);
+   N.nbatch = 0;
+   const size_t V64 = units_for(L.g.V, 1);
+   int wmax = 4;
+   bool ok = true;
+   for (int l = 1; l < N.nl; l++)
+   {
+      N.d_act[l] = (float2 *)dev_alloc(nb * V64 * 3 * N.w[l] * sizeof(float2));
+      wmax = std::max(wmax, N.w[l]);
+      ok = ok && N.d_act[l];
+   }
+   for (int k = 0; k < 2; k++) N.d_gb[k] = (float2 *)dev_alloc(nb * V64 * 3 * wmax * sizeof(float2));
+   const int np = (L.g.V + PNS - 1) / PNS;
+   N.d_part = (float2 *)dev_alloc((size_t)nb * np * NDIR * CMAX * CMAX * sizeof(float2));
+   N.d_out = (float2 *)dev_alloc(nb * V64 * 12 * sizeof(float2));
+   ok = ok && N.d_gb[0] && N.d_gb[1] && N.d_part && N.d_out;
+   // the unused end of a field's last storage block takes part in the loss
+   if (N.d_out) HIP_OK(hipMemsetAsync(N.d_out, 0, nb * V64 * 12 * sizeof(float2), L.stream));
+   if (N.V != L.g.V)
+   {
+      for (int k = 0; k < 2; k++) { dev_free(N.d_inf[k]); N.d_inf[k] = nullptr; }
+      dev_free(N.d_tmp); dev_free(N.d_u16);
+      N.u16_epoch = -1;
+      N.V = L.g.V;
+      N.d_tmp = (float2 *)dev_alloc(units_for(N.V, 12) * sizeof(float2));
+      for (int k = 0; k < 2; k++) N.d_inf[k] = (bf16x2 *)dev_alloc(units_for(N.V, 3 * CMAX) * sizeof(bf16x2));
+      N.d_u16 = (__half2 *)dev_alloc(units_for(N.V / 2, 72) * sizeof(__half2));
+   }
+   ok = ok && N.d_tmp && N.d_inf[0] && N.d_inf[1] && N.d_u16;
+   if (ok) N.nbatch = nb;
+   return ok;
+}
+
+template <int CI, int CO> void launch_layer(const Batch &bt, int n, const __bf16 *wp)
 {
    Lib &L = lib();
    const int V = L.g.V;
-   k_ptc<CI, CO><<<(V + PNS - 1) / PNS, PWG, 0, L.stream>>>(in, out, wp, L.d_u, L.d_nbr, V, accum);
+   k_ptc<CI, CO><<<dim3((V + PNS - 1) / PNS, n), PWG, 0, L.stream>>>(bt, wp, L.d_u, L.d_nbr, V, 0);
 }
 
 // one layer of the preconditioner: mode 0 FP32 -> BF16, 1 BF16 -> BF16,
 // 2 BF16 -> FP32 added to out, 3 FP32 -> FP32 added to out
-template <int CI, int CO>
-void launch_inf(const void *in, void *out, const __bf16 *wp, int mode)
+template <int CI, int CO> void launch_inf(const void *in, void *out, const __bf16 *wp, int mode)
 {
    Lib &L = lib();
    const int V = L.g.V;
    const unsigned nb = (V + PNS - 1) / PNS;
    const __half2 *u = N.d_u16;
+   Batch bt = {};
+   bt.in[0] = in;
+   bt.out[0] = out;
    if (mode == 0)
-      k_ptc<CI, CO, float2, bf16x2, __half2><<<nb, PWG, 0, L.stream>>>((const float2 *)in, (bf16x2 *)out, wp, u,
-                                                                       L.d_nbr, V, 0);
+      k_ptc<CI, CO, float2, bf16x2, __half2><<<nb, PWG, 0, L.stream>>>(bt, wp, u, L.d_nbr, V, 0);
    else if (mode == 1)
-      k_ptc<CI, CO, bf16x2, bf16x2, __half2><<<nb, PWG, 0, L.stream>>>((const bf16x2 *)in, (bf16x2 *)out, wp, u,
-                                                                       L.d_nbr, V, 0);
+      k_ptc<CI, CO, bf16x2, bf16x2, __half2><<<nb, PWG, 0, L.stream>>>(bt, wp, u, L.d_nbr, V, 0);
    else if (mode == 2)
-      k_ptc<CI, CO, bf16x2, float2, __half2><<<nb, PWG, 0, L.stream>>>((const bf16x2 *)in, (float2 *)out, wp, u,
-                                                                       L.d_nbr, V, 1);
+      k_ptc<CI, CO, bf16x2, float2, __half2><<<nb, PWG, 0, L.stream>>>(bt, wp, u, L.d_nbr, V, 1);
    else
-      k_ptc<CI, CO, float2, float2, __half2><<<nb, PWG, 0, L.stream>>>((const float2 *)in, (float2 *)out, wp, u,
-                                                                       L.d_nbr, V, 1);
+      k_ptc<CI, CO, float2, float2, __half2><<<nb, PWG, 0, L.stream>>>(bt, wp, u, L.d_nbr, V, 1);
 }
 
-template <int CI, int CO> void launch_wgrad(const float2 *in, const float2 *g)
+template <int CI, int CO> void launch_wgrad(const Batch &bt, int n)
 {
    Lib &L = lib();
    const int V = L.g.V, nb = (V + PNS - 1) / PNS;
-   k_ptc_wgrad<CI, CO><<<nb, PWG, 0, L.stream>>>(in, g, L.d_u, L.d_nbr, V, N.d_part);
+   k_ptc_wgrad<CI, CO><<<dim3(nb, n), PWG, 0, L.stream>>>(bt, L.d_u, L.d_nbr, V, N.d_part);
 }
 
 #define OQH_PTC_DISPATCH(F, ci, co, ...)                                             \
@@ -594,70 +675,81 @@ template <int CI, int CO> void launch_wgrad(const float2 *in, const float2 *g)
       done_ = true;                                                                 \
    }
 
-// forward pass; keeps the activations of the hidden layers
-void forward(const float2 *in, float2 *out)
+// sample k of a workspace of n samples with nc units per point
+float2 *sample(float2 *f, int k, int nc) { return f + (size_t)k * units_for(lib().g.V, nc); }
+
+// forward pass of n samples; keeps the activations of the hidden layers
+void forward(int n, const float2 *const *in, float2 *const *out)
 {
    pack();
-   const float2 *x = in;
+   Batch bt = {};
+   for (int k = 0; k < n; k++) bt.in[k] = in[k];
    for (int l = 0; l < N.nl; l++)
    {
-      float2 *y = (l == N.nl - 1) ? out : N.d_act[l + 1];
-      OQH_PTC_DISPATCH(launch_layer, N.w[l], N.w[l + 1], x, y, N.d_pf[l], 0);
-      x = y;
+      for (int k = 0; k < n; k++) bt.out[k] = (l == N.nl - 1) ? out[k] : sample(N.d_act[l + 1], k, 3 * N.w[l + 1]);
+      OQH_PTC_DISPATCH(launch_layer, N.w[l], N.w[l + 1], bt, n, N.d_pf[l]);
+      for (int k = 0; k < n; k++) bt.in[k] = bt.out[k];
    }
 }
 
-// gradients of the weights (added to d_g) for the output gradient g of the
-// last forward pass with input in
-void backward(const float2 *in, const float2 *g)
+// gradients of the weights (added to d_g) for the output gradients g of the
+// last forward pass with inputs in
+void backward(int n, const float2 *const *in, float2 *const *g)
 {
    Lib &L = lib();
    const int nb = (L.g.V + PNS - 1) / PNS;
-   const float2 *gl = g;
+   Batch bt = {}, bg = {};  // layer inputs and output gradients; the layer's adjoint
+   for (int k = 0; k < n; k++) bt.out[k] = g[k];
    for (int l = N.nl - 1; l >= 0; l--)
    {
-      const float2 *al = l ? N.d_act[l] : in;
-      OQH_PTC_DISPATCH(launch_wgrad, N.w[l], N.w[l + 1], al, gl);
-      const int n = NDIR * N.w[l] * N.w[l + 1];
-      k_ptc_wgrad_sum<<<(n + 63) / 64, 64 * WSW, 0, L.stream>>>(N.d_part, nb * WG_KSPLIT(N.w[l], N.w[l + 1]), n,
-                                                                N.d_g + N.off[l]);
+      for (int k = 0; k < n; k++) bt.in[k] = l ? sample(N.d_act[l], k, 3 * N.w[l]) : in[k];
+      OQH_PTC_DISPATCH(launch_wgrad, N.w[l], N.w[l + 1], bt, n);
+      const int nw = NDIR * N.w[l] * N.w[l + 1];
+      k_ptc_wgrad_sum<<<(nw + 63) / 64, 64 * WSW, 0, L.stream>>>(N.d_part, n * nb * WG_KSPLIT(N.w[l], N.w[l + 1]), nw,
+                                                                 N.d_g + N.off[l]);
       if (l > 0)
       {
-         float2 *gn = (gl == N.d_gb[0]) ? N.d_gb[1] : N.d_gb[0];
-         OQH_PTC_DISPATCH(launch_layer, N.w[l + 1], N.w[l], gl, gn, N.d_pa[l], 0);
-         gl = gn;
+         for (int k = 0; k < n; k++)
+         {
+            bg.in[k] = bt.out[k];
+            bt.out[k] = bg.out[k] = sample(N.d_gb[l & 1], k, 3 * N.w[l]);
+         }
+         OQH_PTC_DISPATCH(launch_layer, N.w[l + 1], N.w[l], bg, n, N.d_pa[l]);
       }
    }
 }
 
+constexpr int LNB = 256;  // work-groups of a sample's loss
+
 // mean loss over the samples; gradients of the mean loss in d_g
-double loss_and_grad(int n, float2 *const *r, float2 *const *e, float2 *out)
+double loss_and_grad(int n, float2 *const *r, float2 *const *e)
 {
    Lib &L = lib();
-   const int V = L.g.V;
-   const size_t nu = units_for(V, 12);
+   const int nu = (int)units_for(L.g.V, 12);
+   const int B = batch_size(n);
+   if (!ensure_fields(B)) return 0.0;
    HIP_OK(hipMemsetAsync(N.d_g, 0, nweights() * sizeof(float2), L.stream));
    double loss = 0.0;
-   const int lb = 256;
-   for (int k = 0; k < n; k++)
+   float2 *out[NBMAX];
+   for (int k = 0; k < B; k++) out[k] = sample(N.d_out, k, 12);
+   for (int k0 = 0; k0 < n; k0 += B)
    {
-      forward(r[k], out);
-      k_ptc_loss<<<lb, 256, 0, L.stream>>>(out, e[k], (int)nu, N.d_lpart);
-      HIP_OK(hipMemcpyAsync(N.h_lpart, N.d_lpart, 2 * lb * sizeof(double), hipMemcpyDeviceToHost, L.stream));
-      HIP_OK(hipStreamSynchronize(L.stream));
-      double se = 0.0, sd = 0.0;
-      for (int b = 0; b < lb; b++)
+      const int m = std::min(B, n - k0);
+      forward(m, r + k0, out);
+      Batch bt = {};
+      for (int k = 0; k < m; k++)
       {
-         se += N.h_lpart[2 * b];
-         sd += N.h_lpart[2 * b + 1];
+         bt.in[k] = e[k0 + k];
+         bt.out[k] = out[k];
       }
-      if (se == 0.0) continue;
-      loss += sd / se / n;
-      // g = 2 (out - e) / (|e|^2 n), into the ping-pong buffer not used by
-      // the first backward step
-      float2 *g = N.d_gb[1];
-      k_ptc_lgrad<<<(unsigned)((nu + 255) / 256), 256, 0, L.stream>>>(out, e[k], (float)(2.0 / (se * n)), (int)nu, g);
-      backward(r[k], g);
+      k_ptc_loss<<<dim3(LNB, m), 256, 0, L.stream>>>(bt, nu, N.d_lpart);
+      k_ptc_loss_sum<<<m, 64, 0, L.stream>>>(N.d_lpart, LNB, N.d_lsum);
+      k_ptc_lgrad<<<dim3((nu + 255) / 256, m), 256, 0, L.stream>>>(bt, N.d_lsum, n, nu);
+      backward(m, r + k0, out);
+      HIP_OK(hipMemcpyAsync(N.h_lsum, N.d_lsum, 2 * m * sizeof(double), hipMemcpyDeviceToHost, L.stream));
+      HIP_OK(hipStreamSynchronize(L.stream));
+      for (int k = 0; k < m; k++)
+         if (N.h_lsum[2 * k] != 0.0) loss += N.h_lsum[2 * k + 1] / N.h_lsum[2 * k] / n;
    }
    return loss;
 }
@@ -763,8 +855,9 @@ extern "C" int oqh_nn_create(int nlayer, const int *widths)
       N.d_pf[l] = (__bf16 *)dev_alloc((size_t)NDIR * 32 * kpad(N.w[l]) * sizeof(__bf16));
       N.d_pa[l] = (__bf16 *)dev_alloc((size_t)NDIR * 32 * kpad(N.w[l + 1]) * sizeof(__bf16));
    }
-   N.d_lpart = (double *)dev_alloc(2 * 256 * sizeof(double));
-   HIP_OK(hipHostMalloc((void **)&N.h_lpart, 2 * 256 * sizeof(double), 0));
+   N.d_lpart = (double *)dev_alloc(2 * NBMAX * LNB * sizeof(double));
+   N.d_lsum = (double *)dev_alloc(2 * NBMAX * sizeof(double));
+   HIP_OK(hipHostMalloc((void **)&N.h_lsum, 2 * NBMAX * sizeof(double), 0));
    HIP_OK(hipMemset(N.d_w, 0, nw * sizeof(float2)));
    HIP_OK(hipMemset(N.d_m, 0, 2 * nw * sizeof(float)));
    HIP_OK(hipMemset(N.d_v, 0, 2 * nw * sizeof(float)));
@@ -822,7 +915,9 @@ extern "C" void oqh_nn_apply(spinor *in, spinor *out)
       fail(where, "the fields must be distinct full fields");
       return;
    }
-   forward((const float2 *)a.dev, (float2 *)b.dev);
+   const float2 *fi = (const float2 *)a.dev;
+   float2 *fo = (float2 *)b.dev;
+   forward(1, &fi, &fo);
    finish(a, F32, V, false);
    finish(b, F32, V, true);
 }
@@ -850,7 +945,7 @@ extern "C" double oqh_nn_grad(int n, spinor **r, spinor **e, double *dw)
    if (!require_net(where)) return 0.0;
    std::vector<float2 *> rr, ee;
    if (!fields_of(n, r, rr, where) || !fields_of(n, e, ee, where)) return 0.0;
-   double loss = loss_and_grad(n, rr.data(), ee.data(), N.d_tmp);
+   double loss = loss_and_grad(n, rr.data(), ee.data());
    size_t nw = nweights();
    std::vector<float2> h(nw);
    HIP_OK(hipStreamSynchronize(lib().stream));
@@ -870,7 +965,7 @@ extern "C" double oqh_nn_train_step(int n, spinor **r, spinor **e, double lr)
    std::vector<float2 *> rr, ee;
    if (!fields_of(n, r, rr, where) || !fields_of(n, e, ee, where)) return 0.0;
    Lib &L = lib();
-   double loss = loss_and_grad(n, rr.data(), ee.data(), N.d_tmp);
+   double loss = loss_and_grad(n, rr.data(), ee.data());
    const float b1 = 0.9f, b2 = 0.999f;
    N.adam_t++;
    const float c1 = 1.0f / (1.0f - powf(b1, (float)N.adam_t)), c2 = 1.0f / (1.0f - powf(b2, (float)N.adam_t));
