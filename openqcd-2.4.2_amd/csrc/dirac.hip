@@ -12,10 +12,10 @@
 //
 // Each (1 -+ gamma_mu) projection is applied before the colour product, so
 // that only two colour vectors are multiplied per direction (the spin
-// structure is that of the reference's doe/deo, Dw_dble.c:1114-1373).  A
-// work-group of 256 handles the 128 even and the 128 odd points with the same
-// offsets in the two halves of the site order; these lie in the same cache
-// block, so the links and spinors shared by them are re-read from L2.
+// structure is that of the reference's doe/deo, Dw_dble.c:1114-1373).  The
+// parity pieces (k_dirac) have one work-item per point; Dw and Dwhat work on
+// tiles of points (k_dw_tile, k_hat1_tile, k_hat2_tile) or, on small lattices,
+// with eight wavefronts per 64 points (k_split).
 //
 // Boundary rules (open bc): odd points on the boundary time slices are zeroed
 // in input and output of Dw and contribute no hopping terms to even points
@@ -30,7 +30,7 @@
 
 namespace oqh {
 
-enum DiracOp { OP_DW = 0, OP_DOE, OP_DEO, OP_HAT1, OP_HAT2, OP_DIAG };
+enum DiracOp { OP_DOE = 0, OP_DEO, OP_DIAG };
 
 template <typename T> struct DArgs
 {
@@ -93,65 +93,21 @@ __device__ inline void hop_all(const DArgs<T> &a, const typename cplx_of<T>::t *
    hop_mu<T, 3>(a, in, x, odd, mask, acc);
 }
 
-#ifndef OQH_DW_WAVES
-#define OQH_DW_WAVES 0
-#endif
-#ifndef OQH_NT_STORE
-#define OQH_NT_STORE 0
-#endif
-#if OQH_DW_WAVES
-#define DW_ATTR __attribute__((amdgpu_waves_per_eu(OQH_DW_WAVES)))
-#else
-#define DW_ATTR
-#endif
-
 template <typename T, int OP>
-__global__ __launch_bounds__(256) DW_ATTR void k_dirac(DArgs<T> a)
+__global__ __launch_bounds__(256) void k_dirac(DArgs<T> a)
 {
    typedef typename cplx_of<T>::t C;
-   int x, odd;
+   int x;
    int b = xcd_tile(blockIdx.x, gridDim.x, a.xcdc);
-   if (OP == OP_DW)
-   {
-      int tid = threadIdx.x;
-      int k = b * 128 + (tid & 127);
-      if (k >= a.h) return;
-      odd = tid >> 7;
-      x = k + odd * a.h;
-   }
-   else
-   {
-      int k = b * 256 + threadIdx.x;
-      if (k >= a.np) return;
-      x = a.p0 + k;
-      odd = x >= a.h;
-   }
+   int k = b * 256 + threadIdx.x;
+   if (k >= a.np) return;
+   x = a.p0 + k;
 
    C acc[12];
 #pragma unroll
    for (int c = 0; c < 12; c++) acc[c] = cmk<C>(0, 0);
 
-   if (OP == OP_DW)
-   {
-      if (a.masked && a.bnd[x])
-      {
-         zero_spinor(a.r, x);
-         zero_spinor(a.s_w, x);
-         return;
-      }
-      hop_all(a, a.s, x, odd, a.masked != 0, acc);
-      C v[12], o[12];
-      load_spinor(a.s, x, v);
-      pauli_site(a.sw, x, odd ? a.muo : a.mu, v, o);
-#pragma unroll
-      for (int c = 0; c < 12; c++) o[c] = cadd(o[c], cscale(acc[c], a.coef));
-#if OQH_NT_STORE
-      store_spinor_nt(a.r, x, o);
-#else
-      store_spinor(a.r, x, o);
-#endif
-   }
-   else if (OP == OP_DOE)
+   if (OP == OP_DOE)
    {
       if (a.masked && a.bnd[x])
       {
@@ -173,35 +129,6 @@ __global__ __launch_bounds__(256) DW_ATTR void k_dirac(DArgs<T> a)
       hop_all(a, a.s, x, 0, a.masked != 0, acc);
       C o[12];
       load_spinor((const C *)a.r, x, o);
-#pragma unroll
-      for (int c = 0; c < 12; c++) o[c] = cadd(o[c], cscale(acc[c], a.coef));
-      store_spinor(a.r, x, o);
-   }
-   else if (OP == OP_HAT1)
-   {
-      if (a.masked && a.bnd[x])
-      {
-         zero_spinor(a.t, x);
-         return;
-      }
-      hop_all(a, a.s, x, 1, a.masked != 0, acc);
-      C o[12];
-#pragma unroll
-      for (int c = 0; c < 12; c++) acc[c] = cscale(acc[c], a.coef);
-      pauli_site(a.sw, x, (T)0, acc, o);
-      store_spinor(a.t, x, o);
-   }
-   else if (OP == OP_HAT2)
-   {
-      if (a.masked && a.bnd[x])
-      {
-         zero_spinor(a.r, x);
-         return;
-      }
-      hop_all(a, (const C *)a.t, x, 0, a.masked != 0, acc);
-      C v[12], o[12];
-      load_spinor(a.s, x, v);
-      pauli_site(a.sw, x, a.mu, v, o);
 #pragma unroll
       for (int c = 0; c < 12; c++) o[c] = cadd(o[c], cscale(acc[c], a.coef));
       store_spinor(a.r, x, o);
@@ -256,13 +183,6 @@ __global__ __launch_bounds__(256) DW_ATTR void k_dirac(DArgs<T> a)
 #endif
 template <typename T> struct TileSize { static constexpr int n = OQH_DW_TPD; };
 template <> struct TileSize<float> { static constexpr int n = OQH_DW_TPF; };
-#ifndef OQH_DW_TILE
-#define OQH_DW_TILE 1
-#endif
-#ifndef OQH_HAT_TILE
-#define OQH_HAT_TILE 1
-#endif
-
 #ifndef OQH_NBR_PRELOAD
 #define OQH_NBR_PRELOAD 1
 #endif
@@ -558,7 +478,7 @@ __global__ __launch_bounds__(TP) void k_hat1_tile(DArgs<T> a)
 #pragma unroll
       for (int c = 0; c < 12; c++) S[c][t] = se[c];
    }
-   __syncthreads();
+   tile_sync<TP>();
    tile_phase<T, 0, true, TP, true, false, REC>(a, t, e0, valid, nb, S, nullptr, nullptr, acc, nullptr, nullptr);
    tile_phase<T, 0, false, TP, true, false, REC>(a, t, e0, valid, nb, S, nullptr, nullptr, acc, nullptr, nullptr);
    tile_phase<T, 1, true, TP, true, false, REC>(a, t, e0, valid, nb, S, nullptr, nullptr, acc, nullptr, nullptr);
@@ -632,6 +552,195 @@ __global__ __launch_bounds__(TP) void k_hat2_tile(DArgs<T> a)
 #pragma unroll
    for (int c = 0; c < 12; c++) out[c] = cadd(out[c], cscale(acc[c], a.coef));
    store_out(a.r, e, out);
+}
+
+// ---------------------------------------------------------------------------
+// Dw, Dwhat on small lattices: the work of a point split over eight lanes
+//
+// A tile of the kernels above does the eight directions one after the other;
+// on a lattice of a few thousand points that is a chain of 27 us on a
+// handful of CUs.  Here eight wavefronts take the same 64 points, each one
+// direction: neighbour, link and the two colour products, which go to LDS.
+// Six of them then form two rows each of the hopping sum and of the
+// SW term, whose matrix they have loaded meanwhile.  Dw_dble at 8^4: 5.1 us,
+// the latency of three dependent loads and a barrier.  Every neighbour's
+// spinor and both ends' links are read from the caches (2.2 times the bytes
+// of a tile; 9 TB/s at 16^4), so larger lattices are left to the tiles
+// (use_split).  The points of an XCD are contiguous (16^4 26.6 us, in dispatch
+// order 32.3).
+// ---------------------------------------------------------------------------
+
+enum SplitOp { SP_DW = 0, SP_HAT1, SP_HAT2 };
+
+// one direction: the two colour products of the projected neighbour
+template <typename T, int MU, bool FWD>
+__device__ inline void split_hop(const DArgs<T> &a, const typename cplx_of<T>::t *in, int x, bool odd,
+                                 typename cplx_of<T>::t *c)
+{
+   typedef typename cplx_of<T>::t C;
+   const int n = a.nbr[(size_t)(FWD ? 2 * MU : 2 * MU + 1) * a.V + x];
+   if (a.masked && n < 0)
+   {
+#pragma unroll
+      for (int k = 0; k < 6; k++) c[k] = cmk<C>(0, 0);
+      return;
+   }
+   const int y = n & 0x7fffffff;
+   C sp[12], h0[3], h1[3];
+   load_spinor(in, y, sp);
+   const C *up = odd ? link_ptr(a.u, x - a.h, FWD ? 2 * MU : 2 * MU + 1)
+                     : link_ptr(a.u, y - a.h, FWD ? 2 * MU + 1 : 2 * MU);
+   spin_project<C, MU, FWD>(sp, h0, h1);
+   C u[9];
+#pragma unroll
+   for (int k = 0; k < 9; k++) u[k] = up[k * SB];
+   su3_mul<C, !FWD>(u, h0, c);
+   su3_mul<C, !FWD>(u, h1, c + 3);
+}
+
+// z times a power of i: k = 0, 1, 2, 3 for 1, i, -1, -i
+template <typename C> __device__ inline C mul_ik(C z, int k)
+{
+   return k == 0 ? z : (k == 1 ? cmk<C>(-z.y, z.x) : (k == 2 ? cmk<C>(-z.x, -z.y) : cmk<C>(z.y, -z.x)));
+}
+
+// storage block of the work-group: consecutive blocks on one XCD (a
+// contiguous range for each), for Dw the even and the odd block of the same
+// offset one after the other
+template <int OP, typename T> __device__ inline int split_block(const DArgs<T> &a)
+{
+   const int b = xcd_tile(blockIdx.x, gridDim.x, 0);
+   if (OP != SP_DW || a.h % SB) return b;
+   return (b >> 1) + ((b & 1) ? a.h / SB : 0);
+}
+
+template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(DArgs<T> a)
+{
+   typedef typename cplx_of<T>::t C;
+   __shared__ C H[8][6][SB];
+   __shared__ C G[OP == SP_HAT1 ? 12 : 1][SB];
+   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & (SB - 1);
+   const int k = split_block<OP>(a) * SB + t;
+   const bool valid = k < a.np;
+   const int x = a.p0 + (valid ? k : 0);
+   const bool odd = x >= a.h;
+   const bool bp = a.masked && a.bnd[x];
+   const C *in = OP == SP_HAT2 ? (const C *)a.t : a.s;
+   // rows 2 wr, 2 wr + 1 of Weyl half hh are summed by wave 3 hh + wr
+   const int hh = w / 3, wr = w % 3;
+   C v[6], m[2][6];
+   if (w < 6 && valid)
+   {
+      const C *mp = a.sw + (size_t)(x >> 6) * (36 * SB) + (x & (SB - 1)) + (size_t)(18 * hh) * SB;
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+      {
+         const int i = 2 * wr + r;
+#pragma unroll
+         for (int j = 0; j < 6; j++)
+         {
+            // unit of the diagonal pair or of the entry (lo, hi) above the
+            // diagonal
+            const int lo = i < j ? i : j, hi = i < j ? j : i;
+            const int unit = i == j ? i >> 1 : 3 + 5 * lo - lo * (lo - 1) / 2 + hi - lo - 1;
+            m[r][j] = mp[unit * SB];
+         }
+      }
+      if (OP != SP_HAT1)
+      {
+         const C *vp = a.s + (size_t)(x >> 6) * (12 * SB) + (x & (SB - 1)) + (size_t)(6 * hh) * SB;
+#pragma unroll
+         for (int j = 0; j < 6; j++) v[j] = vp[j * SB];
+      }
+   }
+   C c[6];
+   switch (w)
+   {
+   case 0: split_hop<T, 0, true>(a, in, x, odd, c); break;
+   case 1: split_hop<T, 0, false>(a, in, x, odd, c); break;
+   case 2: split_hop<T, 1, true>(a, in, x, odd, c); break;
+   case 3: split_hop<T, 1, false>(a, in, x, odd, c); break;
+   case 4: split_hop<T, 2, true>(a, in, x, odd, c); break;
+   case 5: split_hop<T, 2, false>(a, in, x, odd, c); break;
+   case 6: split_hop<T, 3, true>(a, in, x, odd, c); break;
+   default: split_hop<T, 3, false>(a, in, x, odd, c);
+   }
+#pragma unroll
+   for (int q = 0; q < 6; q++) H[w][q][t] = c[q];
+   __syncthreads();
+   if (OP != SP_HAT1 && w >= 6) return;
+   C hs[2], out[2];
+   if (w < 6)
+   {
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+      {
+         const int i = 2 * wr + r, sp = i / 3, q = i % 3;
+         C z = cmk<C>(0, 0);
+         if (hh == 0)
+         {
+#pragma unroll
+            for (int d = 0; d < 8; d++) z = cadd(z, H[d][i][t]);
+         }
+         else
+         {
+            // lower components (spin_expand_add): spin 2 + sp takes the
+            // upper component sp (mu = 0, 3) or 1 - sp (mu = 1, 2) times a
+            // power of i, negative for backward terms
+            const int same = 3 * sp + q, other = 3 * (1 - sp) + q;
+            z = cadd(z, csub(H[0][same][t], H[1][same][t]));
+            z = cadd(z, mul_ik(csub(H[2][other][t], H[3][other][t]), 3));
+            z = cadd(z, mul_ik(csub(H[4][other][t], H[5][other][t]), sp ? 0 : 2));
+            z = cadd(z, mul_ik(csub(H[6][same][t], H[7][same][t]), sp ? 1 : 3));
+         }
+         hs[r] = cscale(z, a.coef);
+      }
+   }
+   if (OP == SP_HAT1)
+   {
+      if (w < 6)
+      {
+         G[6 * hh + 2 * wr][t] = hs[0];
+         G[6 * hh + 2 * wr + 1][t] = hs[1];
+      }
+      __syncthreads();
+      if (w >= 6) return;
+#pragma unroll
+      for (int j = 0; j < 6; j++) v[j] = G[6 * hh + j][t];
+      hs[0] = hs[1] = cmk<C>(0, 0);
+   }
+   if (!valid) return;
+   const T mm = OP == SP_HAT1 ? (T)0 : (odd ? a.muo : a.mu);
+   const T mu = hh ? -mm : mm;
+#pragma unroll
+   for (int r = 0; r < 2; r++)
+   {
+      const int i = 2 * wr + r;
+      C o = hs[r];
+#pragma unroll
+      for (int j = 0; j < 6; j++)
+      {
+         if (i == j)
+         {
+            const T d = (i & 1) ? m[r][j].y : m[r][j].x;
+            o = cadd(o, cmk<C>(d * v[j].x - mu * v[j].y, d * v[j].y + mu * v[j].x));
+         }
+         else
+            o = cadd(o, i < j ? cmul(m[r][j], v[j]) : cmulc(m[r][j], v[j]));
+      }
+      out[r] = o;
+   }
+   // boundary points of open bc are zeroed in output and (Dw) input
+   if (bp) out[0] = out[1] = cmk<C>(0, 0);
+   C *op = (OP == SP_HAT1 ? a.t : a.r) + (size_t)(x >> 6) * (12 * SB) + (x & (SB - 1)) +
+           (size_t)(6 * hh + 2 * wr) * SB;
+   op[0] = out[0];
+   op[SB] = out[1];
+   if (OP == SP_DW && bp)
+   {
+      C *ip = a.s_w + (size_t)(x >> 6) * (12 * SB) + (x & (SB - 1)) + (size_t)(6 * hh + 2 * wr) * SB;
+      ip[0] = ip[SB] = cmk<C>(0, 0);
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -799,28 +908,66 @@ template <typename T> static DArgs<T> base_args()
 
 template <typename T, int OP> static void launch(const DArgs<T> &a)
 {
-   Lib &L = lib();
-#if OQH_DW_TILE
-   if (OP == OP_DW)
-   {
-      constexpr int TP = TileSize<T>::n;
-      unsigned nt = (unsigned)((a.h + TP - 1) / TP);
-      if (!nt) return;
-      const bool sws = a.sws_par == 3;
-      if (a.lsign && sws)
-         k_dw_tile<T, TP, true, true><<<nt, TP, 0, L.stream>>>(a);
-      else if (a.lsign)
-         k_dw_tile<T, TP, true, false><<<nt, TP, 0, L.stream>>>(a);
-      else if (sws)
-         k_dw_tile<T, TP, false, true><<<nt, TP, 0, L.stream>>>(a);
-      else
-         k_dw_tile<T, TP, false, false><<<nt, TP, 0, L.stream>>>(a);
-      return;
-   }
-#endif
-   unsigned nb = (OP == OP_DW) ? (unsigned)((a.h + 127) / 128) : (unsigned)((a.np + 255) / 256);
+   unsigned nb = (unsigned)((a.np + 255) / 256);
    if (nb == 0) return;
-   k_dirac<T, OP><<<nb, 256, 0, L.stream>>>(a);
+   k_dirac<T, OP><<<nb, 256, 0, lib().stream>>>(a);
+}
+
+enum { K_DW, K_DEE, K_DOO, K_DOE, K_DEO, K_HAT };
+
+// the split kernel up to this many pairs of points, tiles above.  Measured
+// (us, split / tile): FP64 Dw 5.1 / 27.2 at 2048 pairs, 26.6 / 42.2 at 32768,
+// 38.4 / 46.1 at 49152, 54.2 / 49.6 at 58320, 90 / 73 at 97200; FP32 Dw 5.1 /
+// 21.8, 13.0 / 32.1, 18.2 / 33.6, 26.2 / 36.9, 41.1 / 44.7, then 63.4 / 57.5 at
+// 165888; Dwhat the same lines (FP64 45.7 / 45.8 at 49152, FP32 42 / 51 at
+// 97200, 65 / 68 at 165888).  Tiles of 64 or 128 pairs are nowhere more than
+// 5 % better than the better of the two, but for FP64 Dwhat at 49152 (41 us).
+static bool use_split(int prec, int h) { return h <= (prec == F64 ? 49152 : 131072); }
+
+template <typename T> static void launch_dw(const DArgs<T> &a)
+{
+   constexpr int TP = TileSize<T>::n;
+   hipStream_t st = lib().stream;
+   const unsigned nt = (unsigned)((a.h + TP - 1) / TP);
+   const bool sws = a.sws_par == 3;
+   if (a.lsign && sws)
+      k_dw_tile<T, TP, true, true><<<nt, TP, 0, st>>>(a);
+   else if (a.lsign)
+      k_dw_tile<T, TP, true, false><<<nt, TP, 0, st>>>(a);
+   else if (sws)
+      k_dw_tile<T, TP, false, true><<<nt, TP, 0, st>>>(a);
+   else
+      k_dw_tile<T, TP, false, false><<<nt, TP, 0, st>>>(a);
+}
+
+// the two passes of Dwhat; a.coef = 1/2, a.mu for the second
+template <typename T> static void launch_hat(const DArgs<T> &a)
+{
+   constexpr int TP = TileSize<T>::n;
+   hipStream_t st = lib().stream;
+   const unsigned nt = (unsigned)((a.h + TP - 1) / TP);
+   DArgs<T> a1 = a;
+   a1.coef = -a.coef;
+   if (a.lsign)
+      k_hat1_tile<T, TP, true><<<nt, TP, 0, st>>>(a1);
+   else
+      k_hat1_tile<T, TP, false><<<nt, TP, 0, st>>>(a1);
+   const bool sws = a.sws_par & 1;  // A_ee uninverted
+   if (a.lsign && sws)
+      k_hat2_tile<T, TP, true, true><<<nt, TP, 0, st>>>(a);
+   else if (a.lsign)
+      k_hat2_tile<T, TP, true, false><<<nt, TP, 0, st>>>(a);
+   else if (sws)
+      k_hat2_tile<T, TP, false, true><<<nt, TP, 0, st>>>(a);
+   else
+      k_hat2_tile<T, TP, false, false><<<nt, TP, 0, st>>>(a);
+}
+
+template <typename T, int OP> static void launch_split(DArgs<T> a, int p0, int np)
+{
+   a.p0 = p0;
+   a.np = np;
+   k_split<T, OP><<<(unsigned)((np + SB - 1) / SB), 8 * SB, 0, lib().stream>>>(a);
 }
 
 template <typename T> static void zero_bnd(typename cplx_of<T>::t *s, int p0, int np)
@@ -852,8 +999,6 @@ static bool prepare(const char *where, int prec)
    }
    return true;
 }
-
-enum { K_DW, K_DEE, K_DOO, K_DOE, K_DEO, K_HAT };
 
 template <typename T> static void apply(int kind, T mu, void *sp, void *rp, const char *where)
 {
@@ -887,7 +1032,10 @@ template <typename T> static void apply(int kind, T mu, void *sp, void *rp, cons
       a.mu = mu;
       a.muo = muo;
       a.coef = (T)-0.5;
-      launch<T, OP_DW>(a);
+      if (use_split(prec, h))
+         launch_split<T, SP_DW>(a, 0, V);
+      else
+         launch_dw<T>(a);
       break;
    case K_DEE:
       a.mu = mu;
@@ -919,38 +1067,17 @@ template <typename T> static void apply(int kind, T mu, void *sp, void *rp, cons
    {
       // odd intermediate t = A_oo^-1 (-1/2 hop(s_e)) in a scratch field
       a.t = (C *)tmp_buffer(units_for(V, 12) * sizeof(C));
-#if OQH_HAT_TILE
-      {
-         constexpr int TPn = TileSize<T>::n;
-         unsigned nt = (unsigned)((h + TPn - 1) / TPn);
-         a.coef = (T)-0.5;
-         if (a.lsign)
-            k_hat1_tile<T, TileSize<T>::n, true><<<nt, TPn, 0, L.stream>>>(a);
-         else
-            k_hat1_tile<T, TileSize<T>::n, false><<<nt, TPn, 0, L.stream>>>(a);
-         a.coef = (T)0.5;
-         a.mu = mu;
-         const bool sws = a.sws_par & 1;  // A_ee uninverted
-         if (a.lsign && sws)
-            k_hat2_tile<T, TileSize<T>::n, true, true><<<nt, TPn, 0, L.stream>>>(a);
-         else if (a.lsign)
-            k_hat2_tile<T, TileSize<T>::n, true, false><<<nt, TPn, 0, L.stream>>>(a);
-         else if (sws)
-            k_hat2_tile<T, TileSize<T>::n, false, true><<<nt, TPn, 0, L.stream>>>(a);
-         else
-            k_hat2_tile<T, TileSize<T>::n, false, false><<<nt, TPn, 0, L.stream>>>(a);
-      }
-#else
-      a.coef = (T)-0.5;
-      a.p0 = h;
-      a.np = h;
-      launch<T, OP_HAT1>(a);
       a.coef = (T)0.5;
       a.mu = mu;
-      a.p0 = 0;
-      a.np = h;
-      launch<T, OP_HAT2>(a);
-#endif
+      if (use_split(prec, h))
+      {
+         DArgs<T> a1 = a;
+         a1.coef = (T)-0.5;
+         launch_split<T, SP_HAT1>(a1, h, h);
+         launch_split<T, SP_HAT2>(a, 0, h);
+      }
+      else
+         launch_hat<T>(a);
       zero_bnd<T>((C *)s.dev, 0, h);   // cps(d)_int_bnd side effect
       break;
    }
