@@ -592,9 +592,26 @@ template <typename S> struct RegBlock
    }
 };
 
-// out = (A + i mu) v on the two Weyl halves (pauli_half); the half hh = 0
-// of A is read at m0 with stride st0, the half hh = 1 at m1 with stride st1
-// (registers or LDS)
+// o = (A + i mu) w on one Weyl half (pauli_half), the 18 units of A in q
+__device__ inline void pauli_half_reg(const float2 *q, float mu, const float2 *w, float2 *o)
+{
+   float d[6] = {q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y};
+#pragma unroll
+   for (int i = 0; i < 6; i++) o[i] = make_float2(d[i] * w[i].x - mu * w[i].y, d[i] * w[i].y + mu * w[i].x);
+   int p = 3;
+#pragma unroll
+   for (int i = 0; i < 6; i++)
+#pragma unroll
+      for (int j = i + 1; j < 6; j++)
+      {
+         o[i] = cmac(o[i], q[p], w[j]);
+         o[j] = cmacc(o[j], q[p], w[i]);
+         p++;
+      }
+}
+
+// both Weyl halves; the half hh = 0 of A is read at m0 with stride st0, the
+// half hh = 1 at m1 with stride st1 (registers or LDS)
 template <typename S>
 __device__ inline void pauli_reg2(const S *m0, int st0, const S *m1, int st1, float mu, const float2 *v, float2 *out)
 {
@@ -606,30 +623,8 @@ __device__ inline void pauli_reg2(const S *m0, int st0, const S *m1, int st1, fl
       const int stride = hh ? st1 : st0;
 #pragma unroll
       for (int k = 0; k < 18; k++) q[k] = to_f2(m[k * stride]);
-      const float2 *w = v + 6 * hh;
-      float2 *o = out + 6 * hh;
-      float mm = hh ? -mu : mu;
-      float d[6] = {q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y};
-#pragma unroll
-      for (int i = 0; i < 6; i++) o[i] = make_float2(d[i] * w[i].x - mm * w[i].y, d[i] * w[i].y + mm * w[i].x);
-      int p = 3;
-#pragma unroll
-      for (int i = 0; i < 6; i++)
-#pragma unroll
-         for (int j = i + 1; j < 6; j++)
-         {
-            float2 hij = q[p];
-            o[i] = cmac(o[i], hij, w[j]);
-            o[j] = cmacc(o[j], hij, w[i]);
-            p++;
-         }
+      pauli_half_reg(q, hh ? -mu : mu, v + 6 * hh, out + 6 * hh);
    }
-}
-
-template <typename S>
-__device__ inline void pauli_reg(const S *m, float mu, const float2 *v, float2 *out, int stride = 1)
-{
-   pauli_reg2(m, stride, m + 18 * stride, stride, mu, v, out);
 }
 
 template <int MU, bool FWD> __device__ inline void weyl_project(const float2 *sp, float2 *h)
@@ -1149,6 +1144,286 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
 #ifndef OQH_FACE_GROUP
 #define OQH_FACE_GROUP 4
 #endif
+
+// ---------------------------------------------------------------------------
+// the Schwarz sweep with the block's spinors on the chip (blocks of up to
+// 1365 points other than 4^4, FP32)
+//
+// Lane i of the work-group owns the even point i and the odd point bh + i of
+// the block.  The block fields s0, s1 stay in its registers; the source of a
+// hopping pass, one parity, lies in LDS (96 bytes per point), where the output
+// lanes gather all eight neighbours.  Links and SW matrices are too many for
+// the chip (600 bytes per point) and are streamed, each once per pass and
+// parity: 864 bytes per point and MinRes step, against 1350 and more of
+// k_sap_blocks, whose fields also pass through global memory.
+// Per cycle (us, k_sap_lds / k_sap_blocks, nmr = 4): 8x4^3 blocks on 16x8^3
+// 146 / 231, on 32^3x16 445 / 680; 8^2x4^2 on 16^2x8^2 203 / 413, on 32^3x16
+// 464 / 830; 4x6^3 on 16x24^3 348 / 675; 6^4 on 12^4 351 / 622, on 36^2x24^2
+// 1359 / 2119 (12 wavefronts, 168 registers, 21 spilled).
+// ---------------------------------------------------------------------------
+
+constexpr int BLV_MAX = 1365;  // points of a block, two per lane: 64 KiB of LDS
+
+// acc += hopping terms into block point i (global point gx) of parity ODD
+// from the values F of the other parity
+template <int MU, bool FWD, bool ODD>
+__device__ inline void lds_hop_one(const SArgs &a, const int *imb, const float2 *F, int i, int gx, float2 *acc)
+{
+   const int j = a.bnb[(2 * MU + (FWD ? 0 : 1)) * a.bvol + i];
+   if (j >= a.bvol) return;
+   const float2 *up = ODD ? link_ptr(a.u, gx - a.h, FWD ? 2 * MU : 2 * MU + 1)
+                          : link_ptr(a.u, imb[j] - a.h, FWD ? 2 * MU + 1 : 2 * MU);
+   float2 u[9], sp[12], h[6], c[6];
+#pragma unroll
+   for (int k = 0; k < 9; k++) u[k] = up[k * SB];
+   const float2 *f = F + (ODD ? j : j - a.bh);
+#pragma unroll
+   for (int k = 0; k < 12; k++) sp[k] = f[k * a.bh];
+   spin_project<float2, MU, FWD>(sp, h, h + 3);
+   su3_mul_f<!FWD>(u, h, c);
+   su3_mul_f<!FWD>(u, h + 3, c + 3);
+   spin_expand_add<float2, MU, FWD>(c, c + 3, acc);
+}
+
+// the loads of a direction stay within it: the compiler would otherwise move
+// those of all eight ahead and spill the block fields
+template <bool ODD, bool WIDE>
+__device__ inline void lds_hop(const SArgs &a, const int *imb, const float2 *F, int i, int gx, float2 *acc)
+{
+   zero12(acc);
+#define OQH_LDS_HOP(MU)                                                \
+   lds_hop_one<MU, true, ODD>(a, imb, F, i, gx, acc);                  \
+   if (!WIDE) __builtin_amdgcn_sched_barrier(0);                       \
+   lds_hop_one<MU, false, ODD>(a, imb, F, i, gx, acc);                 \
+   __builtin_amdgcn_sched_barrier(0);
+   OQH_LDS_HOP(0)
+   OQH_LDS_HOP(1)
+   OQH_LDS_HOP(2)
+   OQH_LDS_HOP(3)
+#undef OQH_LDS_HOP
+}
+
+__device__ inline void lds_put(float2 *F, int bh, int i, const float2 *v)
+{
+#pragma unroll
+   for (int c = 0; c < 12; c++) F[c * bh + i] = v[c];
+}
+
+// o = (A + i mu gamma5) v at global point gx, one Weyl half after the other
+__device__ inline void lds_pauli(const SArgs &a, int gx, float mu, const float2 *v, float2 *o)
+{
+   const float2 *m = a.sw + (size_t)(gx >> 6) * (36 * SB) + (gx & (SB - 1));
+#pragma unroll
+   for (int hh = 0; hh < 2; hh++)
+   {
+      float2 q[18];
+#pragma unroll
+      for (int k = 0; k < 18; k++) q[k] = m[(18 * hh + k) * SB];
+      pauli_half_reg(q, hh ? -mu : mu, v + 6 * hh, o + 6 * hh);
+      __builtin_amdgcn_sched_barrier(0);
+   }
+}
+
+// |s2|^2 and (s2, s1) of a point, added as in blk_mres_dev
+__device__ inline void point_sums(const float2 *s2, const float2 *s1, double &rr, double &zr, double &zi)
+{
+#pragma unroll
+   for (int k = 0; k < 4; k++)
+   {
+      float nr = 0.0f, pr = 0.0f, pi = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+      {
+         float2 u = s2[3 * k + c], v = s1[3 * k + c];
+         nr += u.x * u.x + u.y * u.y;
+         pr += u.x * v.x + u.y * v.y;
+         pi += u.x * v.y - u.y * v.x;
+      }
+      rr += (double)nr;
+      zr += (double)pr;
+      zi += (double)pi;
+   }
+}
+
+// psi += s0 (or = s0 for pz), rho = s1, correction s0 of one point
+__device__ inline void lds_store(const SArgs &a, int gx, const float2 *s0, const float2 *s1)
+{
+   float2 p[12];
+   if (a.pz)
+   {
+#pragma unroll
+      for (int c = 0; c < 12; c++) p[c] = s0[c];
+   }
+   else
+   {
+      load_spinor((const float2 *)a.psi, gx, p);
+#pragma unroll
+      for (int c = 0; c < 12; c++) p[c] = cadd(p[c], s0[c]);
+   }
+   store_spinor(a.psi, gx, p);
+   store_spinor(a.rho, gx, s1);
+   store_spinor(a.s0g, gx, s0);
+}
+
+template <int ISOLV, int TPB, bool MASKED>
+__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(TPB <= 512 ? 2 : 3))) void k_sap_lds(SArgs a)
+{
+   extern __shared__ float2 F[];  // [12][bh]
+   constexpr bool WIDE = TPB <= 512 && ISOLV;
+   const int n = a.n0 + blockIdx.x, bh = a.bh, i = threadIdx.x;
+   const int *imb = a.imb + (size_t)n * a.bvol;
+   const bool own = i < bh;  // lanes without points take part in the barriers
+   int ge = imb[own ? i : 0], go = imb[own ? bh + i : bh];
+   const bool be = MASKED && a.bnd[ge], bo = MASKED && a.bnd[go];
+   const float2 zero = make_float2(0.0f, 0.0f);
+   float2 s0[12], s1[12], w[12];
+   // ISOLV = 0: the odd point's fields
+   float2 t0[ISOLV ? 1 : 12], t1[ISOLV ? 1 : 12], tw[ISOLV ? 1 : 12];
+   zero12(s0);
+   zero12(s1);
+   if (ISOLV)
+   {
+      // odd points: A_oo^-1 rho, then even points: s1 = rho + 1/2 hops
+      if (own)
+      {
+         float2 o[12];
+         load_spinor((const float2 *)a.rho, go, w);
+         lds_pauli(a, go, 0.0f, w, o);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = bo ? zero : o[c];
+         lds_put(F, bh, i, w);
+         load_spinor((const float2 *)a.rho, ge, s1);
+      }
+      __syncthreads();
+      if (own)
+      {
+         lds_hop<false, WIDE>(a, imb, F, i, ge, w);
+#pragma unroll
+         for (int c = 0; c < 12; c++) s1[c] = be ? zero : cadd(s1[c], cscale(w[c], 0.5f));
+      }
+      __syncthreads();
+   }
+   else if (own)
+   {
+      load_spinor((const float2 *)a.rho, ge, s1);
+      load_spinor((const float2 *)a.rho, go, t1);
+      zero12(t0);
+#pragma unroll
+      for (int c = 0; c < 12; c++)
+      {
+         if (be) s1[c] = zero;
+         if (bo) t1[c] = zero;
+      }
+   }
+
+   // minimal residual steps (blk_solv.c:1117-1186): w = D s1
+   for (int imr = 0; imr < a.nmr; imr++)
+   {
+      double rr = 0.0, zr = 0.0, zi = 0.0;
+      // links and matrices are read again in every step: without this the
+      // compiler loads them once, before the loop, and spills them
+      asm volatile("" : "+v"(ge), "+v"(go), "+s"(a.bnb));
+      if (own) lds_put(F, bh, i, s1);
+      __syncthreads();
+      if (ISOLV)
+      {
+         float2 o[12];
+         if (own)
+         {
+            lds_hop<true, WIDE>(a, imb, F, bh + i, go, w);
+#pragma unroll
+            for (int c = 0; c < 12; c++) w[c] = cscale(w[c], -0.5f);
+            lds_pauli(a, go, 0.0f, w, o);
+#pragma unroll
+            for (int c = 0; c < 12; c++) o[c] = bo ? zero : o[c];
+         }
+         __syncthreads();
+         if (own) lds_put(F, bh, i, o);
+         __syncthreads();
+         if (own)
+         {
+            lds_hop<false, WIDE>(a, imb, F, i, ge, w);
+            lds_pauli(a, ge, a.mu, s1, o);
+#pragma unroll
+            for (int c = 0; c < 12; c++) w[c] = be ? zero : cadd(o[c], cscale(w[c], 0.5f));
+            point_sums(w, s1, rr, zr, zi);
+         }
+      }
+      else
+      {
+         float2 o[12];
+         if (own)
+         {
+            lds_hop<true, WIDE>(a, imb, F, bh + i, go, tw);
+            lds_pauli(a, go, a.muo, t1, o);
+#pragma unroll
+            for (int c = 0; c < 12; c++) tw[c] = bo ? zero : cadd(o[c], cscale(tw[c], -0.5f));
+            point_sums(tw, t1, rr, zr, zi);
+         }
+         __syncthreads();
+         if (own) lds_put(F, bh, i, t1);
+         __syncthreads();
+         if (own)
+         {
+            lds_hop<false, WIDE>(a, imb, F, i, ge, w);
+            lds_pauli(a, ge, a.mu, s1, o);
+#pragma unroll
+            for (int c = 0; c < 12; c++) w[c] = be ? zero : cadd(o[c], cscale(w[c], -0.5f));
+            point_sums(w, s1, rr, zr, zi);
+         }
+      }
+      wg_sum3(rr, zr, zi, TPB);
+      float r = (float)rr;
+      if (r < 2.0f * FLT_MIN) break;
+      r = 1.0f / r;
+      const float2 z = make_float2((float)zr * r, (float)zi * r), mz = make_float2(-z.x, -z.y);
+      if (own)
+      {
+#pragma unroll
+         for (int c = 0; c < 12; c++)
+         {
+            s0[c] = cmac(s0[c], z, s1[c]);
+            s1[c] = cmac(s1[c], mz, w[c]);
+            if (!ISOLV)
+            {
+               t0[c] = cmac(t0[c], z, t1[c]);
+               t1[c] = cmac(t1[c], mz, tw[c]);
+            }
+         }
+      }
+   }
+
+   if (ISOLV)
+   {
+      // odd solution A_oo^-1 (rho_o + 1/2 hops of s0_e), odd residual
+      // -i mu gamma5 s0 (update_flds1) or 0 (eoflg, update_flds2)
+      __syncthreads();
+      if (own) lds_put(F, bh, i, s0);
+      __syncthreads();
+      if (!own) return;
+      lds_store(a, ge, s0, s1);
+      float2 v[12], o[12];
+      lds_hop<true, WIDE>(a, imb, F, bh + i, go, w);
+      load_spinor((const float2 *)a.rho, go, v);
+#pragma unroll
+      for (int c = 0; c < 12; c++) v[c] = cadd(v[c], cscale(w[c], 0.5f));
+      lds_pauli(a, go, 0.0f, v, o);
+      const float m = a.eoflg ? 0.0f : a.mu;
+#pragma unroll
+      for (int c = 0; c < 12; c++)
+      {
+         if (bo) o[c] = zero;
+         const float cm = (c < 6) ? -m : m;
+         v[c] = make_float2(-cm * o[c].y, cm * o[c].x);
+      }
+      lds_store(a, go, o, v);
+   }
+   else if (own)
+   {
+      lds_store(a, ge, s0, s1);
+      lds_store(a, go, t0, t1);
+   }
+}
 
 // rho(y) -= hopping terms into y from the block corrections of the
 // neighbouring blocks, for the face points y of the blocks of one colour
@@ -1686,6 +1961,23 @@ static bool half_variant()
           G.d_swb16;
 }
 
+// the block's spinors fit on the chip (k_sap_lds)
+static bool lds_kernel() { return G.bvol != RBV && G.bvol <= BLV_MAX; }
+
+template <int TPB> static void launch_lds(const SArgs &a, int isolv, unsigned nb)
+{
+   hipStream_t st = lib().stream;
+   const size_t lds = (size_t)12 * G.bh * sizeof(float2);
+   if (isolv && a.masked)
+      k_sap_lds<1, TPB, true><<<nb, TPB, lds, st>>>(a);
+   else if (isolv)
+      k_sap_lds<1, TPB, false><<<nb, TPB, lds, st>>>(a);
+   else if (a.masked)
+      k_sap_lds<0, TPB, true><<<nb, TPB, lds, st>>>(a);
+   else
+      k_sap_lds<0, TPB, false><<<nb, TPB, lds, st>>>(a);
+}
+
 // block solves of the blocks of colour ic; the register kernel first adds
 // the terms of the other colour's face fields if pull is set
 static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
@@ -1717,19 +2009,21 @@ static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
       else
          k_sap_reg<0, float2, false><<<nb, RBV, 0, L.stream>>>(a, nullptr, nullptr);
    }
-   else if (G.bvol >= SWG_MAX)
+   else if (lds_kernel())
    {
-      // large blocks (6^4, 8^4): 1024 threads per block, the few blocks of a
-      // small lattice would otherwise leave most of the chip idle
-      if (isolv)
-         k_sap_blocks<1, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
+      if (G.bh <= 256)
+         launch_lds<256>(a, isolv, nb);
+      else if (G.bh <= 512)
+         launch_lds<512>(a, isolv, nb);
       else
-         k_sap_blocks<0, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
+         launch_lds<768>(a, isolv, nb);
    }
    else if (isolv)
-      k_sap_blocks<1><<<nb, SWG, 0, L.stream>>>(a);
+      // 1024 threads per block: the few blocks of a lattice would otherwise
+      // leave most of the chip idle
+      k_sap_blocks<1, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
    else
-      k_sap_blocks<0><<<nb, SWG, 0, L.stream>>>(a);
+      k_sap_blocks<0, float2, SWG_MAX><<<nb, SWG_MAX, 0, L.stream>>>(a);
 }
 
 // face terms from the corrections of the colour-(1-c) blocks into rho on
@@ -1931,7 +2225,7 @@ void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho,
    a.rho = rho;
    const int V = L.g.V;
    const unsigned nbk = (V + 255) / 256;
-   const bool pz = zero && reg_kernel();
+   const bool pz = zero && (reg_kernel() || lds_kernel());
    if (zero && !pz) HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
    if (half_variant())
    {
