@@ -6,7 +6,11 @@
 // and the SAP_BLOCKS parts of block/blk_grid.c, map_u2blk.c, map_sw2blk.c and
 // map_s2blk.c.
 //
-// One work-group handles one block of the current colour.  The block's three
+// Blocks of 4^4 points are held in the registers of a work-group (k_sap_reg),
+// larger ones of multiples of 4 in those of several (k_sap_cluster), other
+// blocks of up to 1365 points in the registers and LDS of one (k_sap_lds).  For
+// the rest and in FP64 (k_sap_blocks) one work-group handles one block of the
+// current colour, and the block's three
 // fields (solution s0, residual s1, work s2) are kept block-compact in a
 // scratch area (site-block layout over the block-local point index, even
 // points first, as the reference's block geometry, lattice/blk_geometry.c);
@@ -69,6 +73,12 @@ struct SapGrid
    float2 *d_wfm = nullptr;              // those of several sources
    int wfm_n = 0;                        // number of sources in d_wfm
    int *d_nbn = nullptr;                 // neighbouring blocks [nb][8] (4^4 blocks)
+   int ns = 0;                           // 4^4 sub-blocks per block (k_sap_cluster) or 0
+   std::vector<int> imb4;                // points of the sub-blocks [nb][ns][256]
+   int *d_imb4 = nullptr, *d_nbs = nullptr;
+   unsigned *d_count = nullptr;          // ticket and arrival counters
+   unsigned long long *d_x = nullptr;    // exchange buffers, sums
+   int *h_dead = nullptr;                // host flag of k_sap_cluster
    double2 *d_swb64 = nullptr;           // FP64 block SW field (FP64 variant)
    int swb64_version = -1;
    double2 *d_h64[3] = {nullptr, nullptr, nullptr};  // FP64 psi, rho, s0g
@@ -636,9 +646,17 @@ template <int MU, bool FWD> __device__ inline void weyl_project(const float2 *sp
 // in-block neighbours (src of the lanes of the other parity, zero on the
 // boundary points of open bc) are added to w of the lanes of parity OUT,
 // forward terms of mu = 0..3, then backward terms.  src and w may be the same
-// registers.  lb: LDS of 18 * RBV float2.
-template <int OUT, typename S>
-__device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w, float2 *lb)
+// registers.  lb: LDS of 18 * RBV float2.  hook.put() and hook.sent() are called
+// by the source lanes once their values are in LDS and once they have formed
+// their terms, hook.take() by the output lanes at the end.
+struct NoHook
+{
+   __device__ void put() const {}
+   __device__ void sent() const {}
+   __device__ void take() const {}
+};
+template <int OUT, typename S, typename HOOK = NoHook>
+__device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w, float2 *lb, const HOOK &hook = HOOK())
 {
    constexpr int RBH = RBV / 2;
    float2(*F)[RBH] = (float2(*)[RBH])lb;
@@ -651,6 +669,7 @@ __device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w
       for (int c = 0; c < 12; c++) F[c][i] = src[c];
    }
    __syncthreads();
+   if (!own) hook.put();
 #pragma unroll
    for (int mu = 0; mu < 4; mu++)
    {
@@ -689,6 +708,7 @@ __device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w
          }
       }
    }
+   if (!own) hook.sent();
    __syncthreads();
    if (own)
    {
@@ -706,6 +726,7 @@ __device__ inline void rb_hop(const RegBlock<S> &b, const float2 *src, float2 *w
             if (mu == 3) spin_expand_add<float2, 3, false>(c, c + 3, w);
          }
       }
+      hook.take();
    }
 }
 
@@ -778,8 +799,9 @@ __device__ inline size_t face_unit(int n, int f) { return ((size_t)n * 8 + f) * 
 
 // acc += hopping terms into the point from outside the block, from the face
 // fields of the neighbouring blocks nbn[0..7] (forward neighbours 2 mu,
-// backward neighbours 2 mu + 1)
-template <typename S>
+// backward neighbours 2 mu + 1; SUB: a sub-block, negative where the face lies
+// inside the block)
+template <bool SUB = false, typename S>
 __device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int *nbn, float2 *acc)
 {
    // all loads first: a point lies on at most one of the faces of a
@@ -789,7 +811,7 @@ __device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int 
    for (int mu = 0; mu < 4; mu++)
    {
       const int x = b.coord(mu);
-      if (x == 3 || x == 0)
+      if ((x == 3 && !(SUB && nbn[2 * mu] < 0)) || (x == 0 && !(SUB && nbn[2 * mu + 1] < 0)))
       {
          const size_t f = (x == 3) ? face_unit(nbn[2 * mu], 2 * mu + 1) : face_unit(nbn[2 * mu + 1], 2 * mu);
          const float2 *p = W + f + b.face_point(mu, !b.odd);
@@ -801,7 +823,7 @@ __device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int 
    for (int mu = 0; mu < 4; mu++)
    {
       const int x = b.coord(mu);
-      if (x == 3)
+      if (x == 3 && !(SUB && nbn[2 * mu] < 0))
       {
          float2 c[6], u[9];
 #pragma unroll
@@ -813,7 +835,7 @@ __device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int 
          if (mu == 2) spin_expand_add<float2, 2, true>(c, c + 3, acc);
          if (mu == 3) spin_expand_add<float2, 3, true>(c, c + 3, acc);
       }
-      else if (x == 0)
+      else if (x == 0 && !(SUB && nbn[2 * mu + 1] < 0))
       {
          if (mu == 0) spin_expand_add<float2, 0, false>(h[mu], h[mu] + 3, acc);
          if (mu == 1) spin_expand_add<float2, 1, false>(h[mu], h[mu] + 3, acc);
@@ -823,14 +845,15 @@ __device__ inline void rb_pull(const RegBlock<S> &b, const float2 *W, const int 
    }
 }
 
-// the block's face fields from its correction s0
-template <typename S> __device__ inline void rb_push(const RegBlock<S> &b, const float2 *s0, float2 *W, int n)
+// the block's face fields from its correction s0, towards the neighbours nbn
+template <bool SUB = false, typename S>
+__device__ inline void rb_push(const RegBlock<S> &b, const float2 *s0, float2 *W, int n, const int *nbn)
 {
 #pragma unroll
    for (int mu = 0; mu < 4; mu++)
    {
       const int x = b.coord(mu);
-      if (x == 3)
+      if (x == 3 && !(SUB && nbn[2 * mu] < 0))
       {
          float2 h[6], c[6], u[9];
 #pragma unroll
@@ -845,7 +868,7 @@ template <typename S> __device__ inline void rb_push(const RegBlock<S> &b, const
 #pragma unroll
          for (int k = 0; k < 6; k++) p[k * FPT] = c[k];
       }
-      else if (x == 0)
+      else if (x == 0 && !(SUB && nbn[2 * mu + 1] < 0))
       {
          float2 h[6];
          if (mu == 0) weyl_project<0, true>(s0, h);
@@ -1072,7 +1095,7 @@ float2 o[12];
       }
    }
 
-   rb_push(b, s0, a.wf, n);
+   rb_push(b, s0, a.wf, n, a.nbn + 8 * (size_t)n);
    if (a.pz)
    {
 #pragma unroll
@@ -1109,9 +1132,9 @@ float2 o[12];
 }
 
 // rho += hopping terms from the face fields of the neighbouring blocks for
-// the blocks from n0 on: completes the residual after the last block solves
+// the 4^4 blocks or sub-blocks (points imb) from n0 on: completes the residual after the last block solves
 template <typename S>
-__global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
+__global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const int *imb, const S *u16)
 {
    constexpr bool H = sizeof(S) == 4;
    const int src = a0.nsrc ? (int)(blockIdx.x % a0.nsrc) : 0;
@@ -1123,7 +1146,7 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
       a.wf = a0.wl[src];
    }
    const int n = a.n0 + bi;
-   const int gx = a.imb[(size_t)n * RBV + threadIdx.x];
+   const int gx = imb[(size_t)n * RBV + threadIdx.x];
    RegBlock<S> b;
    rb_load<S, false, true>(a, H ? u16 : (const S *)a.u, threadIdx.x, gx, b);
    float2 r[12], acc[12];
@@ -1132,7 +1155,7 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
    else
       load_spinor((const float2 *)a.rho, gx, r);
    zero12(acc);
-   rb_pull(b, a.wf, a.nbn + 8 * (size_t)n, acc);
+   rb_pull<true>(b, a.wf, a.nbn + 8 * (size_t)n, acc);
 #pragma unroll
    for (int c = 0; c < 12; c++) r[c] = cadd(r[c], cscale(acc[c], 0.5f));
    if (H)
@@ -1146,8 +1169,425 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
 #endif
 
 // ---------------------------------------------------------------------------
+// the Schwarz sweep with a block shared by several work-groups (block sizes
+// that are multiples of 4, FP32)
+//
+// The block is cut into sub-blocks of 4^4 points, each held in the registers of
+// one work-group as in k_sap_reg.  In every hopping pass the work-groups of a
+// block pass the Weyl fields on their common faces (those of rb_push, the
+// points of one parity) through global memory, and for every MinRes step
+// their shares of the block sums.
+//
+// Which sub-block a work-group takes is decided by a ticket drawn when it
+// starts to run, block by block, so at any time all but the last block begun
+// have all their work-groups running and can finish; the last one gets its
+// missing work-groups as the others end.  A block needs only as many
+// work-groups running at once as it has sub-blocks (at most CLMAX, far fewer
+// than the device holds), and no wait depends on the order in which
+// work-groups are started.  Waits are bounded all the same: a work-group that
+// has waited CLSPIN times gives up waiting for good and reports it.
+//
+// The exchanged values are written and read with relaxed atomics of device
+// scope; a work-group counts itself in after its writes have completed.  Two
+// exchange buffers alternate: who writes the one of pass k + 2 has seen
+// everybody arrive in pass k + 1, that is, done with reading pass k.
+//
+// Per cycle (us, nmr = 4; k_sap_cluster / k_sap_lds or, for 8^4, k_sap_blocks):
+// 8^4 blocks on 16^4 213 / 1436, on 32^4 1100 / 2605, on 32^3x64 2190 / 3700;
+// 8x4^3 on 16x8^3 132 / 146, on 32^3x16 388 / 446; 8^2x4^2 on 16^2x8^2 149 /
+// 203, on 32^3x16 436 / 463.  Bound by the 14 exchanges of a block solve, about
+// 3.5 us each (write, count, poll, read).  With the counters of all blocks in
+// one line they took 20 us (8^4 on 32^4: 3400).
+// ---------------------------------------------------------------------------
+
+// psi += s0 (or = s0 for pz), rho = s1, correction s0 (if asked for) of one point
+template <bool COR> __device__ inline void lds_store(const SArgs &a, int gx, const float2 *s0, const float2 *s1)
+{
+   float2 p[12];
+   if (a.pz)
+   {
+#pragma unroll
+      for (int c = 0; c < 12; c++) p[c] = s0[c];
+   }
+   else
+   {
+      load_spinor((const float2 *)a.psi, gx, p);
+#pragma unroll
+      for (int c = 0; c < 12; c++) p[c] = cadd(p[c], s0[c]);
+   }
+   store_spinor(a.psi, gx, p);
+   store_spinor(a.rho, gx, s1);
+   if (COR) store_spinor(a.s0g, gx, s0);
+}
+
+constexpr int CLMAX = 64;         // sub-blocks of a block
+constexpr int CLSPIN = 1 << 22;   // polls of a wait
+constexpr int CLPAD = 64;         // distance of the counters: a line each
+constexpr int CLSLEEP = 8;        // pause between polls, 64 clocks each
+
+struct ClArgs
+{
+   int ns;                     // sub-blocks per block
+   const int *imb4;            // [nb][ns][RBV] points of the sub-blocks
+   const int *nbs;             // [ns][8] neighbouring sub-block in the block or -1
+   unsigned *ticket, *count;   // [CLPAD], [nbh][CLPAD]: zero at the start
+   unsigned long long *x;      // [2][nbh][ns] face fields
+   unsigned long long *sums;   // [nbh][ns][4]
+   size_t xlen;                // length of one of the two
+   int *dead;                  // set if a wait was given up (host memory)
+};
+
+__device__ inline void cl_store(unsigned long long *p, unsigned long long v)
+{
+   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned long long cl_load(const unsigned long long *p)
+{
+   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned long long cl_bits(float2 v)
+{
+   return ((unsigned long long)__float_as_uint(v.y) << 32) | __float_as_uint(v.x);
+}
+__device__ inline float2 cl_value(unsigned long long b)
+{
+   return make_float2(__uint_as_float((unsigned)b), __uint_as_float((unsigned)(b >> 32)));
+}
+
+struct ClState
+{
+   int bi, sub;       // block of the colour, sub-block
+   unsigned phase;    // arrivals so far
+   int buf;           // exchange buffer of the next pass
+   bool gone;         // a wait was given up
+};
+
+// Arrivals are counted in wavefronts, two per work-group and phase: in a hopping
+// pass those of the source points, for the sums twice the first.
+
+// the wavefront's writes and reads are done: count it in n times
+__device__ inline void cl_arrive(const ClArgs &q, const ClState &st, unsigned n)
+{
+   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+   if ((threadIdx.x & 63) == 0)
+      __hip_atomic_fetch_add(q.count + (size_t)st.bi * CLPAD, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// until all work-groups of the block have arrived (the wavefront as a whole)
+__device__ inline void cl_wait(const ClArgs &q, ClState &st)
+{
+   const unsigned want = 2u * st.phase * (unsigned)q.ns;
+   int k = 0;
+   while (!st.gone && __hip_atomic_load(q.count + (size_t)st.bi * CLPAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want)
+   {
+      if (++k >= CLSPIN)
+      {
+         st.gone = true;
+         __hip_atomic_store(q.dead, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+      __builtin_amdgcn_s_sleep(CLSLEEP);
+   }
+   asm volatile("" ::: "memory");
+}
+
+// the face values of the lane (a source) for the neighbouring sub-blocks nb
+template <typename S>
+__device__ inline void cl_push(const ClArgs &q, const ClState &st, const RegBlock<S> &b, const int *nb, const float2 *s)
+{
+   unsigned long long *X = q.x + st.buf * q.xlen;
+   const int n = st.bi * q.ns + st.sub;
+#pragma unroll
+   for (int mu = 0; mu < 4; mu++)
+   {
+      const int x = b.coord(mu);
+      if (x == 3 && nb[2 * mu] >= 0)
+      {
+         float2 h[6], c[6], u[9];
+#pragma unroll
+         for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[mu][k]);
+         if (mu == 0) weyl_project<0, false>(s, h);
+         if (mu == 1) weyl_project<1, false>(s, h);
+         if (mu == 2) weyl_project<2, false>(s, h);
+         if (mu == 3) weyl_project<3, false>(s, h);
+         su3_mul_f<true>(u, h, c);
+         su3_mul_f<true>(u, h + 3, c + 3);
+         unsigned long long *p = X + face_unit(n, 2 * mu) + b.face_point(mu, b.odd);
+#pragma unroll
+         for (int k = 0; k < 6; k++) cl_store(p + k * FPT, cl_bits(c[k]));
+      }
+      else if (x == 0 && nb[2 * mu + 1] >= 0)
+      {
+         float2 h[6];
+         if (mu == 0) weyl_project<0, true>(s, h);
+         if (mu == 1) weyl_project<1, true>(s, h);
+         if (mu == 2) weyl_project<2, true>(s, h);
+         if (mu == 3) weyl_project<3, true>(s, h);
+         unsigned long long *p = X + face_unit(n, 2 * mu + 1) + b.face_point(mu, b.odd);
+#pragma unroll
+         for (int k = 0; k < 6; k++) cl_store(p + k * FPT, cl_bits(h[k]));
+      }
+   }
+}
+
+// w += the terms from the neighbouring sub-blocks
+template <typename S>
+__device__ inline void cl_pull(const ClArgs &q, const ClState &st, const RegBlock<S> &b, const int *nb, float2 *w)
+{
+   const unsigned long long *X = q.x + st.buf * q.xlen;
+#pragma unroll
+   for (int mu = 0; mu < 4; mu++)
+   {
+      const int x = b.coord(mu);
+      const bool fw = x == 3 && nb[2 * mu] >= 0, bw = x == 0 && nb[2 * mu + 1] >= 0;
+      if (fw || bw)
+      {
+         const size_t f = fw ? face_unit(st.bi * q.ns + nb[2 * mu], 2 * mu + 1)
+                             : face_unit(st.bi * q.ns + nb[2 * mu + 1], 2 * mu);
+         const unsigned long long *p = X + f + b.face_point(mu, !b.odd);
+         float2 h[6];
+#pragma unroll
+         for (int c = 0; c < 6; c++) h[c] = cl_value(cl_load(p + c * FPT));
+         if (fw)
+         {
+            float2 c[6], u[9];
+#pragma unroll
+            for (int k = 0; k < 9; k++) u[k] = to_f2(b.u[mu][k]);
+            su3_mul_f<false>(u, h, c);
+            su3_mul_f<false>(u, h + 3, c + 3);
+            if (mu == 0) spin_expand_add<float2, 0, true>(c, c + 3, w);
+            if (mu == 1) spin_expand_add<float2, 1, true>(c, c + 3, w);
+            if (mu == 2) spin_expand_add<float2, 2, true>(c, c + 3, w);
+            if (mu == 3) spin_expand_add<float2, 3, true>(c, c + 3, w);
+         }
+         else
+         {
+            if (mu == 0) spin_expand_add<float2, 0, false>(h, h + 3, w);
+            if (mu == 1) spin_expand_add<float2, 1, false>(h, h + 3, w);
+            if (mu == 2) spin_expand_add<float2, 2, false>(h, h + 3, w);
+            if (mu == 3) spin_expand_add<float2, 3, false>(h, h + 3, w);
+         }
+      }
+   }
+}
+
+// hopping pass over the whole block: the terms across the sub-blocks' faces
+// travel while the work-group forms its own
+template <typename S> struct ClHook
+{
+   const ClArgs &q;
+   ClState &st;
+   const RegBlock<S> &b;
+   const int *nb;
+   const float2 *src;
+   float2 *w;
+   __device__ void put() const { cl_push(q, st, b, nb, src); }
+   __device__ void sent() const { cl_arrive(q, st, 1); }
+   __device__ void take() const
+   {
+      cl_wait(q, st);
+      cl_pull(q, st, b, nb, w);
+   }
+};
+
+template <int OUT, typename S>
+__device__ inline void cl_hop(const ClArgs &q, ClState &st, const RegBlock<S> &b, const int *nb, const float2 *src,
+                              float2 *w, float2 *lb)
+{
+   st.phase++;
+   rb_hop<OUT>(b, src, w, lb, ClHook<S>{q, st, b, nb, src, w});
+   st.buf ^= 1;
+}
+
+// sums over the block from the work-groups' shares
+// (sh may be written again only after another barrier has been passed)
+__device__ inline void cl_sums(const ClArgs &q, ClState &st, double *sh, double &rr, double &zr, double &zi)
+{
+   unsigned long long *p = q.sums + (size_t)st.bi * q.ns * 4;
+   st.phase++;
+   if (threadIdx.x < 64)
+   {
+      const int l = threadIdx.x;
+      if (l == 0)
+      {
+         cl_store(p + 4 * st.sub, (unsigned long long)__double_as_longlong(rr));
+         cl_store(p + 4 * st.sub + 1, (unsigned long long)__double_as_longlong(zr));
+         cl_store(p + 4 * st.sub + 2, (unsigned long long)__double_as_longlong(zi));
+      }
+      cl_arrive(q, st, 2);
+      cl_wait(q, st);
+      double v[3] = {0.0, 0.0, 0.0};
+      if (l < q.ns)
+      {
+#pragma unroll
+         for (int k = 0; k < 3; k++) v[k] = __longlong_as_double((long long)cl_load(p + 4 * l + k));
+      }
+#pragma unroll
+      for (int k = 0; k < 3; k++) v[k] = wave_sum63(v[k]);
+      if (l == 63)
+      {
+         sh[0] = v[0];
+         sh[1] = v[1];
+         sh[2] = v[2];
+      }
+   }
+   __syncthreads();
+   rr = sh[0];
+   zr = sh[1];
+   zi = sh[2];
+}
+
+__global__ void k_cl_reset(unsigned *p, int n)
+{
+   const int k = blockIdx.x * 256 + threadIdx.x;
+   if (k < n) p[(size_t)k * CLPAD] = 0;
+}
+
+template <int ISOLV, bool MASKED>
+__global__ __launch_bounds__(RBV) __attribute__((amdgpu_waves_per_eu(2))) void k_sap_cluster(SArgs a, ClArgs q)
+{
+   __shared__ float2 LB[18 * RBV];  // hopping exchange (rb_hop)
+   __shared__ float2 MS[18][RBV];   // first Pauli matrix of each point
+   __shared__ double sh[3][4], shc[3];
+   __shared__ int tk, nb[8];
+   const int x = threadIdx.x;
+   if (x == 0) tk = (int)__hip_atomic_fetch_add(q.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+   __syncthreads();
+   ClState st;
+   st.bi = tk / q.ns;
+   st.sub = tk % q.ns;
+   st.phase = 0;
+   st.buf = 0;
+   st.gone = false;
+   if (x < 8) nb[x] = q.nbs[8 * st.sub + x];
+   const int gx = q.imb4[((size_t)(a.n0 + st.bi) * q.ns + st.sub) * RBV + x];
+   const bool even = x < RBV / 2;
+   RegBlock<float2> b;
+   rb_load<float2, MASKED>(a, a.u, x, gx, b);
+   float2 mreg[18];
+   {
+      const float2 *m = a.sw + (size_t)(gx >> 6) * (36 * SB) + (gx & (SB - 1));
+#pragma unroll
+      for (int k = 0; k < 18; k++)
+      {
+         MS[k][x] = m[k * SB];
+         mreg[k] = m[(18 + k) * SB];
+      }
+   }
+   const float2 zero = make_float2(0.0f, 0.0f);
+   float2 s0[12], s1[12], w[12], o[12];
+   load_spinor((const float2 *)a.rho, gx, s1);
+   const int sb = (a.n0 + st.bi) * q.ns + st.sub;  // number of the sub-block
+   if (a.pull)
+   {
+      zero12(w);
+      rb_pull<true>(b, a.wf, a.nbn + 8 * (size_t)sb, w);
+#pragma unroll
+      for (int c = 0; c < 12; c++) s1[c] = cadd(s1[c], cscale(w[c], 0.5f));
+   }
+#pragma unroll
+   for (int c = 0; c < 12; c++)
+   {
+      s0[c] = zero;
+      if (!ISOLV && b.bp) s1[c] = zero;
+   }
+   __syncthreads();
+
+   if (ISOLV)
+   {
+      // odd points: s1 = A_oo^-1 s1, then even points: s1 += 1/2 hops
+      zero12(w);
+      if (!even)
+      {
+         pauli_reg2(&MS[0][x], RBV, mreg, 1, 0.0f, s1, w);
+#pragma unroll
+         for (int c = 0; c < 12; c++)
+         {
+            if (b.bp) w[c] = zero;
+            s1[c] = w[c];
+         }
+      }
+      cl_hop<0>(q, st, b, nb, w, w, LB);
+      if (even)
+      {
+#pragma unroll
+         for (int c = 0; c < 12; c++) s1[c] = b.bp ? zero : cadd(s1[c], cscale(w[c], 0.5f));
+      }
+   }
+
+   // minimal residual steps: w = D s1 (k_sap_reg)
+   for (int imr = 0; imr < a.nmr; imr++)
+   {
+      if (ISOLV)
+      {
+         zero12(w);
+         cl_hop<1>(q, st, b, nb, s1, w, LB);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = even ? s1[c] : cscale(w[c], -0.5f);
+         pauli_reg2(&MS[0][x], RBV, mreg, 1, even ? a.mu : 0.0f, w, o);
+         const float f = even ? 2.0f : 1.0f;
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = (b.bp && !even) ? zero : cscale(o[c], f);
+         cl_hop<0>(q, st, b, nb, w, w, LB);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = (b.bp && even) ? zero : cscale(w[c], 0.5f);
+      }
+      else
+      {
+         pauli_reg2(&MS[0][x], RBV, mreg, 1, even ? a.mu : a.muo, s1, o);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = cscale(o[c], -2.0f);
+         cl_hop<1>(q, st, b, nb, s1, w, LB);
+         cl_hop<0>(q, st, b, nb, s1, w, LB);
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = b.bp ? zero : cscale(w[c], -0.5f);
+      }
+      double rr, zr, zi;
+      rb_sums(ISOLV ? even : true, w, s1, sh, rr, zr, zi);
+      cl_sums(q, st, shc, rr, zr, zi);
+      float r = (float)rr;
+      if (r < 2.0f * FLT_MIN) break;
+      r = 1.0f / r;
+      const float2 z = make_float2((float)zr * r, (float)zi * r), mz = make_float2(-z.x, -z.y);
+      if (!ISOLV || even)
+      {
+#pragma unroll
+         for (int c = 0; c < 12; c++)
+         {
+            s0[c] = cmac(s0[c], z, s1[c]);
+            s1[c] = cmac(s1[c], mz, w[c]);
+         }
+      }
+   }
+
+   if (ISOLV)
+   {
+      // odd solution s0_o = s1_o - A_oo^-1 (-1/2 hops of s0_e)
+      zero12(w);
+      cl_hop<1>(q, st, b, nb, s0, w, LB);
+      if (!even)
+      {
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = cscale(w[c], -0.5f);
+         pauli_reg2(&MS[0][x], RBV, mreg, 1, 0.0f, w, o);
+         const float m = a.eoflg ? 0.0f : a.mu;
+#pragma unroll
+         for (int c = 0; c < 12; c++)
+         {
+            if (b.bp) o[c] = zero;
+            s0[c] = csub(s1[c], o[c]);
+            // odd residual -i mu gamma5 s0 (update_flds1) or 0 (eoflg, update_flds2)
+            const float cm = (c < 6) ? -m : m;
+            s1[c] = make_float2(-cm * s0[c].y, cm * s0[c].x);
+         }
+      }
+   }
+   rb_push<true>(b, s0, a.wf, sb, a.nbn + 8 * (size_t)sb);
+   lds_store<false>(a, gx, s0, s1);
+}
+
+// ---------------------------------------------------------------------------
 // the Schwarz sweep with the block's spinors on the chip (blocks of up to
-// 1365 points other than 4^4, FP32)
+// 1365 points whose sizes are not all multiples of 4, FP32)
 //
 // Lane i of the work-group owns the even point i and the odd point bh + i of
 // the block.  The block fields s0, s1 stay in its registers; the source of a
@@ -1156,10 +1596,9 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const S *u16)
 // the chip (600 bytes per point) and are streamed, each once per pass and
 // parity: 864 bytes per point and MinRes step, against 1350 and more of
 // k_sap_blocks, whose fields also pass through global memory.
-// Per cycle (us, k_sap_lds / k_sap_blocks, nmr = 4): 8x4^3 blocks on 16x8^3
-// 146 / 231, on 32^3x16 445 / 680; 8^2x4^2 on 16^2x8^2 203 / 413, on 32^3x16
-// 464 / 830; 4x6^3 on 16x24^3 348 / 675; 6^4 on 12^4 351 / 622, on 36^2x24^2
-// 1359 / 2119 (12 wavefronts, 168 registers, 21 spilled).
+// Per cycle (us, k_sap_lds / k_sap_blocks, nmr = 4): 4x6^3 blocks on 8x12^3
+// 229 / 445, on 16x24^3 348 / 675; 6^4 on 12^4 351 / 622, on 36^2x24^2 1359 /
+// 2119 (12 wavefronts, 168 registers, 21 spilled).
 // ---------------------------------------------------------------------------
 
 constexpr int BLV_MAX = 1365;  // points of a block, two per lane: 64 KiB of LDS
@@ -1243,26 +1682,6 @@ __device__ inline void point_sums(const float2 *s2, const float2 *s1, double &rr
       zr += (double)pr;
       zi += (double)pi;
    }
-}
-
-// psi += s0 (or = s0 for pz), rho = s1, correction s0 of one point
-__device__ inline void lds_store(const SArgs &a, int gx, const float2 *s0, const float2 *s1)
-{
-   float2 p[12];
-   if (a.pz)
-   {
-#pragma unroll
-      for (int c = 0; c < 12; c++) p[c] = s0[c];
-   }
-   else
-   {
-      load_spinor((const float2 *)a.psi, gx, p);
-#pragma unroll
-      for (int c = 0; c < 12; c++) p[c] = cadd(p[c], s0[c]);
-   }
-   store_spinor(a.psi, gx, p);
-   store_spinor(a.rho, gx, s1);
-   store_spinor(a.s0g, gx, s0);
 }
 
 template <int ISOLV, int TPB, bool MASKED>
@@ -1401,7 +1820,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(TPB <= 512 
       if (own) lds_put(F, bh, i, s0);
       __syncthreads();
       if (!own) return;
-      lds_store(a, ge, s0, s1);
+      lds_store<true>(a, ge, s0, s1);
       float2 v[12], o[12];
       lds_hop<true, WIDE>(a, imb, F, bh + i, go, w);
       load_spinor((const float2 *)a.rho, go, v);
@@ -1416,12 +1835,12 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(TPB <= 512 
          const float cm = (c < 6) ? -m : m;
          v[c] = make_float2(-cm * o[c].y, cm * o[c].x);
       }
-      lds_store(a, go, o, v);
+      lds_store<true>(a, go, o, v);
    }
    else if (own)
    {
-      lds_store(a, ge, s0, s1);
-      lds_store(a, go, t0, t1);
+      lds_store<true>(a, ge, s0, s1);
+      lds_store<true>(a, go, t0, t1);
    }
 }
 
@@ -1714,11 +2133,71 @@ static void free_grid()
    for (int k = 0; k < 3; k++) dev_free(G.d_h64[k]);
    dev_free(G.d_swb64); dev_free(G.d_scr64); dev_free(G.d_bsd);
    dev_free(G.d_wf); dev_free(G.d_wfm); dev_free(G.d_nbn);
+   dev_free(G.d_imb4); dev_free(G.d_nbs); dev_free(G.d_count); dev_free(G.d_x);
+   if (G.h_dead) HIP_OK(hipHostFree(G.h_dead));
    dev_free(G.d_ipp); dev_free(G.d_bw);
    G = SapGrid();
 }
 
 static bool reg_kernel() { return OQH_SAP_REG && G.bvol == RBV; }
+
+// tables and buffers of k_sap_cluster; false if the block size does not allow
+// it (bipt: block point of a position in the block)
+static bool build_cluster(const int *bs, const std::vector<int> &bipt)
+{
+   int ns = 1, nd[4];
+   for (int mu = 0; mu < 4; mu++)
+   {
+      if (bs[mu] % 4) return false;
+      nd[mu] = bs[mu] / 4;
+      ns *= nd[mu];
+   }
+   if (ns < 2 || ns > CLMAX) return false;
+   std::vector<int> &imb4 = G.imb4, nbs(8 * (size_t)ns), loc(G.bvol);
+   imb4.assign((size_t)G.nb * G.bvol, 0);
+   int m[4], y[4], x[4];
+   for (int k = 0; k < ns; k++)
+   {
+      int r = k;
+      for (int mu = 3; mu >= 0; mu--)
+      {
+         m[mu] = r % nd[mu];
+         r /= nd[mu];
+      }
+      for (int mu = 0; mu < 4; mu++)
+         for (int s = 0; s < 2; s++)
+         {
+            const int c = m[mu] + (s ? -1 : 1);
+            int z[4] = {m[0], m[1], m[2], m[3]};
+            z[mu] = c;
+            nbs[8 * (size_t)k + 2 * mu + s] =
+               (c < 0 || c >= nd[mu]) ? -1 : z[3] + nd[3] * (z[2] + nd[2] * (z[1] + nd[1] * z[0]));
+         }
+      int ofs[2] = {0, RBV / 2};
+      for (x[0] = 0; x[0] < 4; x[0]++)
+      for (x[1] = 0; x[1] < 4; x[1]++)
+      for (x[2] = 0; x[2] < 4; x[2]++)
+      for (x[3] = 0; x[3] < 4; x[3]++)
+      {
+         for (int mu = 0; mu < 4; mu++) y[mu] = 4 * m[mu] + x[mu];
+         loc[(size_t)k * RBV + ofs[(x[0] + x[1] + x[2] + x[3]) & 1]++] = bipt[lexb(bs, y)];
+      }
+   }
+   for (int n = 0; n < G.nb; n++)
+      for (int i = 0; i < G.bvol; i++) imb4[(size_t)n * G.bvol + i] = G.imb[(size_t)n * G.bvol + loc[i]];
+   const size_t nx = (size_t)G.nbh * ns * FUN;
+   G.d_imb4 = (int *)dev_alloc(sizeof(int) * imb4.size());
+   G.d_nbs = (int *)dev_alloc(sizeof(int) * nbs.size());
+   G.d_count = (unsigned *)dev_alloc(sizeof(unsigned) * CLPAD * ((size_t)G.nbh + 1));
+   G.d_x = (unsigned long long *)dev_alloc(sizeof(unsigned long long) * (2 * nx + (size_t)G.nbh * ns * 4));
+   if (hipHostMalloc((void **)&G.h_dead, sizeof(int), 0) != hipSuccess) G.h_dead = nullptr;
+   if (!G.d_imb4 || !G.d_nbs || !G.d_count || !G.d_x || !G.h_dead) return false;
+   *G.h_dead = 0;
+   HIP_OK(hipMemcpy(G.d_imb4, imb4.data(), sizeof(int) * imb4.size(), hipMemcpyHostToDevice));
+   HIP_OK(hipMemcpy(G.d_nbs, nbs.data(), sizeof(int) * nbs.size(), hipMemcpyHostToDevice));
+   G.ns = ns;
+   return true;
+}
 
 static bool build_grid(const char *where)
 {
@@ -1861,24 +2340,25 @@ static bool build_grid(const char *where)
       }
    }
    G.d_swb = (float2 *)dev_alloc(units_for(L.g.V, 36) * sizeof(float2));
-   if (reg_kernel())
+   if (reg_kernel() || build_cluster(bs, bipt))
    {
-      // neighbouring blocks: the block of a point one step outside
-      std::vector<int> blk(L.g.V), nbn(8 * (size_t)G.nb);
-      for (int n = 0; n < G.nb; n++)
-         for (int i = 0; i < G.bvol; i++) blk[G.imb[(size_t)n * G.bvol + i]] = n;
-      for (int n = 0; n < G.nb; n++)
+      // neighbouring 4^4 (sub-)blocks across the block's faces: that of a
+      // point one step outside, -1 inside the block
+      const int ns = std::max(G.ns, 1);
+      const std::vector<int> &im = G.ns ? G.imb4 : G.imb;
+      std::vector<int> sub(L.g.V), nbn(8 * (size_t)G.nb * ns, -1);
+      for (size_t k = 0; k < im.size(); k++) sub[im[k]] = (int)(k / RBV);
+      for (size_t k = 0; k < im.size(); k++)
          for (int mu = 0; mu < 4; mu++)
-            for (int i = 0; i < G.bvol; i++)
-            {
-               const size_t gx = G.imb[(size_t)n * G.bvol + i];
-               if (bnb[(size_t)(2 * mu) * G.bvol + i] == G.bvol) nbn[8 * (size_t)n + 2 * mu] = blk[L.g.iup[4 * gx + mu]];
-               if (bnb[(size_t)(2 * mu + 1) * G.bvol + i] == G.bvol)
-                  nbn[8 * (size_t)n + 2 * mu + 1] = blk[L.g.idn[4 * gx + mu]];
-            }
+         {
+            const size_t gx = im[k];
+            const int n = (int)(k / RBV), up = sub[L.g.iup[4 * gx + mu]], dn = sub[L.g.idn[4 * gx + mu]];
+            if (fm[gx] & (1 << (2 * mu))) nbn[8 * (size_t)n + 2 * mu] = up;
+            if (fm[gx] & (2 << (2 * mu))) nbn[8 * (size_t)n + 2 * mu + 1] = dn;
+         }
       G.d_nbn = (int *)dev_alloc(sizeof(int) * nbn.size());
       HIP_OK(hipMemcpy(G.d_nbn, nbn.data(), sizeof(int) * nbn.size(), hipMemcpyHostToDevice));
-      G.d_wf = (float2 *)dev_alloc((size_t)G.nb * FUN * sizeof(float2));
+      G.d_wf = (float2 *)dev_alloc((size_t)G.nb * ns * FUN * sizeof(float2));
    }
    else
    {
@@ -1962,7 +2442,7 @@ static bool half_variant()
 }
 
 // the block's spinors fit on the chip (k_sap_lds)
-static bool lds_kernel() { return G.bvol != RBV && G.bvol <= BLV_MAX; }
+static bool lds_kernel() { return G.bvol != RBV && !G.ns && G.bvol <= BLV_MAX; }
 
 template <int TPB> static void launch_lds(const SArgs &a, int isolv, unsigned nb)
 {
@@ -1976,6 +2456,33 @@ template <int TPB> static void launch_lds(const SArgs &a, int isolv, unsigned nb
       k_sap_lds<0, TPB, true><<<nb, TPB, lds, st>>>(a);
    else
       k_sap_lds<0, TPB, false><<<nb, TPB, lds, st>>>(a);
+}
+
+// a block shared by several work-groups (k_sap_cluster)
+static void launch_cluster(const SArgs &a, int isolv)
+{
+   hipStream_t st = lib().stream;
+   if (*G.h_dead) fail("sap [sap.c]", "a work-group of a Schwarz block did not get its neighbours' values");
+   ClArgs q;
+   q.ns = G.ns;
+   q.imb4 = G.d_imb4;
+   q.nbs = G.d_nbs;
+   q.ticket = G.d_count;
+   q.count = G.d_count + CLPAD;
+   q.x = G.d_x;
+   q.xlen = (size_t)G.nbh * G.ns * FUN;
+   q.sums = G.d_x + 2 * q.xlen;
+   q.dead = G.h_dead;
+   const unsigned nb = (unsigned)(G.nbh * G.ns);
+   k_cl_reset<<<(G.nbh + 256) / 256, 256, 0, st>>>(G.d_count, G.nbh + 1);
+   if (isolv && a.masked)
+      k_sap_cluster<1, true><<<nb, RBV, 0, st>>>(a, q);
+   else if (isolv)
+      k_sap_cluster<1, false><<<nb, RBV, 0, st>>>(a, q);
+   else if (a.masked)
+      k_sap_cluster<0, true><<<nb, RBV, 0, st>>>(a, q);
+   else
+      k_sap_cluster<0, false><<<nb, RBV, 0, st>>>(a, q);
 }
 
 // block solves of the blocks of colour ic; the register kernel first adds
@@ -2009,6 +2516,8 @@ static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
       else
          k_sap_reg<0, float2, false><<<nb, RBV, 0, L.stream>>>(a, nullptr, nullptr);
    }
+   else if (G.ns)
+      launch_cluster(a, isolv);
    else if (lds_kernel())
    {
       if (G.bh <= 256)
@@ -2035,23 +2544,23 @@ static void sap_push_faces(const SArgs &a, int c)
 }
 
 // one Schwarz cycle (sap.c:720-790): colour 0, faces of colour 1, colour 1,
-// faces of colour 0.  With the register kernel the face terms into a colour
+// faces of colour 0.  With the 4^4 (sub-)block kernels the face terms into a colour
 // are added by its next block solve; first: rho is complete on entry (none
 // for colour 0); finish: complete rho at the end (faces of colour 0).
 static void sap_cycle(const SArgs &a, int isolv, bool first, bool finish)
 {
-   if (reg_kernel())
+   if (reg_kernel() || G.ns)
    {
       sap_blocks(a, 0, isolv, !first);
       sap_blocks(a, 1, isolv, 1);
       if (!finish) return;
       SArgs c = a;
       c.n0 = 0;
-      const unsigned nb = (unsigned)(G.nbh * std::max(a.nsrc, 1));
+      const unsigned nb = (unsigned)(G.nbh * std::max(G.ns, 1) * std::max(a.nsrc, 1));
       if (half_variant() && !a.nsrc)
-         k_sap_complete<__half2><<<nb, RBV, 0, lib().stream>>>(c, G.d_u16);
+         k_sap_complete<__half2><<<nb, RBV, 0, lib().stream>>>(c, G.d_imb, G.d_u16);
       else
-         k_sap_complete<float2><<<nb, RBV, 0, lib().stream>>>(c, nullptr);
+         k_sap_complete<float2><<<nb, RBV, 0, lib().stream>>>(c, G.ns ? G.d_imb4 : G.d_imb, nullptr);
    }
    else
    {
@@ -2225,7 +2734,7 @@ void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho,
    a.rho = rho;
    const int V = L.g.V;
    const unsigned nbk = (V + 255) / 256;
-   const bool pz = zero && (reg_kernel() || lds_kernel());
+   const bool pz = zero && (reg_kernel() || lds_kernel() || G.ns);
    if (zero && !pz) HIP_OK(hipMemsetAsync(psi, 0, nu * sizeof(float2), L.stream));
    if (half_variant())
    {

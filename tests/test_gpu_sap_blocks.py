@@ -1,7 +1,8 @@
 """Schwarz cycles with blocks other than 4^4: the kernel that keeps the block's
 spinors on the chip (sap.hip k_sap_lds; each of its three work-group sizes,
-with idle lanes and without) and the one for larger blocks, both solvers and
-boundary conditions, with a twisted mass, against the oracle's FP64 cycles on
+with idle lanes), the one that shares a block among work-groups
+(k_sap_cluster, 2, 4, 8 and 16 of them) and the one for other large blocks, both
+solvers and boundary conditions, with a twisted mass, against the oracle's FP64 cycles on
 the same FP32-rounded inputs: 2e-6 of the field's norm for the solution and
 1e-5 for the residual (measured 1.5e-7 and 3e-7 after five cycles)."""
 import ctypes as C
@@ -16,10 +17,11 @@ P = C.c_void_p
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("bs,L,T", [((8, 4, 4, 4), (16, 8, 8, 8), None), ((4, 4, 6, 4), (8, 8, 12, 8), (8, 8, 6, 8)),
+@pytest.mark.parametrize("bs,L,T", [((8, 4, 4, 4), (16, 8, 8, 8), None), ((4, 4, 6, 4), (8, 8, 12, 8), (8, 8, 6, 8)), ((6, 4, 4, 4), (12, 8, 8, 8), (6, 8, 8, 8)),
                                     ((4, 6, 6, 6), (8, 12, 12, 12), (8, 6, 6, 6)),
                                     ((8, 8, 4, 4), (16, 16, 8, 8), (8, 8, 8, 8)), ((6, 6, 6, 6), (12, 12, 12, 12), None),
-                                    ((4, 8, 6, 8), (8, 16, 12, 16), (8, 8, 6, 8))])
+                                    ((4, 8, 6, 8), (8, 16, 12, 16), (8, 8, 6, 8)),
+                                    ((8, 8, 8, 4), (16, 16, 16, 8), (8, 8, 8, 8)), ((8, 8, 8, 8), (16, 16, 16, 16), (8, 8, 8, 8))])
 @pytest.mark.parametrize("isolv", [0, 1])
 @pytest.mark.parametrize("bc,mu", [(3, 0.0), (0, 0.05)])
 def test_cycles(bs, L, T, isolv, bc, mu):
