@@ -129,6 +129,8 @@ bool require_geometry(const char *where);
 void *dev_alloc(size_t bytes);
 void dev_free(void *p);
 void *tmp_buffer(size_t bytes);
+void copy_in(void *dev, const void *host, size_t bytes);
+void copy_out(void *host, const void *dev, size_t bytes);
 
 // field resolution: device base pointer (and site offset) of an argument
 struct Res

@@ -602,8 +602,7 @@ extern "C" void oqh_export_frc(double *frc)
    size_t bytes = (size_t)h * 8 * 8 * sizeof(double);
    void *aos = tmp_buffer(bytes);
    blocks_to_aos_f64(d_frc, (double2 *)aos, h, 32, L.stream);
-   HIP_OK(hipMemcpyAsync(frc, aos, bytes, hipMemcpyDeviceToHost, L.stream));
-   HIP_OK(hipStreamSynchronize(L.stream));
+   copy_out(frc, aos, bytes);
 }
 
 extern "C" void fwd_euler(int n, double eps)
