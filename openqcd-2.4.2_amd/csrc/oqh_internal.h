@@ -129,6 +129,10 @@ bool require_geometry(const char *where);
 void *dev_alloc(size_t bytes);
 void dev_free(void *p);
 void *tmp_buffer(size_t bytes);
+// reserve_ws, reserve_wsd; without clear the fields hold what was left in
+// them, for callers that write every point before they read it
+spinor **take_ws(int n, bool clear);
+spinor_dble **take_wsd(int n, bool clear);
 void copy_in(void *dev, const void *host, size_t bytes);
 void copy_out(void *host, const void *dev, size_t bytes);
 
@@ -177,6 +181,7 @@ void gs_step(float2 *s, const float2 *r, const float2 *q, float2 *coef, int ic, 
 // coef[ir] = (|rho|, |rho|^2); the Gram entries of q[k-1] are formed on the
 // way into gram[(k-1) ldg + j] (q[0..k-2] must be the vectors of the
 // previous calls with the same gram; ldg >= k)
+void gcr_solution(double2 *psi, float2 *const *phi, const complex *c, int k, float2 *wrk, int n);
 void gs_classical(float2 *s, float2 *const *q, int k, float2 *rho, float2 *coef, int ib, int ic, int ir, int n,
                   float2 *gram, int ldg);
 

@@ -190,9 +190,19 @@ extern "C" double fgcr(int vol, void (*Dop)(spinor_dble *s, spinor_dble *r),
          c[l].re = zr * r;
          c[l].im = zi * r;
       }
-      set_s2zero(vol, 2, rho);
-      for (int l = k; l >= 0; l--) mulc_spinor_add(vol, 2, rho, phi[l], c[l]);
-      add_s2sd(vol, 2, rho, psi);
+      int poff = 0;
+      double2 *pd = fused ? (double2 *)device_field(psi, F64, &poff) : nullptr;
+      if (pd && !poff)
+      {
+         for (int l = 0; l <= k; l++) qv[l] = F(phi[l]);
+         gcr_solution(pd, qv.data(), c.data(), k, F(rho), npts);
+      }
+      else
+      {
+         set_s2zero(vol, 2, rho);
+         for (int l = k; l >= 0; l--) mulc_spinor_add(vol, 2, rho, phi[l], c[l]);
+         add_s2sd(vol, 2, rho, psi);
+      }
       Dop(psi, wrk);
       diff_sd2s(vol, 2, eta, wrk, rho);
       rn = get_res(vol, istop, rho);
@@ -300,8 +310,8 @@ extern "C" double sap_gcr(int nkv, int nmx, int istop, double res, double mu, sp
          const int nwsd = nn_use ? 4 : 2;
          alloc_ws(L.ws_used + 2 * nkv + 1);
          alloc_wsd(L.wsd_used + nwsd);
-         spinor **ws = reserve_ws(2 * nkv + 1);
-         spinor_dble **wsd = reserve_wsd(nwsd);
+         spinor **ws = take_ws(2 * nkv + 1, false);
+         spinor_dble **wsd = take_wsd(nwsd, false);
          spinor_dble *rsd = wsd[1];
          mud = mu;
          assign_sd2sd(vt, 2, eta, rsd);
@@ -442,8 +452,8 @@ extern "C" void sap_gcr_multi(int n, int nkv, int nmx, int istop, double res, do
    for (int s = 0; s < n; s++)
    {
       MultiSrc &m = S[s];
-      spinor **ws = reserve_ws(2 * nkv + 1);
-      spinor_dble **wsd = reserve_wsd(2);
+      spinor **ws = take_ws(2 * nkv + 1, false);
+      spinor_dble **wsd = take_wsd(2, false);
       m.phi = ws;
       m.rho = ws[nkv];
       m.chi = ws + nkv + 1;
@@ -540,9 +550,19 @@ extern "C" void sap_gcr_multi(int n, int nkv, int nmx, int istop, double res, do
             m.c[l].re = zr * r;
             m.c[l].im = zi * r;
          }
-         set_s2zero(vt, 2, m.rho);
-         for (int l = k; l >= 0; l--) mulc_spinor_add(vt, 2, m.rho, m.phi[l], m.c[l]);
-         add_s2sd(vt, 2, m.rho, m.psi);
+         int poff = 0;
+         double2 *pd = (double2 *)device_field(m.psi, F64, &poff);
+         if (pd && !poff)
+         {
+            for (int l = 0; l <= k; l++) qv[l] = F(m.phi[l]);
+            gcr_solution(pd, qv.data(), m.c.data(), k, F(m.rho), V);
+         }
+         else
+         {
+            set_s2zero(vt, 2, m.rho);
+            for (int l = k; l >= 0; l--) mulc_spinor_add(vt, 2, m.rho, m.phi[l], m.c[l]);
+            add_s2sd(vt, 2, m.rho, m.psi);
+         }
          Dw_dble(mud, m.psi, m.wrk);
          diff_sd2s(vt, 2, m.rsd, m.wrk, m.rho);
          m.rn = get_res(vt, 0, m.rho);

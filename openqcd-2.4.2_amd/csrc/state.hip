@@ -908,7 +908,7 @@ extern "C" void alloc_ws(int n)
    while ((int)L.ws.size() < n) L.ws.push_back((spinor *)register_field(F32, L.g.V));
 }
 
-extern "C" spinor **reserve_ws(int n)
+spinor **oqh::take_ws(int n, bool clear)
 {
    Lib &L = lib();
    if (n <= 0) return nullptr;
@@ -921,13 +921,16 @@ extern "C" spinor **reserve_ws(int n)
    for (int k = 0; k < n; k++)
    {
       p[k] = L.ws[L.ws_used + k];
-      HIP_OK(hipMemsetAsync(p[k], 0, units_for(L.g.V, 12) * sizeof(float2), L.stream));
+      if (clear)
+         HIP_OK(hipMemsetAsync(p[k], 0, units_for(L.g.V, 12) * sizeof(float2), L.stream));
    }
    ws_marks.push_back(n);
    L.ws_used += n;
    L.ws_ptrs.push_back((spinor *)p);
    return p;
 }
+
+extern "C" spinor **reserve_ws(int n) { return take_ws(n, true); }
 
 extern "C" int release_ws(void)
 {
@@ -948,7 +951,7 @@ extern "C" void alloc_wsd(int n)
    while ((int)L.wsd.size() < n) L.wsd.push_back((spinor_dble *)register_field(F64, L.g.V));
 }
 
-extern "C" spinor_dble **reserve_wsd(int n)
+spinor_dble **oqh::take_wsd(int n, bool clear)
 {
    Lib &L = lib();
    if (n <= 0) return nullptr;
@@ -961,13 +964,16 @@ extern "C" spinor_dble **reserve_wsd(int n)
    for (int k = 0; k < n; k++)
    {
       p[k] = L.wsd[L.wsd_used + k];
-      HIP_OK(hipMemsetAsync(p[k], 0, units_for(L.g.V, 12) * sizeof(double2), L.stream));
+      if (clear)
+         HIP_OK(hipMemsetAsync(p[k], 0, units_for(L.g.V, 12) * sizeof(double2), L.stream));
    }
    wsd_marks.push_back(n);
    L.wsd_used += n;
    L.wsd_ptrs.push_back((spinor_dble *)p);
    return p;
 }
+
+extern "C" spinor_dble **reserve_wsd(int n) { return take_wsd(n, true); }
 
 extern "C" int release_wsd(void)
 {
