@@ -39,6 +39,7 @@
 
 #include "dirac_dev.h"
 #include "oqh_internal.h"
+#include "lastgroup.h"
 
 namespace oqh {
 bool sap_prepare(int isolv, const char *where, bool quiet);
@@ -96,7 +97,6 @@ struct Dfl
    double2 *d_lw = nullptr, *d_law = nullptr;
    float2 *d_lw32 = nullptr, *d_law32 = nullptr;
    double2 *d_lM = nullptr;     // [Ns][Ns] row-major
-   double2 *d_lc = nullptr;     // [Ns] products, then [2][Ns] coefficients d, -d
    double2 *d_ld = nullptr;
    double2 *d_lB = nullptr;     // [Ns][Ns] (w_l, Ahat w_j) at column j
    double2 *d_lpart = nullptr;  // [Ns][LNBK] work-group shares
@@ -1109,16 +1109,23 @@ float2 *wv(int k)
 // The Krylov vectors of a little solver are stored contiguously, phi_0..
 // phi_{nmx-1} then chi_0..chi_{nmx-1}, ld complex numbers apart.  One step n
 // of the classical Gram-Schmidt process of gcr4v.c / fgcr4vd.c runs as
-//   k_lmdot + k_lsum:      a[n][l] = (chi_l, chi_n), l < n
-//   k_lmaxpy + k_lsum_bc:  chi_n -= sum_l a[n][l] chi_l; b_n = |chi_n|,
-//                          c_n = (chi_n, rho) / b_n
-//   k_lscale + k_lsum_bc:  chi_n /= b_n; rho -= c_n chi_n; |rho|^2
-// and the host reads the four numbers of step n once.  The sums are taken in
+//   k_lmdot:   a[n][l] = (chi_l, chi_n), l < n
+//   k_lmaxpy:  chi_n -= sum_l a[n][l] chi_l; b_n = |chi_n|,
+//              c_n = (chi_n, rho) / b_n
+//   k_lscale:  chi_n /= b_n; rho -= c_n chi_n; |rho|^2
+// and the host reads the four numbers of step n, which the last kernel writes
+// to its memory.  Little vectors are short (24^4, Ns = 20: 100 KB), so a step
+// is bound by its launches: the work-group of a kernel that finishes last adds
+// the shares of all (last_group) instead of a kernel after it, and the back
+// substitution of the solution runs on the device.  14 launches per step, 5
+// copies and 2 synchronisations per solution became 8 launches, no copy and no
+// synchronisation (dfl_sap_gcr at 24^4, 11 vectors: 24.6 -> 22.4 ms).  The sums are taken in
 // double precision in a fixed order (per lane, per work-group, then over the
 // work-groups), so the results do not depend on the launch timing.
 
 constexpr int LRB = 256;     // lanes of the little-vector kernels
 constexpr int LNBK = 512;    // largest number of work-groups of a reduction
+constexpr int LCPAD = 32;    // a 128-byte line per counter
 
 int lnbk(size_t nv)
 {
@@ -1137,11 +1144,33 @@ __device__ inline double2 wave_sum2(double2 v)
    return v;
 }
 
-// part[l * gridDim.x + blockIdx.x] = this work-group's share of (X_l, y)
+__device__ inline void put_part(double2 *p, double2 v)
+{
+   put_share(&p->x, v.x);
+   put_share(&p->y, v.y);
+}
+
+// sum_b part[b], b < nbk, in every lane of the wave, fixed order
+__device__ inline double2 wave_parts(const double2 *part, int nbk)
+{
+   double2 v = make_double2(0.0, 0.0);
+   for (int b = threadIdx.x & 63; b < nbk; b += 64)
+   {
+      v.x += get_share(&part[b].x);
+      v.y += get_share(&part[b].y);
+   }
+   return wave_sum2(v);
+}
+
+// (X_l, y), l < gridDim.y: to out[l], or (M != null, gridDim.y = Ns) out[k] =
+// sign * sum_l M[k][l] (X_l, y) and its negative to out[Ns + k];
+// part[l * gridDim.x + blockIdx.x] are the work-groups' shares
 template <typename C>
-__global__ __launch_bounds__(LRB) void k_lmdot(const C *X, size_t ld, const C *yv, size_t nv, double2 *part)
+__global__ __launch_bounds__(LRB) void k_lmdot(const C *X, size_t ld, const C *yv, size_t nv, double2 *part,
+                                               unsigned *cnt, double2 *out, const double2 *M, double sign)
 {
    __shared__ double2 sh[LRB / 64];
+   __shared__ double2 cs[NS_MAX];
    const int l = blockIdx.y;
    const C *cl = X + (size_t)l * ld, *cn = yv;
    double x = 0.0, y = 0.0;
@@ -1152,57 +1181,36 @@ __global__ __launch_bounds__(LRB) void k_lmdot(const C *X, size_t ld, const C *y
       y += ax * by - ay * bx;
    }
    const double2 s = wg_sum(make_double2(x, y), sh);
-   if (threadIdx.x == 0) part[(size_t)l * gridDim.x + blockIdx.x] = s;
+   double2 *pl = part + (size_t)l * gridDim.x;
+   if (threadIdx.x == 0) put_part(pl + blockIdx.x, s);
+   // a count per column: on one count for all, 1000 work-groups wait 9 us
+   if (!last_group(cnt + (l + 1) * LCPAD, gridDim.x)) return;
+   const int nq = gridDim.y, t = threadIdx.x;
+   if (t < 64)
+   {
+      const double2 v = wave_parts(pl, gridDim.x);
+      if (t == 0 && M)
+         put_part(pl, v);
+      else if (t == 0)
+         out[l] = v;
+   }
+   if (!M) return;
+   __syncthreads();
+   if (!last_group(cnt, nq)) return;
+   if (t < nq) cs[t] = make_double2(get_share(&part[(size_t)t * gridDim.x].x), get_share(&part[(size_t)t * gridDim.x].y));
+   __syncthreads();
+   if (t >= nq) return;
+   double2 z = make_double2(0.0, 0.0);
+   for (int q = 0; q < nq; q++) z = cadd(z, cmul(M[(size_t)t * nq + q], cs[q]));
+   out[t] = make_double2(sign * z.x, sign * z.y);
+   out[nq + t] = make_double2(-sign * z.x, -sign * z.y);
 }
 
-// out[q] = sum_b part[q * nbk + b] for q < nq; one wave per q, fixed order
-__global__ __launch_bounds__(LRB) void k_lsum(const double2 *part, int nbk, int nq, double2 *out)
-{
-   const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
-   for (int q = w; q < nq; q += LRB / 64)
-   {
-      double2 v = make_double2(0.0, 0.0);
-      for (int b = t; b < nbk; b += 64)
-      {
-         v.x += part[(size_t)q * nbk + b].x;
-         v.y += part[(size_t)q * nbk + b].y;
-      }
-      v = wave_sum2(v);
-      if (t == 0) out[q] = v;
-   }
-}
-
-// mode 0: bc[0] = |chi_n|, bc[1] + i bc[2] = (chi_n, rho) / |chi_n| from the
-// columns (chi_n, rho) and (|chi_n|^2, 0); mode 1: bc[3] = |rho|^2
-__global__ __launch_bounds__(64) void k_lsum_bc(const double2 *part, int nbk, int mode, double *bc)
-{
-   const int t = threadIdx.x;
-   double2 v0 = make_double2(0.0, 0.0), v1 = make_double2(0.0, 0.0);
-   for (int b = t; b < nbk; b += 64)
-   {
-      v0.x += part[b].x;
-      v0.y += part[b].y;
-      if (mode == 0) v1.x += part[nbk + b].x;
-   }
-   v0 = wave_sum2(v0);
-   v1 = wave_sum2(v1);
-   if (t != 0) return;
-   if (mode == 0)
-   {
-      const double bn = sqrt(v1.x);
-      bc[0] = bn;
-      bc[1] = (bn > 0.0) ? v0.x / bn : 0.0;
-      bc[2] = (bn > 0.0) ? v0.y / bn : 0.0;
-   }
-   else
-      bc[3] = v0.x;
-}
-
-// chi_n -= sum_{l<n} a[l] chi_l (in the precision of C), then this
-// work-group's shares of (chi_n, rho) and |chi_n|^2
+// chi_n -= sum_{l<n} a[l] chi_l (in the precision of C), then bc[0] =
+// |chi_n|, bc[1] + i bc[2] = (chi_n, rho) / |chi_n|
 template <typename C>
 __global__ __launch_bounds__(LRB) void k_lmaxpy(C *chi, size_t ld, int n, size_t nv, const double2 *a, const C *rho,
-                                                double2 *part)
+                                                double2 *part, unsigned *cnt, double *bc)
 {
    typedef decltype(C::x) R;
    __shared__ double2 sh[LRB / 64];
@@ -1228,14 +1236,23 @@ __global__ __launch_bounds__(LRB) void k_lmaxpy(C *chi, size_t ld, int n, size_t
    const double2 s1 = wg_sum(make_double2(z, 0.0), sh);
    if (threadIdx.x == 0)
    {
-      part[blockIdx.x] = s0;
-      part[gridDim.x + blockIdx.x] = s1;
+      put_part(part + blockIdx.x, s0);
+      put_part(part + gridDim.x + blockIdx.x, s1);
    }
+   if (!last_group(cnt, gridDim.x) || threadIdx.x >= 64) return;
+   const double2 v0 = wave_parts(part, gridDim.x), v1 = wave_parts(part + gridDim.x, gridDim.x);
+   if (threadIdx.x != 0) return;
+   const double bn = sqrt(v1.x);
+   bc[0] = bn;
+   bc[1] = (bn > 0.0) ? v0.x / bn : 0.0;
+   bc[2] = (bn > 0.0) ? v0.y / bn : 0.0;
 }
 
-// chi_n /= b_n, rho -= c_n chi_n (nothing if b_n = 0), shares of |rho|^2
+// chi_n /= b_n, next = rho - c_n chi_n (rho if b_n = 0; next may be rho), bc[3] =
+// |next|^2, and all of bc to the host's h
 template <typename C>
-__global__ __launch_bounds__(LRB) void k_lscale(C *cn, C *rho, size_t nv, const double *bc, double2 *part)
+__global__ __launch_bounds__(LRB) void k_lscale(C *cn, const C *rho, C *next, size_t nv, double *bc, double2 *part,
+                                                unsigned *cnt, double *h)
 {
    typedef decltype(C::x) R;
    __shared__ double2 sh[LRB / 64];
@@ -1251,13 +1268,37 @@ __global__ __launch_bounds__(LRB) void k_lscale(C *cn, C *rho, size_t nv, const 
          cn[i] = cmk<C>(vx, vy);
          rx -= cr * vx - ci * vy;
          ry -= cr * vy + ci * vx;
-         rho[i] = cmk<C>(rx, ry);
       }
+      next[i] = cmk<C>(rx, ry);
       const double px = rx, py = ry;
       z += px * px + py * py;
    }
    const double2 s = wg_sum(make_double2(z, 0.0), sh);
-   if (threadIdx.x == 0) part[blockIdx.x] = s;
+   if (threadIdx.x == 0) put_part(part + blockIdx.x, s);
+   if (!last_group(cnt, gridDim.x) || threadIdx.x >= 64) return;
+   const double2 v = wave_parts(part, gridDim.x);
+   if (threadIdx.x != 0) return;
+   bc[3] = v.x;
+   h[0] = bn;
+   h[1] = bc[1];
+   h[2] = bc[2];
+   h[3] = v.x;
+}
+
+// back substitution of gcr4v.c / fgcr4vd.c (update_psi): c_l = (c_l -
+// sum_{i>l} (chi_l, chi_i) c_i) / b_l, l = m-1..0; one wave, its lanes over i
+__global__ __launch_bounds__(64) void k_lback(const double2 *a, int nmx, const double *bc, int m, double2 *c)
+{
+   const int t = threadIdx.x;
+   for (int l = m - 1; l >= 0; l--)
+   {
+      double2 z = make_double2(0.0, 0.0);
+      // (chi_l, chi_i) is stored in column i
+      for (int i = l + 1 + t; i < m; i += 64) z = cadd(z, cmul(a[(size_t)i * nmx + l], c[i]));
+      z = wave_sum2(z);
+      if (t == 0) c[l] = make_double2((bc[4 * l + 1] - z.x) / bc[4 * l], (bc[4 * l + 2] - z.y) / bc[4 * l]);
+      __syncthreads();
+   }
 }
 
 // x = (add ? x : 0) + sum_{l<m} c[l] phi_l
@@ -1287,20 +1328,37 @@ __global__ __launch_bounds__(LRB) void k_lcomb(C *x, const C *phi, size_t ld, in
 // one little solver's Krylov space and Gram-Schmidt state
 template <typename C> struct LKry
 {
-   C *v = nullptr;          // [2 nmx][ld]: phi_0.., then chi_0..
+   C *v = nullptr;          // [2 nmx + 1][ld]: phi_0..phi_nmx, then chi_0..
    int nmx = 0;
    size_t ld = 0, nv = 0;
    double2 *a = nullptr;    // [nmx][nmx]: a[n * nmx + l] = (chi_l, chi_n)
    double *bc = nullptr;    // [nmx][4]: |chi_n|, c_n, |rho|^2 after step n
    double2 *c = nullptr;    // [nmx] coefficients of the solution
    double2 *part = nullptr; // [nmx][LNBK] work-group shares
-   double *h = nullptr;     // pinned host copy of a, bc, then c
+   double *h = nullptr;     // pinned: bc of the last step
    C *phi(int k) const { return v + (size_t)k * ld; }
-   C *chi(int k) const { return v + (size_t)(nmx + k) * ld; }
+   C *chi(int k) const { return v + (size_t)(nmx + 1 + k) * ld; }
 };
 
 LKry<float2> K32;
 LKry<double2> K64;
+
+// the counters of last_group, one for the launch and n for its columns; the
+// kernels of the library's stream share them
+unsigned *d_lcnt = nullptr;
+int lcnt_n = 0;
+
+unsigned *lcount(int n = 0)
+{
+   if (n <= lcnt_n && d_lcnt) return d_lcnt;
+   HIP_OK(hipStreamSynchronize(lib().stream));
+   dev_free(d_lcnt);
+   const size_t bytes = sizeof(unsigned) * LCPAD * (size_t)(n + 1);
+   d_lcnt = (unsigned *)dev_alloc(bytes);
+   lcnt_n = d_lcnt ? n : 0;
+   if (d_lcnt) HIP_OK(hipMemsetAsync(d_lcnt, 0, bytes, lib().stream));
+   return d_lcnt;
+}
 
 template <typename C> void lkry_free(LKry<C> &K)
 {
@@ -1315,13 +1373,13 @@ template <typename C> bool lkry_alloc(LKry<C> &K, int nmx, size_t nv)
    if (K.v && K.nmx == nmx && K.ld == ld) return true;
    lkry_free(K);
    const int nm = std::max(nmx, 2);
-   K.v = (C *)dev_alloc(sizeof(C) * 2 * (size_t)nmx * ld);
+   K.v = (C *)dev_alloc(sizeof(C) * (2 * (size_t)nmx + 1) * ld);
    K.a = (double2 *)dev_alloc(sizeof(double2) * (size_t)nmx * nmx);
    K.bc = (double *)dev_alloc(sizeof(double) * 4 * (size_t)nmx);
    K.c = (double2 *)dev_alloc(sizeof(double2) * (size_t)nmx);
    K.part = (double2 *)dev_alloc(sizeof(double2) * (size_t)nm * LNBK);
-   HIP_OK(hipHostMalloc((void **)&K.h, sizeof(double) * (2 * (size_t)nmx * nmx + 6 * (size_t)nmx), 0));
-   if (!K.v || !K.a || !K.bc || !K.c || !K.part || !K.h)
+   HIP_OK(hipHostMalloc((void **)&K.h, sizeof(double) * 4, 0));
+   if (!K.v || !K.a || !K.bc || !K.c || !K.part || !K.h || !lcount(nmx))
    {
       lkry_free(K);
       return false;
@@ -1348,9 +1406,12 @@ void dfl_free_grid()
    D.grid = D.basis_ok = D.aw_ok = D.awhat_ok = false;
    lkry_free(K32);
    lkry_free(K64);
+   dev_free(d_lcnt);
+   d_lcnt = nullptr;
+   lcnt_n = 0;
    dev_free(D.d_lw); dev_free(D.d_law); dev_free(D.d_lw32); dev_free(D.d_law32); dev_free(D.d_lM);
-   dev_free(D.d_lc); dev_free(D.d_ld); dev_free(D.d_lB); dev_free(D.d_lpart); dev_free(D.d_lbc);
-   D.d_lw = D.d_law = nullptr; D.d_lw32 = D.d_law32 = nullptr; D.d_lM = D.d_lc = D.d_ld = D.d_lB = nullptr;
+   dev_free(D.d_ld); dev_free(D.d_lB); dev_free(D.d_lpart); dev_free(D.d_lbc);
+   D.d_lw = D.d_law = nullptr; D.d_lw32 = D.d_law32 = nullptr; D.d_lM = D.d_ld = D.d_lB = nullptr;
    D.d_lpart = nullptr; D.d_lbc = nullptr;
    D.lm_ok = false;
    dev_free(D.d_gcoef); dev_free(D.d_ggram); dev_free(D.d_gscr);
@@ -1358,9 +1419,10 @@ void dfl_free_grid()
    D.gcap = 0;
 }
 
-// step n of the Gram-Schmidt process on chi_n (see above); returns false if
-// |chi_n| = 0, else the residual norm |rho| after the step in *rn
-template <typename C> bool lgs_step(LKry<C> &K, int n, C *rho, double *rn)
+// step n of the Gram-Schmidt process on chi_n (see above), next = the new
+// residual (next may be rho); returns false if |chi_n| = 0, else the residual
+// norm |next| in *rn
+template <typename C> bool lgs_step(LKry<C> &K, int n, const C *rho, C *next, double *rn)
 {
    Lib &L = lib();
    const size_t nv = K.nv;
@@ -1368,15 +1430,10 @@ template <typename C> bool lgs_step(LKry<C> &K, int n, C *rho, double *rn)
    double2 *acol = K.a + (size_t)n * K.nmx;
    double *bcn = K.bc + 4 * (size_t)n;
    if (n > 0)
-   {
-      k_lmdot<C><<<dim3(nbk, n), LRB, 0, L.stream>>>(K.chi(0), K.ld, K.chi(n), nv, K.part);
-      k_lsum<<<1, LRB, 0, L.stream>>>(K.part, nbk, n, acol);
-   }
-   k_lmaxpy<C><<<nbk, LRB, 0, L.stream>>>(K.chi(0), K.ld, n, nv, acol, rho, K.part);
-   k_lsum_bc<<<1, 64, 0, L.stream>>>(K.part, nbk, 0, bcn);
-   k_lscale<C><<<nbk, LRB, 0, L.stream>>>(K.chi(n), rho, nv, bcn, K.part);
-   k_lsum_bc<<<1, 64, 0, L.stream>>>(K.part, nbk, 1, bcn);
-   HIP_OK(hipMemcpyAsync(K.h, bcn, sizeof(double) * 4, hipMemcpyDeviceToHost, L.stream));
+      k_lmdot<C><<<dim3(nbk, n), LRB, 0, L.stream>>>(K.chi(0), K.ld, K.chi(n), nv, K.part, lcount(), acol, nullptr,
+                                                     1.0);
+   k_lmaxpy<C><<<nbk, LRB, 0, L.stream>>>(K.chi(0), K.ld, n, nv, acol, rho, K.part, lcount(), bcn);
+   k_lscale<C><<<nbk, LRB, 0, L.stream>>>(K.chi(n), rho, next, nv, bcn, K.part, lcount(), K.h);
    HIP_OK(hipStreamSynchronize(L.stream));
    *rn = sqrt(K.h[3]);
    return K.h[0] > 0.0;
@@ -1392,29 +1449,8 @@ template <typename C> void lgs_solution(LKry<C> &K, int m, C *x, int add)
       if (!add) HIP_OK(hipMemsetAsync(x, 0, sizeof(C) * K.nv, L.stream));
       return;
    }
-   const int nmx = K.nmx;
-   double *ha = K.h, *hb = K.h + 2 * (size_t)nmx * nmx, *hc = hb + 4 * (size_t)nmx;
-   HIP_OK(hipMemcpyAsync(ha, K.a, sizeof(double2) * (size_t)m * nmx, hipMemcpyDeviceToHost, L.stream));
-   HIP_OK(hipMemcpyAsync(hb, K.bc, sizeof(double) * 4 * (size_t)m, hipMemcpyDeviceToHost, L.stream));
-   HIP_OK(hipStreamSynchronize(L.stream));
-   for (int l = m - 1; l >= 0; l--)
-   {
-      double zr = hb[4 * l + 1], zi = hb[4 * l + 2];
-      for (int i = l + 1; i < m; i++)
-      {
-         // (chi_l, chi_i) is stored in column i
-         const double ar = ha[2 * ((size_t)i * nmx + l)], ai = ha[2 * ((size_t)i * nmx + l) + 1];
-         const double cr = hc[2 * i], ci = hc[2 * i + 1];
-         zr -= ar * cr - ai * ci;
-         zi -= ar * ci + ai * cr;
-      }
-      hc[2 * l] = zr / hb[4 * l];
-      hc[2 * l + 1] = zi / hb[4 * l];
-   }
-   HIP_OK(hipMemcpyAsync(K.c, hc, sizeof(double2) * (size_t)m, hipMemcpyHostToDevice, L.stream));
+   k_lback<<<1, 64, 0, L.stream>>>(K.a, K.nmx, K.bc, m, K.c);
    k_lcomb<C><<<(unsigned)((K.nv + LRB - 1) / LRB), LRB, 0, L.stream>>>(x, K.phi(0), K.ld, m, K.nv, K.c, add);
-   // the pinned coefficients must stay until the copy has run
-   HIP_OK(hipStreamSynchronize(L.stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -1427,17 +1463,6 @@ template <typename C> void lgs_solution(LKry<C> &K, int m, C *x, int add)
 // M = (P0 Ahat P0)^-1 (the Ns x Ns matrix (w_l, Ahat w_j)^-1), the little
 // solver works with P_L = 1 - Ahat P0 M P0, which removes the lowest modes of
 // Ahat from the Krylov iteration.  All coefficients stay on the device.
-
-// d[k] = sign * sum_l M[k][l] c[l], and d[Ns + k] = -d[k]
-__global__ __launch_bounds__(64) void k_lmatvec(const double2 *M, int Ns, const double2 *c, double sign, double2 *d)
-{
-   const int k = threadIdx.x;
-   if (k >= Ns) return;
-   double2 s = make_double2(0.0, 0.0);
-   for (int l = 0; l < Ns; l++) s = cadd(s, cmul(M[(size_t)k * Ns + l], c[l]));
-   d[k] = make_double2(sign * s.x, sign * s.y);
-   d[Ns + k] = make_double2(-sign * s.x, -sign * s.y);
-}
 
 // v /= bc[0] (bc[0] > 0)
 template <typename C> __global__ __launch_bounds__(LRB) void k_lnorm(C *v, size_t nv, const double *bc)
@@ -1455,9 +1480,7 @@ template <typename C> void lm_coef(const C *X, const C *v, double sign)
    Lib &L = lib();
    const size_t nv = (size_t)D.nbh * D.Ns;
    const int nbk = lnbk(nv);
-   k_lmdot<C><<<dim3(nbk, D.Ns), LRB, 0, L.stream>>>(X, D.ldv, v, nv, D.d_lpart);
-   k_lsum<<<1, LRB, 0, L.stream>>>(D.d_lpart, nbk, D.Ns, D.d_lc);
-   k_lmatvec<<<1, 64, 0, L.stream>>>(D.d_lM, D.Ns, D.d_lc, sign, D.d_ld);
+   k_lmdot<C><<<dim3(nbk, D.Ns), LRB, 0, L.stream>>>(X, D.ldv, v, nv, D.d_lpart, lcount(), D.d_ld, D.d_lM, sign);
 }
 
 template <typename C> void lm_comb(C *x, const C *Y, const double2 *c, int add)
@@ -1512,20 +1535,19 @@ int set_ltl_modes()
    if (!D.d_lw || D.ldv != ldv)
    {
       dev_free(D.d_lw); dev_free(D.d_law); dev_free(D.d_lw32); dev_free(D.d_law32); dev_free(D.d_lM);
-      dev_free(D.d_lc); dev_free(D.d_ld); dev_free(D.d_lB); dev_free(D.d_lpart); dev_free(D.d_lbc);
+      dev_free(D.d_ld); dev_free(D.d_lB); dev_free(D.d_lpart); dev_free(D.d_lbc);
       D.ldv = ldv;
       D.d_lw = (double2 *)dev_alloc(sizeof(double2) * ldv * Ns);
       D.d_law = (double2 *)dev_alloc(sizeof(double2) * ldv * Ns);
       D.d_lw32 = (float2 *)dev_alloc(sizeof(float2) * ldv * Ns);
       D.d_law32 = (float2 *)dev_alloc(sizeof(float2) * ldv * Ns);
       D.d_lM = (double2 *)dev_alloc(sizeof(double2) * Ns * Ns);
-      D.d_lc = (double2 *)dev_alloc(sizeof(double2) * Ns);
       D.d_ld = (double2 *)dev_alloc(sizeof(double2) * 2 * Ns);
       D.d_lB = (double2 *)dev_alloc(sizeof(double2) * Ns * Ns);
       D.d_lpart = (double2 *)dev_alloc(sizeof(double2) * (size_t)std::max(Ns, 2) * LNBK);
       D.d_lbc = (double *)dev_alloc(sizeof(double) * 4 * Ns);
-      if (!D.d_lw || !D.d_law || !D.d_lw32 || !D.d_law32 || !D.d_lM || !D.d_lc || !D.d_ld || !D.d_lB ||
-          !D.d_lpart || !D.d_lbc)
+      if (!D.d_lw || !D.d_law || !D.d_lw32 || !D.d_law32 || !D.d_lM || !D.d_ld || !D.d_lB ||
+          !D.d_lpart || !D.d_lbc || !lcount(Ns))
          return 1;
    }
    D.lm_ok = false;
@@ -1536,12 +1558,9 @@ int set_ltl_modes()
       double2 *wl = D.d_lw + (size_t)l * ldv;
       vconv<float2, double2>(D.d_vmds + (size_t)l * D.nb * Ns, wl, nv);
       if (l > 0)
-      {
-         k_lmdot<double2><<<dim3(nbk, l), LRB, 0, L.stream>>>(D.d_lw, ldv, wl, nv, D.d_lpart);
-         k_lsum<<<1, LRB, 0, L.stream>>>(D.d_lpart, nbk, l, acol);
-      }
-      k_lmaxpy<double2><<<nbk, LRB, 0, L.stream>>>(D.d_lw, ldv, l, nv, acol, wl, D.d_lpart);
-      k_lsum_bc<<<1, 64, 0, L.stream>>>(D.d_lpart, nbk, 0, D.d_lbc + 4 * l);
+         k_lmdot<double2><<<dim3(nbk, l), LRB, 0, L.stream>>>(D.d_lw, ldv, wl, nv, D.d_lpart, lcount(), acol, nullptr,
+                                                              1.0);
+      k_lmaxpy<double2><<<nbk, LRB, 0, L.stream>>>(D.d_lw, ldv, l, nv, acol, wl, D.d_lpart, lcount(), D.d_lbc + 4 * l);
       k_lnorm<double2><<<(unsigned)((nv + LRB - 1) / LRB), LRB, 0, L.stream>>>(wl, nv, D.d_lbc + 4 * l);
    }
    // Ahat w_l (vds2Avds) and the FP32 copies
@@ -1555,8 +1574,8 @@ int set_ltl_modes()
    // B[l][j] = (w_l, Ahat w_j), stored by columns (set_Ads)
    for (int j = 0; j < Ns; j++)
    {
-      k_lmdot<double2><<<dim3(nbk, Ns), LRB, 0, L.stream>>>(D.d_lw, ldv, D.d_law + (size_t)j * ldv, nv, D.d_lpart);
-      k_lsum<<<1, LRB, 0, L.stream>>>(D.d_lpart, nbk, Ns, D.d_lB + (size_t)j * Ns);
+      k_lmdot<double2><<<dim3(nbk, Ns), LRB, 0, L.stream>>>(D.d_lw, ldv, D.d_law + (size_t)j * ldv, nv, D.d_lpart,
+                                                            lcount(), D.d_lB + (size_t)j * Ns, nullptr, 1.0);
    }
    std::vector<double2> Bc((size_t)Ns * Ns);
    std::vector<double> bc(4 * (size_t)Ns);
@@ -1618,21 +1637,21 @@ int gcr4v(int nmx, double res, const float2 *b, float2 *x)
 {
    const size_t nv = (size_t)D.nbh * D.Ns;
    if (!lkry_alloc(K32, nmx, nv)) return -1;
-   float2 *rho = wv(0), *t = wv(1);
+   float2 *t = wv(1);
    Lib &L = lib();
-   HIP_OK(hipMemcpyAsync(rho, b, sizeof(float2) * nv, hipMemcpyDeviceToDevice, L.stream));
+   // phi_n is the residual of step n, so the step writes the next one there
+   HIP_OK(hipMemcpyAsync(K32.phi(0), b, sizeof(float2) * nv, hipMemcpyDeviceToDevice, L.stream));
    double r0;
-   vdot<float2>(rho, rho, nv, nullptr, nullptr, &r0);
+   vdot<float2>(b, b, nv, nullptr, nullptr, &r0);
    r0 = sqrt(r0);
    double rn = r0;
    int n = 0, status = -1;
    if (r0 > 0.0)
       for (; n < nmx; n++)
       {
-         ahat<float2>(D.d_MT32, rho, t, K32.chi(n));
+         ahat<float2>(D.d_MT32, K32.phi(n), t, K32.chi(n));
          dfl_Lv_dev(K32.chi(n));
-         HIP_OK(hipMemcpyAsync(K32.phi(n), rho, sizeof(float2) * nv, hipMemcpyDeviceToDevice, L.stream));
-         if (!lgs_step(K32, n, rho, &rn)) break;
+         if (!lgs_step<float2>(K32, n, K32.phi(n), K32.phi(n + 1), &rn)) break;
          if (rn <= res * r0)
          {
             n++;
@@ -2121,7 +2140,7 @@ double ltl_solve(const double2 *eta, double2 *psi, int *ifail, int *status)
             vconv<float2, double2>(x32, K64.phi(k), nv);
             ahat<double2>(D.d_MT, K64.phi(k), t, K64.chi(k));
             if (D.lm_ok) dfl_RLvd_dev(K64.phi(k), K64.chi(k));
-            if (!lgs_step(K64, k, r, &rn))
+            if (!lgs_step<double2>(K64, k, r, r, &rn))
             {
                zero = true;
                break;
@@ -2295,8 +2314,8 @@ extern "C" double dfl_sap_gcr(int nkv, int nmx, int istop, double res, double mu
       {
          alloc_ws(L.ws_used + 2 * nkv + 1);
          alloc_wsd(L.wsd_used + 2);
-         spinor **ws = reserve_ws(2 * nkv + 1);
-         spinor_dble **wsd = reserve_wsd(2);
+         spinor **ws = take_ws(2 * nkv + 1, false);
+         spinor_dble **wsd = take_wsd(2, false);
          spinor_dble *rsd = wsd[1];
          assign_sd2sd(vt, 2, eta, rsd);
          scale_dble(vt, 2, 1.0 / rho0, rsd);
