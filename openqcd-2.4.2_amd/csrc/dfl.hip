@@ -1117,11 +1117,11 @@ float2 *wv(int k)
 // to its memory.  Little vectors are short (24^4, Ns = 20: 100 KB), so a step
 // is bound by its launches: the work-group of a kernel that finishes last adds
 // the shares of all (last_group) instead of a kernel after it, and the back
-// substitution of the solution runs on the device.  14 launches per step, 5
+// substitution of the solution runs on the device.  14 launches per step, 3
 // copies and 2 synchronisations per solution became 8 launches, no copy and no
-// synchronisation (dfl_sap_gcr at 24^4, 11 vectors: 24.6 -> 22.4 ms).  The sums are taken in
-// double precision in a fixed order (per lane, per work-group, then over the
-// work-groups), so the results do not depend on the launch timing.
+// synchronisation (dfl_sap_gcr at 24^4, 11 vectors: 24.6 -> 22.4 ms).  The sums
+// are taken in double precision in a fixed order (per lane, per work-group, then
+// over the work-groups), so the results do not depend on the launch timing.
 
 constexpr int LRB = 256;     // lanes of the little-vector kernels
 constexpr int LNBK = 512;    // largest number of work-groups of a reduction
