@@ -102,6 +102,14 @@ void oqh_set_sap_prec(int prec);
    launched kernel by kernel (0); no counterpart in the reference, the
    results are the same */
 void oqh_set_sap_graph(int on);
+/* bound on the waits between the work-groups that share a Schwarz block
+   (FP32 cycles, block sizes that are multiples of 4 and not 4^4): a wait is
+   given up after n polls of about a microsecond (default 4194304).  The call
+   that ran the cycles then fails: sap() leaves host arrays as they were,
+   fgcr() and the solvers end with status -1 (ifail -1), dfl_modes() and
+   dfl_update() with ifail -1 and no subspace.  No counterpart in the
+   reference. */
+void oqh_set_sap_polls(int n);
 /* SAP block-size autotuner (no counterpart in the reference): among the
    legal block sizes of sap_parms.c (even, >= 4, an even number of blocks per
    axis; here with equal spatial sizes and at most maxvol points, 4096 if

@@ -2437,9 +2437,20 @@ void dfl_smooth_fields(spinor **mds, spinor **ws, int *st)
    }
 }
 
+// true if a Schwarz cycle of the generation did not finish: the modes are
+// useless (ifail = -1, which no other fault has)
+bool gen_gave_up(const char *where, int *ifail)
+{
+   HIP_OK(hipStreamSynchronize(lib().stream));
+   if (!sap_gave_up(where)) return false;
+   D.basis_ok = D.aw_ok = D.awhat_ok = false;
+   ifail[0] = -1;
+   return true;
+}
+
 // n deflated steps (set_Awhat, dfl_smooth_fields, renormalisation, new
 // subspace) while ifail[0] == 0; returns the number of steps done
-int dfl_steps(int n, spinor **mds, spinor **ws, int *ifail, int *status)
+int dfl_steps(const char *where, int n, spinor **mds, spinor **ws, int *ifail, int *status)
 {
    int k = 0;
    for (; k < n && ifail[0] == 0; k++)
@@ -2452,6 +2463,7 @@ int dfl_steps(int n, spinor **mds, spinor **ws, int *ifail, int *status)
       dfl_smooth_fields(mds, ws, status);
       dfl_renormalize_modes(mds);
       dfl_subspace(mds);
+      gen_gave_up(where, ifail);
    }
    return k;
 }
@@ -2493,16 +2505,19 @@ extern "C" void dfl_modes(int *ifail, int *status)
    else
    {
       // smooth_fields: n+1 Schwarz cycles on D psi = mds[l], n = 0, 1, 2
-      for (int n = 0; n < 3; n++)
+      for (int n = 0; n < 3 && ifail[0] == 0; n++)
+      {
          for (int l = 0; l < D.Ns; l++)
          {
             assign_s2s(vt, 2, mds[l], ws[0]);
             gen_cycles(mus, n + 1, mds[l], ws[0]);
          }
-      dfl_subspace(mds);
-      const int nd = dfl_steps(D.ninv - 3, mds, ws, ifail, status);
+         gen_gave_up(where, ifail);
+      }
+      if (ifail[0] == 0) dfl_subspace(mds);
+      const int nd = dfl_steps(where, D.ninv - 3, mds, ws, ifail, status);
       average_status(D.Ns * nd, status);
-      gen_done = true;
+      gen_done = ifail[0] != -1;
    }
    release_ws();
    release_ws();
@@ -2530,8 +2545,9 @@ extern "C" void dfl_update(int nsm, int *ifail, int *status)
       spinor **mds = reserve_ws(D.Ns);
       spinor **ws = reserve_ws(2);
       dfl_restore_modes(mds);
-      const int nd = dfl_steps(nsm, mds, ws, ifail, status);
+      const int nd = dfl_steps(where, nsm, mds, ws, ifail, status);
       average_status(D.Ns * nd, status);
+      if (ifail[0] == -1) gen_done = false;
       release_ws();
       release_ws();
    }

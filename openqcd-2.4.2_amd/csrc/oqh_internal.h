@@ -69,6 +69,7 @@ struct Lib
    int sap_bs[4] = {0, 0, 0, 0}, sap_isolv = 0, sap_nmr = 0, sap_ncy = 0;
    int sap_prec = 0;  // SAP storage: 0 FP32, 1 FP16 links, SW and spinors (per-site scales)
    int sap_graph = 1; // FP16 preconditioner of sap_gcr replayed as a HIP graph
+   int sap_polls = 1 << 22;  // polls of a wait between the work-groups of a Schwarz block
    int gcr_cgs = 1;
    int nn_prec = 0;   // network correction in the preconditioner of sap_gcr   // fgcr orthogonalisation on the device: 1 two-pass (compact WY) MGS, 0 per-term MGS
 
@@ -155,6 +156,7 @@ void finish(const Res &r, int prec, int nsites, bool download);
 void build_geometry(Geometry &g, const int *L, const int *Ltrd);
 void upload_tables();
 void sap_release();  // frees the SAP block grid (made for the current geometry)
+bool sap_gave_up(const char *where);  // a Schwarz cycle did not finish (sap.hip)
 void release_flow(); // frees the force field of the Wilson flow
 void release_nn();   // frees the network of the learned preconditioner
 void release_rng();  // frees the device random number streams

@@ -1184,8 +1184,10 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const int *imb, 
 // missing work-groups as the others end.  A block needs only as many
 // work-groups running at once as it has sub-blocks (at most CLMAX, far fewer
 // than the device holds), and no wait depends on the order in which
-// work-groups are started.  Waits are bounded all the same: a work-group that
-// has waited CLSPIN times gives up waiting for good and reports it.
+// work-groups are started.  Waits are bounded all the same: a wavefront that
+// has polled Lib::sap_polls times gives up waiting for good, the kernel ends
+// with incomplete sums and faces, and the call that launched it reports the
+// error once it has waited for the stream (sap_gave_up).
 //
 // The exchanged values are written and read with relaxed atomics of device
 // scope; a work-group counts itself in after its writes have completed.  Two
@@ -1221,7 +1223,6 @@ template <bool COR> __device__ inline void lds_store(const SArgs &a, int gx, con
 }
 
 constexpr int CLMAX = 64;         // sub-blocks of a block
-constexpr int CLSPIN = 1 << 22;   // polls of a wait
 constexpr int CLPAD = 64;         // distance of the counters: a line each
 constexpr int CLSLEEP = 8;        // pause between polls, 64 clocks each
 
@@ -1234,6 +1235,7 @@ struct ClArgs
    unsigned long long *x;      // [2][nbh][ns] face fields
    unsigned long long *sums;   // [nbh][ns][4]
    size_t xlen;                // length of one of the two
+   int polls;                  // polls of a wait
    int *dead;                  // set if a wait was given up (host memory)
 };
 
@@ -1280,7 +1282,7 @@ __device__ inline void cl_wait(const ClArgs &q, ClState &st)
    int k = 0;
    while (!st.gone && __hip_atomic_load(q.count + (size_t)st.bi * CLPAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want)
    {
-      if (++k >= CLSPIN)
+      if (++k >= q.polls)
       {
          st.gone = true;
          __hip_atomic_store(q.dead, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2462,7 +2464,6 @@ template <int TPB> static void launch_lds(const SArgs &a, int isolv, unsigned nb
 static void launch_cluster(const SArgs &a, int isolv)
 {
    hipStream_t st = lib().stream;
-   if (*G.h_dead) fail("sap [sap.c]", "a work-group of a Schwarz block did not get its neighbours' values");
    ClArgs q;
    q.ns = G.ns;
    q.imb4 = G.d_imb4;
@@ -2472,6 +2473,7 @@ static void launch_cluster(const SArgs &a, int isolv)
    q.x = G.d_x;
    q.xlen = (size_t)G.nbh * G.ns * FUN;
    q.sums = G.d_x + 2 * q.xlen;
+   q.polls = lib().sap_polls;
    q.dead = G.h_dead;
    const unsigned nb = (unsigned)(G.nbh * G.ns);
    k_cl_reset<<<(G.nbh + 256) / 256, 256, 0, st>>>(G.d_count, G.nbh + 1);
@@ -2957,6 +2959,17 @@ bool sap_prepare(int isolv, const char *where, bool quiet)
    return true;
 }
 
+// true if a wait in the Schwarz cycles since the last call was given up, so
+// that what they left is wrong: an error at where (none for a null pointer).
+// The caller has waited for the stream.
+bool sap_gave_up(const char *where)
+{
+   if (!G.h_dead || !*(volatile int *)G.h_dead) return false;
+   *G.h_dead = 0;
+   if (where) fail(where, "a work-group of a Schwarz block did not get its neighbours' values");
+   return true;
+}
+
 int sap_grid_nblocks() { return G.ready ? G.nb : 0; }
 
 // the grid belongs to the geometry: released with it
@@ -2984,6 +2997,11 @@ extern "C" void sap(float mu, int isolv, int nmr, spinor *psi, spinor *eta)
       return;
    }
    sap_cycles(mu, isolv, nmr, 1, (float2 *)p.dev, (float2 *)r.dev, false, true);
+   if (G.ns)
+   {
+      HIP_OK(hipStreamSynchronize(L.stream));
+      if (sap_gave_up("sap [sap.c]")) return;
+   }
    finish(p, F32, V, true);
    finish(r, F32, V, true);
 }
@@ -3058,6 +3076,16 @@ extern "C" void oqh_set_sap_graph(int on)
       return;
    }
    lib().sap_graph = on;
+}
+
+extern "C" void oqh_set_sap_polls(int n)
+{
+   if (n < 1)
+   {
+      fail("oqh_set_sap_polls", "the number of polls must be positive");
+      return;
+   }
+   lib().sap_polls = n;
 }
 
 extern "C" void oqh_set_sap_prec(int prec)
@@ -3469,7 +3497,7 @@ extern "C" double oqh_sap_autotune(int isolv, int nmr, int ncy, int maxvol, int 
       float ms = 0.0f;
       HIP_OK(hipEventElapsedTime(&ms, e0, e1));
       const double r1 = field_norm(rho, nu, d_part, h_part);
-      if (!(r1 > 0.0) || r1 >= r0) continue;
+      if (sap_gave_up(nullptr) || !(r1 > 0.0) || r1 >= r0) continue;
       const double score = 1e-3 * ms / log(r0 / r1);
       if (best == 0.0 || score < best)
       {

@@ -143,6 +143,11 @@ extern "C" double fgcr(int vol, void (*Dop)(spinor_dble *s, spinor_dble *r),
             }
             HIP_OK(hipMemcpyAsync(hcoef, dcoef, sizeof(float2) * (nkv + 3), hipMemcpyDeviceToHost, L.stream));
             HIP_OK(hipStreamSynchronize(L.stream));
+            if (sap_gave_up("fgcr [fgcr.c]"))
+            {
+               status[0] = -1;
+               return rn_old;
+            }
             for (int l = 0; l < k; l++)
             {
                a[(size_t)nkv * l + k].re = hcoef[l].x;
@@ -174,6 +179,11 @@ extern "C" double fgcr(int vol, void (*Dop)(spinor_dble *s, spinor_dble *r),
          z.im = -c[k].im;
          mulc_spinor_add(vol, 2, rho, chi[k], z);
          rn = get_res(vol, istop, rho);
+         if (sap_gave_up("fgcr [fgcr.c]"))
+         {
+            status[0] = -1;
+            return rn_old;
+         }
          status[0] += 1;
          if (rn <= tol || rn < PRECISION_LIMIT * rn_old || k == nkv - 1 || status[0] >= nmx) break;
       }

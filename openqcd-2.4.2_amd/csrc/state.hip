@@ -611,6 +611,7 @@ extern "C" void oqh_finalize(void)
    release_dfl();
    L.nn_prec = 0;
    L.sap_graph = 1;
+   L.sap_polls = Lib().sap_polls;
    for (auto &kv : L.reg) dev_free(kv.second.base);
    L.reg.clear();
    for (int k = 0; k < 4; k++)

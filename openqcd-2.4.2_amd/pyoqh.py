@@ -78,7 +78,7 @@ _SIG = {
     "set_ud_phase": (None, []), "unset_ud_phase": (None, []),
     "oqh_set_sap_prec": (None, [_I]),
     "oqh_set_gcr_orth": (None, [_I]),
-    "oqh_set_sap_graph": (None, [_I]),
+    "oqh_set_sap_graph": (None, [_I]), "oqh_set_sap_polls": (None, [_I]),
     "oqh_sap_autotune": (_D, [_I, _I, _I, _I, P]),
     "start_ranlux": (None, [_I, _I]), "random_ud": (None, []),
     "random_sd": (None, [_I, _I, P, _D]), "oqh_random_source": (None, [_I, P]), "oqh_random_start_field": (None, [P]), "ranlxd": (None, [P, _I]),
