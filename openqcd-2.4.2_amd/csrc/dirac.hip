@@ -736,7 +736,7 @@ template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(
            (size_t)(6 * hh + 2 * wr) * SB;
    op[0] = out[0];
    op[SB] = out[1];
-   if (OP == SP_DW && bp)
+   if (OP == SP_DW && bp && a.s_w)
    {
       C *ip = a.s_w + (size_t)(x >> 6) * (12 * SB) + (x & (SB - 1)) + (size_t)(6 * hh + 2 * wr) * SB;
       ip[0] = ip[SB] = cmk<C>(0, 0);
@@ -745,22 +745,21 @@ template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(
 
 // ---------------------------------------------------------------------------
 // Dw / Dw_dble on several fields at once (no reference counterpart): tiles of
-// 64 even and 64 odd points, each worked on by one wavefront per field.  The
-// four wavefronts of a work-group take the same tile for four fields and
-// share its links and SW matrices through the L1, the groups of four follow
-// each other on one XCD and share them through its L2.  A wavefront exchanges
-// hopping terms with itself only, so there are no barriers.
-// 12 fields FP64 at 24^4: 0.83 ms against 1.11 ms with 8 lanes per pair of
-// points, 256-lane work-groups and barriers.  Bound by the 4.9 GB that miss
-// the L2 (the neighbours in x2 and x3 lie four to eight lines apart).  Two
-// fields per work-group: 0.85 ms; all tiles of a thread block for four fields
-// before the next four: 0.90 ms; third link rows rebuilt and the S-form of
-// the SW term, as Dw_dble has them: 0.80 ms, but twice the rounding error
-// (3e-16 for 1.3e-16), so the stored links are read.
+// TP even and TP odd points, each worked on by TP lanes per field.  The W
+// fields of a work-group share the links and SW matrices of their tile through
+// the L1, the work-groups of the same tile follow each other on one XCD and
+// share them through its L2.  With TP = 64 a wavefront exchanges hopping terms with
+// itself only, so there are no barriers.
+// 12 fields FP64 at 24^4: 0.83 ms with W = 4, TP = 64, against 1.11 ms with 8
+// lanes per pair of points, 256-lane work-groups and barriers.  Bound by the
+// 4.9 GB that miss the L2 (the neighbours in x2 and x3 lie four to eight lines
+// apart).  All tiles of a thread block for four fields before the next four:
+// 0.90 ms; third link rows rebuilt and the S-form of the SW term, as Dw_dble
+// has them: 0.80 ms, but twice the rounding error (3e-16 for 1.3e-16), so the
+// stored links are read.
 // ---------------------------------------------------------------------------
 
-constexpr int MTP = 64;    // pairs of points per tile
-constexpr int MWV = 4;     // fields per work-group
+constexpr int MWV = 4;     // fields per work-group, at most
 constexpr int NRMAX = 16;  // fields per launch
 
 template <typename T> struct MFields
@@ -768,21 +767,22 @@ template <typename T> struct MFields
    typedef typename cplx_of<T>::t C;
    const C *s[NRMAX];
    C *r[NRMAX];
-   int n, ng;  // fields, groups of MWV fields
+   int n, ng;  // fields, groups of W fields
 };
 
-template <typename T> __global__ __launch_bounds__(MWV * 64) void k_dw_multi(DArgs<T> a, MFields<T> f)
+// TP > 64: n is a multiple of W (the barriers are for all lanes)
+template <typename T, int W, int TP> __global__ __launch_bounds__(W * TP) void k_dw_multi(DArgs<T> a, MFields<T> f)
 {
    typedef typename cplx_of<T>::t C;
-   __shared__ C S[MWV][12][MTP];
-   __shared__ C X[MWV][XBUF][6][MTP];
+   __shared__ C S[W][12][TP];
+   __shared__ C X[W][XBUF][6][TP];
    const int b = xcd_tile(blockIdx.x, gridDim.x, a.xcdc);
-   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-   const int k = (b % f.ng) * MWV + w;
+   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / TP);
+   const int k = (b % f.ng) * W + w;
    if (k >= f.n) return;
    a.s = f.s[k];
    a.r = f.r[k];
-   dw_tile<T, MTP, false, false, false>(a, threadIdx.x & 63, (b / f.ng) * MTP, S[w], X[w]);
+   dw_tile<T, TP, false, false, false>(a, threadIdx.x & (TP - 1), (b / f.ng) * TP, S[w], X[w]);
 }
 
 template <typename T>
@@ -1152,36 +1152,54 @@ extern "C" void Dwhat(float mu, spinor *s, spinor *r) { apply<float>(K_HAT, mu, 
 
 namespace oqh {
 
-// n fields in launches of up to NRMAX
+// run: tiles per XCD run
+template <typename T, int W, int TP> static void launch_multi(DArgs<T> a, MFields<T> f, int run)
+{
+   f.ng = (f.n + W - 1) / W;
+   a.xcdc = run * f.ng;
+   const unsigned nt = (unsigned)((a.h + TP - 1) / TP);
+   k_dw_multi<T, W, TP><<<nt * f.ng, W * TP, 0, lib().stream>>>(a, f);
+}
+
+// n fields in launches of up to NRMAX, in as few groups of at most MWV fields
+// as hold them, of the same size but for the last one.  A work-group has
+// the LDS of all its fields, so one with fields missing leaves part of the CU
+// empty (5 fields FP64 as 4 + 1 of 4 at 32^3x64: 2.89 ms, as 3 + 2 of 3: 2.50;
+// one field in a group of four: 0.97 ms, by itself 0.72).  One field goes to the
+// kernels of the single operators, with the stored links and SW matrices.  Two on
+// a large lattice go in tiles of 128 pairs, with fewer neighbours outside
+// (FP64 / FP32 at 32^3x64: 1.12 / 0.62 ms, tiles of 64: 1.17 / 0.65, at 24^4 208
+// / 105 against 222 / 112 us, but at 16^4 43.3 / 29.2 against 42.4 / 25.4 us).
+// Runs of 16 tiles of 64 or 2 tiles of 128 pairs (2-32: within 5 %).
 template <typename T> static void apply_multi(T mu, int n, void **sp, void **rp, const char *where)
 {
    typedef typename cplx_of<T>::t C;
+   const int prec = (sizeof(T) == 8) ? F64 : F32;
    Lib &L = lib();
-   int prec = sizeof(T) == 8 ? F64 : F32;
    if (!prepare(where, prec)) return;
-   if (n < 1 || !sp || !rp)
+   if (n <= 0)
    {
       fail(where, "the number of fields must be positive");
       return;
    }
    DArgs<T> a = base_args<T>();
+   a.lsign = nullptr;
+   a.sws_par = 0;
    a.mu = mu;
    a.muo = L.eoflg ? (T)0 : mu;
    a.coef = (T)-0.5;
-   const unsigned nt = (unsigned)((a.h + MTP - 1) / MTP);
+   const bool small = use_split(prec, a.h);
    for (int k0 = 0; k0 < n; k0 += NRMAX)
    {
       MFields<T> f;
       f.n = std::min(NRMAX, n - k0);
-      f.ng = (f.n + MWV - 1) / MWV;
-      a.xcdc = 16 * f.ng;  // runs of 16 tiles per XCD (2 tiles: 5 % slower, 32: 1 %)
       for (int k = 0; k < f.n; k++)
       {
          int o1 = 0, o2 = 0;
          void *s = device_field(sp[k0 + k], prec, &o1), *r = device_field(rp[k0 + k], prec, &o2);
          if (!s || !r || o1 || o2)
          {
-            fail(where, "the fields must be full device fields of the library");
+            fail(where, "the arguments must be full device fields");
             return;
          }
          if (s == r)
@@ -1192,8 +1210,26 @@ template <typename T> static void apply_multi(T mu, int n, void **sp, void **rp,
          f.s[k] = (const C *)s;
          f.r[k] = (C *)r;
       }
-      const unsigned nb = nt * f.ng;
-      k_dw_multi<T><<<nb, MWV * 64, 0, L.stream>>>(a, f);
+      const int ng = (f.n + MWV - 1) / MWV, w = (f.n + ng - 1) / ng;
+      if (f.n == 1)
+      {
+         DArgs<T> b = a;
+         b.s = f.s[0];
+         b.r = f.r[0];
+         b.xcdc = 32;
+         if (small)
+            launch_split<T, SP_DW>(b, 0, a.V);
+         else
+            launch_dw<T>(b);
+      }
+      else if (f.n == 2 && !small)
+         launch_multi<T, 2, 128>(a, f, 2);
+      else if (w == 2)
+         launch_multi<T, 2, 64>(a, f, 16);
+      else if (w == 3)
+         launch_multi<T, 3, 64>(a, f, 16);
+      else
+         launch_multi<T, MWV, 64>(a, f, 16);
    }
 }
 

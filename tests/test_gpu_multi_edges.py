@@ -51,3 +51,42 @@ def test_multi_edges(L, bc, su3, pset, n):
                 lat.free(f)
     finally:
         lat.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,prec", [((24, 18, 18, 14), 64), ((26, 22, 22, 22), 32)])
+@pytest.mark.parametrize("bc", [3, 0])
+@pytest.mark.parametrize("n", [1, 2, 3, 18])
+def test_few_fields(L, prec, bc, n):
+    """Lattices beyond the split kernel's, where one field takes the tiles of
+    the single operator and two take tiles of 128 pairs (V/2 is no multiple of
+    them): the inputs stay, also on the boundary points of open bc, where the
+    output vanishes."""
+    print("L", L, "prec", prec, "bc", bc, "n", n, flush=True)
+    rng = np.random.default_rng(8)
+    lat = pyoqh.Lattice(L, None, bc=bc, m0=-0.2, csw=1.77)
+    try:
+        V = lat.V
+        lat.lib.start_ranlux(0, 9)
+        lat.lib.random_ud()
+        assert lat.sw_term(3) == 0
+        alloc, put, get = ((lat.alloc_sd, lat.put_sd, lat.get_sd) if prec == 64 else
+                           (lat.alloc_s, lat.put_s, lat.get_s))
+        fs = rng.standard_normal((V, 24)).astype(np.float64 if prec == 64 else np.float32)
+        s, r = [alloc() for _ in range(n)], [alloc() for _ in range(n)]
+        one, ref = alloc(), alloc()
+        for k in range(n):
+            put(s[k], fs * (k + 1))
+        put(one, fs)
+        multi, single = ((lat.lib.oqh_Dw_dble_multi, lat.lib.Dw_dble) if prec == 64 else
+                         (lat.lib.oqh_Dw_multi, lat.lib.Dw))
+        multi(0.03, n, (P * n)(*s), (P * n)(*r))
+        single(0.03, one, ref)
+        b = get(ref)
+        for k in range(n):
+            assert np.array_equal(get(s[k]), fs * (k + 1))
+            a = get(r[k])
+            assert not a[(b == 0).all(axis=1)].any()
+            assert np.linalg.norm(a - (k + 1) * b) <= (1e-14 if prec == 64 else 1e-6) * np.linalg.norm((k + 1) * b)
+    finally:
+        lat.close()
