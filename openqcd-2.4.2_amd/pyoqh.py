@@ -59,6 +59,7 @@ class DflGenParms(C.Structure):
 _SIG = {
     "oqh_init": (_I, [_I]), "oqh_finalize": (None, []),
     "oqh_set_error_mode": (None, [_I]), "oqh_last_error": (_I, [C.c_char_p, _I]),
+    "oqh_set_alloc_max": (None, [C.c_ulonglong]),
     "oqh_geometry": (_I, [P, P]), "oqh_volume": (_I, []), "oqh_get_ipt": (None, [P]),
     "oqh_set_bc_parms": (None, [_I, _D, _D]), "oqh_set_sw_parms": (None, [_D, _D]),
     "oqh_set_tm_parms": (None, [_I]), "oqh_set_sap_parms": (None, [P, _I, _I, _I]),
