@@ -415,14 +415,19 @@ __global__ __launch_bounds__(64 * WSW) void k_ptc_wgrad_sum(const float2 *part, 
    grad[e].y += (float)zi;
 }
 
+// point of a unit of a spinor field; the last storage block may have more
+// than the lattice
+__device__ inline int unit_point(int k) { return k / (12 * SB) * SB + (k & (SB - 1)); }
+
 // loss terms of a sample (blockIdx.y): partial sums of |e|^2 and |out - e|^2
-__global__ void k_ptc_loss(Batch bt, int n, double *part)
+__global__ void k_ptc_loss(Batch bt, int V, int n, double *part)
 {
    const float2 *out = (const float2 *)bt.out[blockIdx.y], *e = (const float2 *)bt.in[blockIdx.y];
    __shared__ double sh[2][256];
    double se = 0.0, sd = 0.0;
    for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256)
    {
+      if (unit_point(k) >= V) continue;
       float2 a = out[k], b = e[k];
       double dx = (double)a.x - b.x, dy = (double)a.y - b.y;
       se += (double)b.x * b.x + (double)b.y * b.y;
@@ -472,14 +477,14 @@ __global__ __launch_bounds__(64) void k_ptc_loss_sum(const double *part, int nb,
 
 // output gradient of the mean loss over npair pairs, g = 2 (out - e) /
 // (npair |e|^2) in place of out (0 for a pair without target)
-__global__ void k_ptc_lgrad(Batch bt, const double *sums, int npair, int n)
+__global__ void k_ptc_lgrad(Batch bt, const double *sums, int npair, int V, int n)
 {
    const float2 *e = (const float2 *)bt.in[blockIdx.y];
    float2 *g = (float2 *)bt.out[blockIdx.y];
    const double se = sums[2 * blockIdx.y];
    const float c = se > 0.0 ? (float)(2.0 / (se * npair)) : 0.0f;
    const int k = blockIdx.x * 256 + threadIdx.x;
-   if (k < n) g[k] = make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y));
+   if (k < n && unit_point(k) < V) g[k] = make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y));
 }
 
 // Adam step on n reals
@@ -518,9 +523,9 @@ struct Net
    int adam_t = 0;
    int V = 0;
    int nbatch = 0;                 // samples the following fields hold
+   int cap = NBMAX;                // samples there was memory for
    float2 *d_act[NLMAX + 1] = {};  // activations of the last forward
-   float2 *d_out = nullptr;        // its outputs, then the output gradients
-   float2 *d_gb[2] = {};           // backward gradients (ping-pong)
+   float2 *d_gb[2] = {};           // outputs, then the gradients of the layers (ping-pong)
    float2 *d_part = nullptr;       // weight-gradient partials
    double *d_lpart = nullptr, *d_lsum = nullptr, *h_lsum = nullptr;  // loss terms
    float2 *d_tmp = nullptr;         // spinor work field of the preconditioner
@@ -539,7 +544,6 @@ void free_net()
    for (int l = 0; l < NLMAX; l++) { dev_free(N.d_pf[l]); dev_free(N.d_pa[l]); }
    for (int l = 0; l <= NLMAX; l++) dev_free(N.d_act[l]);
    dev_free(N.d_gb[0]); dev_free(N.d_gb[1]); dev_free(N.d_part); dev_free(N.d_lpart); dev_free(N.d_lsum); dev_free(N.d_tmp);
-   dev_free(N.d_out);
    dev_free(N.d_inf[0]); dev_free(N.d_inf[1]); dev_free(N.d_u16);
    if (N.h_lsum) HIP_OK(hipHostFree(N.h_lsum));
    N = Net();
@@ -559,13 +563,14 @@ void pack()
    N.packed = true;
 }
 
-// samples that are worked on together: as many as 2 GiB of activations and
-// gradients allow (a batch of 16 at 16^4; one at 32^3x64, whose layers fill
-// the device by themselves)
+// samples that are worked on together: as many as 2 GiB of activations,
+// gradients and weight-gradient shares allow (a batch of 16 at 16^4; one at
+// 32^3x64, whose layers fill the device by themselves), and no more than could
+// be allocated before (N.cap)
 int batch_size(int n)
 {
    const size_t V = lib().g.V;
-   size_t units = 12;
+   size_t units = 0;
    int wmax = 4;
    for (int l = 1; l < N.nl; l++)
    {
@@ -573,36 +578,36 @@ int batch_size(int n)
       wmax = std::max(wmax, N.w[l]);
    }
    units += 2 * 3 * wmax;
-   const size_t bytes = V * units * sizeof(float2);
-   return (int)std::max<size_t>(1, std::min<size_t>(std::min(n, NBMAX), ((size_t)2 << 30) / bytes));
+   const size_t bytes = V * (units + NDIR * CMAX * CMAX / PNS) * sizeof(float2);
+   return (int)std::max<size_t>(1, std::min<size_t>(std::min(n, N.cap), ((size_t)2 << 30) / bytes));
 }
 
-// activations of nb samples for the current lattice
+// activations of nb samples for the current lattice; the fields of several
+// samples are given up without an error if they cannot be had
 bool ensure_fields(int nb = 1)
 {
    Lib &L = lib();
    if (N.V == L.g.V && N.nbatch >= nb) return true;
+   auto alloc = [nb](size_t bytes) { return nb > 1 ? dev_try_alloc(bytes) : dev_alloc(bytes); };
    HIP_OK(hipStreamSynchronize(L.stream));
    for (int l = 0; l <= NLMAX; l++) { dev_free(N.d_act[l]); N.d_act[l] = nullptr; }
    for (int k = 0; k < 2; k++) { dev_free(N.d_gb[k]); N.d_gb[k] = nullptr; }
-   dev_free(N.d_part); dev_free(N.d_out);
+   dev_free(N.d_part);
+   N.d_part = nullptr;
    N.nbatch = 0;
    const size_t V64 = units_for(L.g.V, 1);
    int wmax = 4;
    bool ok = true;
    for (int l = 1; l < N.nl; l++)
    {
-      N.d_act[l] = (float2 *)dev_alloc(nb * V64 * 3 * N.w[l] * sizeof(float2));
+      N.d_act[l] = (float2 *)alloc(nb * V64 * 3 * N.w[l] * sizeof(float2));
       wmax = std::max(wmax, N.w[l]);
       ok = ok && N.d_act[l];
    }
-   for (int k = 0; k < 2; k++) N.d_gb[k] = (float2 *)dev_alloc(nb * V64 * 3 * wmax * sizeof(float2));
+   for (int k = 0; k < 2; k++) N.d_gb[k] = (float2 *)alloc(nb * V64 * 3 * wmax * sizeof(float2));
    const int np = (L.g.V + PNS - 1) / PNS;
-   N.d_part = (float2 *)dev_alloc((size_t)nb * np * NDIR * CMAX * CMAX * sizeof(float2));
-   N.d_out = (float2 *)dev_alloc(nb * V64 * 12 * sizeof(float2));
-   ok = ok && N.d_gb[0] && N.d_gb[1] && N.d_part && N.d_out;
-   // the unused end of a field's last storage block takes part in the loss
-   if (N.d_out) HIP_OK(hipMemsetAsync(N.d_out, 0, nb * V64 * 12 * sizeof(float2), L.stream));
+   N.d_part = (float2 *)alloc((size_t)nb * np * NDIR * CMAX * CMAX * sizeof(float2));
+   ok = ok && N.d_gb[0] && N.d_gb[1] && N.d_part;
    if (N.V != L.g.V)
    {
       for (int k = 0; k < 2; k++) { dev_free(N.d_inf[k]); N.d_inf[k] = nullptr; }
@@ -616,6 +621,20 @@ bool ensure_fields(int nb = 1)
    ok = ok && N.d_tmp && N.d_inf[0] && N.d_inf[1] && N.d_u16;
    if (ok) N.nbatch = nb;
    return ok;
+}
+
+// activations of as many of n samples as there is memory for; their number, 0
+// (an error) if there is none for one
+int ensure_batch(int n)
+{
+   int B = batch_size(n);
+   while (!ensure_fields(B))
+   {
+      if (B == 1) return 0;
+      B /= 2;
+      N.cap = B;
+   }
+   return B;
 }
 
 template <int CI, int CO> void launch_layer(const Batch &bt, int n, const __bf16 *wp)
@@ -721,17 +740,19 @@ void backward(int n, const float2 *const *in, float2 *const *g)
 
 constexpr int LNB = 256;  // work-groups of a sample's loss
 
-// mean loss over the samples; gradients of the mean loss in d_g
-double loss_and_grad(int n, float2 *const *r, float2 *const *e)
+// mean loss over the samples; gradients of the mean loss in d_g; false if
+// there is no memory for the activations
+bool loss_and_grad(int n, float2 *const *r, float2 *const *e, double &loss)
 {
    Lib &L = lib();
    const int nu = (int)units_for(L.g.V, 12);
-   const int B = batch_size(n);
-   if (!ensure_fields(B)) return 0.0;
+   const int B = ensure_batch(n);
+   loss = 0.0;
+   if (!B) return false;
    HIP_OK(hipMemsetAsync(N.d_g, 0, nweights() * sizeof(float2), L.stream));
-   double loss = 0.0;
    float2 *out[NBMAX];
-   for (int k = 0; k < B; k++) out[k] = sample(N.d_out, k, 12);
+   // the buffer that the first backward step does not write
+   for (int k = 0; k < B; k++) out[k] = sample(N.d_gb[N.nl & 1], k, 12);
    for (int k0 = 0; k0 < n; k0 += B)
    {
       const int m = std::min(B, n - k0);
@@ -742,16 +763,16 @@ double loss_and_grad(int n, float2 *const *r, float2 *const *e)
          bt.in[k] = e[k0 + k];
          bt.out[k] = out[k];
       }
-      k_ptc_loss<<<dim3(LNB, m), 256, 0, L.stream>>>(bt, nu, N.d_lpart);
+      k_ptc_loss<<<dim3(LNB, m), 256, 0, L.stream>>>(bt, L.g.V, nu, N.d_lpart);
       k_ptc_loss_sum<<<m, 64, 0, L.stream>>>(N.d_lpart, LNB, N.d_lsum);
-      k_ptc_lgrad<<<dim3((nu + 255) / 256, m), 256, 0, L.stream>>>(bt, N.d_lsum, n, nu);
+      k_ptc_lgrad<<<dim3((nu + 255) / 256, m), 256, 0, L.stream>>>(bt, N.d_lsum, n, L.g.V, nu);
       backward(m, r + k0, out);
       HIP_OK(hipMemcpyAsync(N.h_lsum, N.d_lsum, 2 * m * sizeof(double), hipMemcpyDeviceToHost, L.stream));
       HIP_OK(hipStreamSynchronize(L.stream));
       for (int k = 0; k < m; k++)
          if (N.h_lsum[2 * k] != 0.0) loss += N.h_lsum[2 * k + 1] / N.h_lsum[2 * k] / n;
    }
-   return loss;
+   return true;
 }
 
 bool require_net(const char *where)
@@ -857,7 +878,15 @@ extern "C" int oqh_nn_create(int nlayer, const int *widths)
    }
    N.d_lpart = (double *)dev_alloc(2 * NBMAX * LNB * sizeof(double));
    N.d_lsum = (double *)dev_alloc(2 * NBMAX * sizeof(double));
-   HIP_OK(hipHostMalloc((void **)&N.h_lsum, 2 * NBMAX * sizeof(double), 0));
+   if (hipHostMalloc((void **)&N.h_lsum, 2 * NBMAX * sizeof(double), 0) != hipSuccess) N.h_lsum = nullptr;
+   bool ok = N.d_w && N.d_g && N.d_m && N.d_v && N.d_lpart && N.d_lsum && N.h_lsum;
+   for (int l = 0; l < nlayer; l++) ok = ok && N.d_pf[l] && N.d_pa[l];
+   if (!ok)
+   {
+      free_net();
+      fail("oqh_nn_create", "no memory for the network");
+      return 1;
+   }
    HIP_OK(hipMemset(N.d_w, 0, nw * sizeof(float2)));
    HIP_OK(hipMemset(N.d_m, 0, 2 * nw * sizeof(float)));
    HIP_OK(hipMemset(N.d_v, 0, 2 * nw * sizeof(float)));
@@ -945,7 +974,8 @@ extern "C" double oqh_nn_grad(int n, spinor **r, spinor **e, double *dw)
    if (!require_net(where)) return 0.0;
    std::vector<float2 *> rr, ee;
    if (!fields_of(n, r, rr, where) || !fields_of(n, e, ee, where)) return 0.0;
-   double loss = loss_and_grad(n, rr.data(), ee.data());
+   double loss;
+   if (!loss_and_grad(n, rr.data(), ee.data(), loss)) return 0.0;
    size_t nw = nweights();
    std::vector<float2> h(nw);
    HIP_OK(hipStreamSynchronize(lib().stream));
@@ -965,7 +995,8 @@ extern "C" double oqh_nn_train_step(int n, spinor **r, spinor **e, double lr)
    std::vector<float2 *> rr, ee;
    if (!fields_of(n, r, rr, where) || !fields_of(n, e, ee, where)) return 0.0;
    Lib &L = lib();
-   double loss = loss_and_grad(n, rr.data(), ee.data());
+   double loss;
+   if (!loss_and_grad(n, rr.data(), ee.data(), loss)) return 0.0;
    const float b1 = 0.9f, b2 = 0.999f;
    N.adam_t++;
    const float c1 = 1.0f / (1.0f - powf(b1, (float)N.adam_t)), c2 = 1.0f / (1.0f - powf(b2, (float)N.adam_t));

@@ -30,3 +30,54 @@ def test_flow_in_place(L, bc):
         finally:
             lat.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [(8, 8, 8, 8), (6, 6, 6, 10)])
+def test_training_batch(L):
+    """The weight gradient of eight pairs with workspaces for all of them and
+    for two only (the sums over the pairs are rounded in another order, in FP32),
+    and without the memory for one: then nothing is returned or changed but
+    the error count."""
+    print("L", L, flush=True)
+    widths, n = np.array([4, 16, 12, 4], np.int32), 8
+    rng = np.random.default_rng(4)
+    lat = pyoqh.Lattice(L, None, bc=3)
+    lib = lat.lib
+    try:
+        lib.start_ranlux(0, 3)
+        lib.random_ud()
+        fr, fe = [lat.alloc_s() for _ in range(n)], [lat.alloc_s() for _ in range(n)]
+        for f in fr + fe:
+            lat.put_s(f, rng.standard_normal((lat.V, 24)).astype(np.float32))
+        args = (n, (P * n)(*fr), (P * n)(*fe))
+        w = rng.standard_normal(2 * 9 * (64 + 192 + 48)) * 0.1
+        grads = []
+        for limit in (0, 2 * 400 * (lat.V + 63), 300 * lat.V):  # activations: 384 bytes per point and pair
+            print("limit", limit, flush=True)
+            assert lib.oqh_nn_create(3, widths.ctypes.data_as(P)) == 0
+            assert lib.oqh_nn_nweights() * 2 == w.size
+            lib.oqh_nn_set_weights(w.ctypes.data_as(P))
+            dw = np.full(w.size, 7.0)
+            lib.oqh_set_alloc_max(limit)
+            lib.oqh_set_error_mode(0)
+            loss = [lib.oqh_nn_grad(*args, dw.ctypes.data_as(P)) for _ in range(2)]
+            err = lib.oqh_last_error(None, 0)
+            w1 = np.empty_like(w)
+            if limit == 0 or limit > 400 * lat.V:
+                assert err == 0 and loss[0] == loss[1] > 0.0
+                grads.append((loss[0], dw))
+            else:
+                assert err > 0 and loss == [0.0, 0.0] and (dw == 7.0).all()
+                assert lib.oqh_nn_train_step(*args, 1e-3) == 0.0
+                lib.oqh_nn_get_weights(w1.ctypes.data_as(P))
+                assert np.array_equal(w1, w.astype(np.float32))
+            lib.oqh_last_error(None, 0)
+        (l0, g0), (l1, g1) = grads
+        assert abs(l0 - l1) <= 1e-12 * l0
+        assert np.linalg.norm(g0 - g1) <= 1e-6 * np.linalg.norm(g0)
+    finally:
+        lib.oqh_set_error_mode(1)
+        lib.oqh_set_alloc_max(0)
+        lib.oqh_nn_free()
+        lat.close()
