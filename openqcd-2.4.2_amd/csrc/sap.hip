@@ -2764,7 +2764,7 @@ void sap_cycles(float mu, int isolv, int nmr, int ncy, float2 *psi, float2 *rho,
 
 // ncy Schwarz cycles (FP32) from psi = 0 on n sources at once (n <= 16):
 // psi[k] and rho[k] are full FP32 device fields; each launch takes all
-// sources
+// sources.  False, with nothing done, if the face fields cannot be had.
 bool sap_multi_device(float mu, int isolv, int nmr, int ncy, int n, float2 *const *psi, float2 *const *rho)
 {
    if (n < 1 || n > 16 || !reg_kernel()) return false;
@@ -2773,7 +2773,7 @@ bool sap_multi_device(float mu, int isolv, int nmr, int ncy, int n, float2 *cons
    {
       HIP_OK(hipStreamSynchronize(lib().stream));
       dev_free(G.d_wfm);
-      G.d_wfm = (float2 *)dev_alloc(n * nw * sizeof(float2));
+      G.d_wfm = (float2 *)dev_try_alloc(n * nw * sizeof(float2));
       G.wfm_n = G.d_wfm ? n : 0;
       if (!G.d_wfm) return false;
    }

@@ -514,7 +514,9 @@ extern "C" void sap_gcr_multi(int n, int nkv, int nmx, int istop, double res, do
             pl.push_back(F(S[act[i]].phi[S[act[i]].k]));
             rl.push_back(F(S[act[i]].chi[S[act[i]].k]));
          }
-         sap_multi_device((float)mud, L.sap_isolv, L.sap_nmr, L.sap_ncy, (int)pl.size(), pl.data(), rl.data());
+         if (!sap_multi_device((float)mud, L.sap_isolv, L.sap_nmr, L.sap_ncy, (int)pl.size(), pl.data(), rl.data()))
+            for (size_t i = 0; i < pl.size(); i++)
+               sap_cycles((float)mud, L.sap_isolv, L.sap_nmr, L.sap_ncy, pl[i], rl[i], true, true);
       }
       for (int s : act) diff_s2s(vt, 2, S[s].rho, S[s].chi[S[s].k]);
       // Gram-Schmidt step of every active source, one read-back for all

@@ -81,3 +81,43 @@ def test_training_batch(L):
         lib.oqh_set_alloc_max(0)
         lib.oqh_nn_free()
         lat.close()
+
+
+@pytest.mark.gpu
+def test_solves_together():
+    """Several solves without the face fields of several sources (96 bytes per
+    point and source): their Schwarz cycles run one after the other, with the
+    same arithmetic."""
+    n, L, T = 8, (16, 8, 8, 8), (8, 8, 8, 8)
+    o, eta, _ = make_oracle(L, T, bc=3, m0=-0.1, csw=1.77, seed=5)
+    lat = pyoqh.Lattice(L, T, bc=3, m0=-0.1, csw=1.77)
+    try:
+        lib, V = lat.lib, lat.V
+        lat.import_ud(o.ud())
+        assert lat.sw_term(3) == 0
+        lib.oqh_set_sap_parms((C.c_int * 4)(4, 4, 4, 4), 1, 4, 5)
+        rng = np.random.default_rng(2)
+        src, sol = [lat.alloc_sd() for _ in range(n)], [lat.alloc_sd() for _ in range(n)]
+        for f in src:
+            lat.put_sd(f, rng.standard_normal((V, 24)))
+        out = []
+        # dirty Krylov vectors: nothing may be taken from them
+        lib.reserve_ws.restype = C.POINTER(P)
+        lib.alloc_ws(17 * n)
+        ws = lib.reserve_ws(17 * n)
+        for k in range(17 * n):
+            lat.put_s(P(ws[k]), np.full((V, 24), np.nan, np.float32))
+        lib.release_ws()
+        for limit in (n * 96 * V - 1, 0):
+            print("limit", limit, flush=True)
+            lib.oqh_set_alloc_max(limit)
+            rho, ifail, status = (C.c_double * n)(), (C.c_int * n)(), (C.c_int * n)()
+            lib.sap_gcr_multi(n, 8, 128, 0, 1e-10, 0.0, (P * n)(*src), (P * n)(*sol), rho, ifail, status)
+            assert not any(ifail)
+            out.append((list(status), [lat.get_sd(f) for f in sol]))
+        assert out[0][0] == out[1][0]
+        for a, b in zip(out[0][1], out[1][1]):
+            assert np.array_equal(a, b)
+    finally:
+        lib.oqh_set_alloc_max(0)
+        lat.close()
