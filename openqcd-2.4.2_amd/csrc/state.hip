@@ -223,7 +223,11 @@ static void host_copy(bool in, void *dev, void *host, size_t bytes)
       }
    }
    if (in)
+   {
       HIP_OK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, L.stream));
+      // from pinned memory the transfer may still be to come
+      if (!plain) HIP_OK(hipStreamSynchronize(L.stream));
+   }
    else
    {
       HIP_OK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, L.stream));
