@@ -263,7 +263,8 @@ __global__ void k_ptc_pack(const float2 *w, int ci, int co, int adj, __bf16 *wp)
    }
 }
 
-// Partial weight gradients: part[b][p][o][i] for the point sets b.
+// Partial weight gradients: part[b][p][o][i] for the point sets b; nothing is
+// taken from a sample without target (sums, k_ptc_loss_sum).
 //
 // With real and imaginary parts as rows the products sum_x g(x) conj(t(x))^T
 // are real GEMMs [2 C_out x K] x [K x 2 C_in], K = 3 colours x 128 points, on
@@ -284,7 +285,8 @@ constexpr int WG_KSPLIT(int ci, int co) { return 4 / WG_TILES(ci, co); }  // poi
 
 template <int CI, int CO>
 __global__ __launch_bounds__(PWG) __attribute__((amdgpu_waves_per_eu(2))) void k_ptc_wgrad(Batch bt, const float2 *__restrict__ u,
-                                                   const int *__restrict__ nbr, int V, float2 *part)
+                                                   const int *__restrict__ nbr, int V, const double *__restrict__ sums,
+                                                   float2 *part)
 {
    const float2 *__restrict__ in = (const float2 *)bt.in[blockIdx.y];
    const float2 *__restrict__ g = (const float2 *)bt.out[blockIdx.y];  // output gradients
@@ -301,9 +303,10 @@ __global__ __launch_bounds__(PWG) __attribute__((amdgpu_waves_per_eu(2))) void k
    const int row = lane & 15, kk = lane >> 4;
    const int s = t & (PNS - 1), hh = t >> 7;
    const int x = x0 + s;
+   const bool live = x < V && sums[2 * blockIdx.y] != 0.0;
    for (int e = t; e < 3 * PNS * LD; e += PWG) (&T[0][0])[e] = 0.0f;
    __syncthreads();
-   if (x < V)
+   if (live)
       for (int c = hh; c < 3 * CO; c += 2)
       {
          const float2 v = g[unit_index(x, c, 3 * CO)];
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(PWG) __attribute__((amdgpu_waves_per_eu(2))) void k
    int yn = x;  // neighbour of the next direction, one step ahead
    for (int p = 0; p < NDIR; p++)
    {
-      if (x < V)
+      if (live)
       {
          const int y = yn;
          if (p + 1 < NDIR) yn = ptc_nbr(nbr, V, x, p + 1);
@@ -482,9 +485,10 @@ __global__ void k_ptc_lgrad(Batch bt, const double *sums, int npair, int V, int 
    const float2 *e = (const float2 *)bt.in[blockIdx.y];
    float2 *g = (float2 *)bt.out[blockIdx.y];
    const double se = sums[2 * blockIdx.y];
-   const float c = se > 0.0 ? (float)(2.0 / (se * npair)) : 0.0f;
+   const float c = (float)(2.0 / (se * npair));
    const int k = blockIdx.x * 256 + threadIdx.x;
-   if (k < n && unit_point(k) < V) g[k] = make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y));
+   if (k >= n || unit_point(k) >= V) return;
+   g[k] = se != 0.0 ? make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y)) : make_float2(0.0f, 0.0f);
 }
 
 // Adam step on n reals
@@ -669,7 +673,7 @@ template <int CI, int CO> void launch_wgrad(const Batch &bt, int n)
 {
    Lib &L = lib();
    const int V = L.g.V, nb = (V + PNS - 1) / PNS;
-   k_ptc_wgrad<CI, CO><<<dim3(nb, n), PWG, 0, L.stream>>>(bt, L.d_u, L.d_nbr, V, N.d_part);
+   k_ptc_wgrad<CI, CO><<<dim3(nb, n), PWG, 0, L.stream>>>(bt, L.d_u, L.d_nbr, V, N.d_lsum, N.d_part);
 }
 
 #define OQH_PTC_DISPATCH(F, ci, co, ...)                                             \

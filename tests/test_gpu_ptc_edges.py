@@ -82,3 +82,34 @@ def test_weight_gradient(widths, n, tol):
     finally:
         lat.lib.oqh_nn_free()
         lat.close()
+
+
+@pytest.mark.gpu
+def test_pair_without_target():
+    """A pair whose target vanishes counts nothing, whatever its input holds."""
+    L, n, widths = (8, 8, 8, 8), 3, np.array([4, 8, 4], np.int32)
+    rng = np.random.default_rng(5)
+    lat = pyoqh.Lattice(L, None, bc=3)
+    try:
+        lib = lat.lib
+        lib.start_ranlux(0, 4)
+        lib.random_ud()
+        assert lib.oqh_nn_create(2, widths.ctypes.data_as(P)) == 0
+        w = 0.1 * rng.standard_normal(2 * lib.oqh_nn_nweights())
+        lib.oqh_nn_set_weights(w.ctypes.data_as(P))
+        fr, fe = [lat.alloc_s() for _ in range(n)], [lat.alloc_s() for _ in range(n)]
+        for f in fr + fe:
+            lat.put_s(f, rng.standard_normal((lat.V, 24)).astype(np.float32))
+        lat.put_s(fe[1], np.zeros((lat.V, 24), np.float32))
+        out = []
+        for x in (0.5, np.inf, np.nan):
+            print("input", x, flush=True)
+            lat.put_s(fr[1], np.full((lat.V, 24), x, np.float32))
+            dw = np.empty_like(w)
+            loss = lib.oqh_nn_grad(n, ptrs(fr), ptrs(fe), dw.ctypes.data_as(P))
+            out.append((loss, dw))
+        for loss, dw in out:
+            assert np.isfinite(dw).all() and loss == out[0][0] and np.array_equal(dw, out[0][1])
+    finally:
+        lat.lib.oqh_nn_free()
+        lat.close()
