@@ -418,9 +418,12 @@ __global__ __launch_bounds__(64 * WSW) void k_ptc_wgrad_sum(const float2 *part, 
    grad[e].y += (float)zi;
 }
 
-// point of a unit of a spinor field; the last storage block may have more
-// than the lattice
-__device__ inline int unit_point(int k) { return k / (12 * SB) * SB + (k & (SB - 1)); }
+// whether unit k of a spinor field belongs to a point: the last storage block
+// may have more than the lattice
+__device__ inline bool unit_used(int k, int V)
+{
+   return V % SB == 0 || k / (12 * SB) * SB + (k & (SB - 1)) < V;
+}
 
 // loss terms of a sample (blockIdx.y): partial sums of |e|^2 and |out - e|^2
 __global__ void k_ptc_loss(Batch bt, int V, int n, double *part)
@@ -428,14 +431,18 @@ __global__ void k_ptc_loss(Batch bt, int V, int n, double *part)
    const float2 *out = (const float2 *)bt.out[blockIdx.y], *e = (const float2 *)bt.in[blockIdx.y];
    __shared__ double sh[2][256];
    double se = 0.0, sd = 0.0;
-   for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256)
+   auto add = [&](int k)
    {
-      if (unit_point(k) >= V) continue;
       float2 a = out[k], b = e[k];
       double dx = (double)a.x - b.x, dy = (double)a.y - b.y;
       se += (double)b.x * b.x + (double)b.y * b.y;
       sd += dx * dx + dy * dy;
-   }
+   };
+   const int full = V / SB * (12 * SB);  // units of full storage blocks
+   int k = blockIdx.x * 256 + threadIdx.x;
+   for (; k < full; k += gridDim.x * 256) add(k);
+   for (; k < n; k += gridDim.x * 256)
+      if (unit_used(k, V)) add(k);
    sh[0][threadIdx.x] = se;
    sh[1][threadIdx.x] = sd;
    __syncthreads();
@@ -487,7 +494,7 @@ __global__ void k_ptc_lgrad(Batch bt, const double *sums, int npair, int V, int 
    const double se = sums[2 * blockIdx.y];
    const float c = (float)(2.0 / (se * npair));
    const int k = blockIdx.x * 256 + threadIdx.x;
-   if (k >= n || unit_point(k) >= V) return;
+   if (k >= n || !unit_used(k, V)) return;
    g[k] = se != 0.0 ? make_float2(c * (g[k].x - e[k].x), c * (g[k].y - e[k].y)) : make_float2(0.0f, 0.0f);
 }
 
