@@ -269,7 +269,7 @@ int oqh_link_rebuild(double *dev);
 double oqh_time_dirac(int op, double mu, void *s, void *r, int ncall);
 /* Dw_dble / Dw applied to n fields at once, r[k] = D s[k] (no counterpart in
    the reference: a batched form of dirac/Dw_dble.c:1377 and dirac/Dw.c:973
-   that loads every link and Pauli matrix once for up to 8 fields).  The
+   whose work-groups share every link and Pauli matrix among up to 4 fields).  The
    fields must be full device fields of the library and s[k] != r[k]; unlike
    Dw_dble, the inputs are left unchanged on the boundary points of open bc. */
 void oqh_Dw_dble_multi(double mu, int n, spinor_dble **s, spinor_dble **r);

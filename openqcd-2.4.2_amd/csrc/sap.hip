@@ -1056,13 +1056,15 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
       }
       else
       {
-         zero12(w);
+         float2 o[12];
+         pauli_reg2(mp0, mst0, mp1, mst1, even ? a.mu : a.muo, s1, o);
+         // the accumulators start from -2 A s1, so that w = -1/2 their sum
+#pragma unroll
+         for (int c = 0; c < 12; c++) w[c] = cscale(o[c], -2.0f);
          rb_hop<1>(b, s1, w, LB);
          rb_hop<0>(b, s1, w, LB);
 #pragma unroll
-         for (int c = 0; c < 12; c++) w[c] = cscale(w[c], -0.5f);
-         pauli_reg2<true>(mp0, mst0, mp1, mst1, even ? a.mu : a.muo, s1, w);
-         if (b.bp) zero12(w);
+         for (int c = 0; c < 12; c++) w[c] = b.bp ? zero : cscale(w[c], -0.5f);
       }
       double rr, zr, zi;
       rb_sums(ISOLV ? even : true, w, s1, sh, rr, zr, zi);
@@ -1138,7 +1140,8 @@ void k_sap_reg(SArgs a0, const S *u16, const S *sw16)
 }
 
 // rho += hopping terms from the face fields of the neighbouring blocks for
-// the 4^4 blocks or sub-blocks (points imb) from n0 on: completes the residual after the last block solves
+// the 4^4 blocks or sub-blocks (points imb) from n0 on: completes the residual
+// after the last block solves
 template <typename S>
 __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const int *imb, const S *u16)
 {
@@ -1200,10 +1203,11 @@ __global__ __launch_bounds__(RBV) void k_sap_complete(SArgs a0, const int *imb, 
 // exchange buffers alternate: who writes the one of pass k + 2 has seen
 // everybody arrive in pass k + 1, that is, done with reading pass k.
 //
-// Per cycle (us, nmr = 4; k_sap_cluster / k_sap_lds or, for 8^4, k_sap_blocks):
-// 8^4 blocks on 16^4 213 / 1436, on 32^4 1100 / 2605, on 32^3x64 2190 / 3700;
-// 8x4^3 on 16x8^3 132 / 146, on 32^3x16 388 / 446; 8^2x4^2 on 16^2x8^2 149 /
-// 203, on 32^3x16 436 / 463.  Bound by the 14 exchanges of a block solve, about
+// Per cycle (us, isolv = 1, nmr = 4; k_sap_cluster / k_sap_lds or, for 8^4,
+// k_sap_blocks): 8^4 blocks on 16^4 213 / 1436, on 32^4 1090 / 2605, on 32^3x64
+// 2150 / 3700; 16x8^3 on 32x16^3 251 / 3050; 8x4^3 on 16x8^3 132 / 146, on 32^3x16
+// 384 / 446; 8^2x4^2 on 16^2x8^2 153 / 203, on 32^3x16 430 / 463 (a call of sap()
+// takes 8 more, for its wait).  Bound by the 14 exchanges of a block solve, about
 // 3.5 us each (write, count, poll, read).  With the counters of all blocks in
 // one line they took 20 us (8^4 on 32^4: 3400).
 // ---------------------------------------------------------------------------
@@ -1541,6 +1545,10 @@ __global__ __launch_bounds__(RBV) __attribute__((amdgpu_waves_per_eu(2))) void k
       }
       else
       {
+         // unlike in k_sap_reg the hops are summed by themselves, which is more
+         // precise than k_sap_blocks was (five cycles of 8^4 blocks on 16^4
+         // against FP64: 1.09e-7 for 1.16e-7; started from -2 A s1 1.20e-7) and
+         // costs 3 % of a cycle
          zero12(w);
          cl_hop<1>(q, st, b, nb, s1, w, LB);
          cl_hop<0>(q, st, b, nb, s1, w, LB);
@@ -1854,7 +1862,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(TPB <= 512 
 
 // rho(y) -= hopping terms into y from the block corrections of the
 // neighbouring blocks, for the face points y of the blocks of one colour
-// (block sizes other than 4^4)
+// (the blocks of k_sap_lds and k_sap_blocks)
 __global__ __launch_bounds__(256) void k_sap_faces(SArgs a, const int *face, const unsigned char *fmask, int nf)
 {
    int k = blockIdx.x * 256 + threadIdx.x;
@@ -2544,7 +2552,7 @@ static void sap_blocks(const SArgs &a0, int ic, int isolv, int pull)
 }
 
 // face terms from the corrections of the colour-(1-c) blocks into rho on
-// the faces of the colour-c blocks (block sizes other than 4^4)
+// the faces of the colour-c blocks (those of k_sap_lds and k_sap_blocks)
 static void sap_push_faces(const SArgs &a, int c)
 {
    if (!G.nface[c]) return;
