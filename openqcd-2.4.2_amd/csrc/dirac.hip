@@ -752,7 +752,7 @@ template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(
 // itself only, so there are no barriers.
 // 12 fields FP64 at 24^4: 0.83 ms with W = 4, TP = 64, against 1.11 ms with 8
 // lanes per pair of points, 256-lane work-groups and barriers.  Bound by the
-// 4.9 GB that miss the L2 (the neighbours in x2 and x3 lie four to eight lines
+// 5.1 GB that miss the L2 (the neighbours in x2 and x3 lie four to eight lines
 // apart).  All tiles of a thread block for four fields before the next four:
 // 0.90 ms; third link rows rebuilt and the S-form of the SW term, as Dw_dble
 // has them: 0.80 ms, but twice the rounding error (3e-16 for 1.3e-16), so the

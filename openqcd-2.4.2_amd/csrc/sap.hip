@@ -23,11 +23,13 @@
 //
 // The reference computes the hopping terms from each block across its faces
 // (Dw_bnd) and subtracts them from the residual of the neighbouring blocks
-// after all blocks of the colour are done (sap_com).  Here the block
-// corrections s0 are written to a global field and a second kernel gathers,
-// for every face point of the blocks of the other colour, the hopping terms
-// from its neighbours in other blocks, so that no point is updated by two
-// work-items.
+// after all blocks of the colour are done (sap_com).  k_sap_reg and
+// k_sap_cluster write these terms as Weyl fields on the faces of their blocks and
+// add those of the other colour at the start of a solve.  k_sap_lds and
+// k_sap_blocks write the block corrections s0 to a global field and a second
+// kernel gathers, for every face point of the blocks of the other colour, the
+// hopping terms from its neighbours in other blocks, so that no point is updated
+// by two work-items.
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -42,7 +44,7 @@
 namespace oqh {
 
 constexpr int SWG = 256;      // work-group size of the block kernels
-constexpr int SWG_MAX = 1024; // work-group size of the generic FP32 block solver for blocks of >= 1024 points
+constexpr int SWG_MAX = 1024; // work-group size of the generic FP32 block solver
 constexpr int NBF = 4;    // block fields of the API per block: s[0..2] + the Dwhat_blk intermediate
 #ifndef OQH_SAP_REG
 #define OQH_SAP_REG 1
@@ -604,25 +606,35 @@ template <typename S> struct RegBlock
 
 // o = (A + i mu) w (ADD: added to o) on one Weyl half (pauli_half), the 18
 // units of A in q.
-// The diagonal term, by far the largest, comes last: each term of a chain of
-// fused operations is rounded at the size of the sum so far.  Five cycles of
-// 8^4 blocks on 16^4, isolv = 1, against FP64: 1.15e-7 (solution) and 3.2e-7
+// LAST: the diagonal term, by far the largest, comes last, for each term of a
+// chain of fused operations is rounded at the size of the sum so far.  Five cycles
+// of 8^4 blocks on 16^4, isolv = 1, against FP64: 1.15e-7 (solution) and 3.2e-7
 // (residual), with the diagonal first 1.47e-7 and 3.9e-7, with the separate
-// products of k_sap_blocks 1.21e-7 and 3.4e-7; the time is the same.
-template <bool ADD = false>
+// products of k_sap_blocks 1.21e-7 and 3.4e-7; the time is the same.  With FP16
+// storage (errors of 1e-4) the diagonal comes first, which takes 1.5 us less of a
+// cycle of 82 at 16^4 (isolv = 0).
+template <bool ADD = false, bool LAST = true>
 __device__ inline void pauli_half_reg(const float2 *q, float mu, const float2 *w, float2 *o)
 {
+   static_assert(LAST || !ADD, "the diagonal starts the sum");
    float d[6] = {q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y};
+   if (!LAST)
+   {
+#pragma unroll
+      for (int i = 0; i < 6; i++) o[i] = make_float2(d[i] * w[i].x - mu * w[i].y, d[i] * w[i].y + mu * w[i].x);
+   }
+   constexpr bool FRESH = LAST && !ADD;
    int p = 3;
 #pragma unroll
    for (int i = 0; i < 6; i++)
 #pragma unroll
       for (int j = i + 1; j < 6; j++)
       {
-         o[i] = (!ADD && i == 0 && j == 1) ? cmul(q[p], w[j]) : cmac(o[i], q[p], w[j]);
-         o[j] = (!ADD && i == 0) ? cmulc(q[p], w[i]) : cmacc(o[j], q[p], w[i]);
+         o[i] = (FRESH && i == 0 && j == 1) ? cmul(q[p], w[j]) : cmac(o[i], q[p], w[j]);
+         o[j] = (FRESH && i == 0) ? cmulc(q[p], w[i]) : cmacc(o[j], q[p], w[i]);
          p++;
       }
+   if (!LAST) return;
 #pragma unroll
    for (int i = 0; i < 6; i++)
       o[i] = make_float2(fmaf(d[i], w[i].x, fmaf(-mu, w[i].y, o[i].x)), fmaf(d[i], w[i].y, fmaf(mu, w[i].x, o[i].y)));
@@ -641,7 +653,7 @@ __device__ inline void pauli_reg2(const S *m0, int st0, const S *m1, int st1, fl
       const int stride = hh ? st1 : st0;
 #pragma unroll
       for (int k = 0; k < 18; k++) q[k] = to_f2(m[k * stride]);
-      pauli_half_reg<ADD>(q, hh ? -mu : mu, v + 6 * hh, out + 6 * hh);
+      pauli_half_reg<ADD, sizeof(S) == sizeof(float2)>(q, hh ? -mu : mu, v + 6 * hh, out + 6 * hh);
    }
 }
 
