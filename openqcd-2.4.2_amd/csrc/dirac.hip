@@ -717,8 +717,8 @@ template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(
    {
       const int i = 2 * wr + r;
       // the diagonal term, the largest, last, for each sum is rounded at its
-      // size (FP32 Dw, Dwhat at 16^4, m0 = -0.3, against FP64 6.3e-8, 6.0e-8;
-      // with the diagonal in its place 7.4e-8, 7.4e-8; the tiles 6.8e-8, 7.2e-8)
+      // size (FP32 Dw, Dwhat at 16^4, m0 = -0.3, against FP64 5.8e-8, 5.3e-8;
+      // with the diagonal in its place 7.4e-8, 7.4e-8; the tiles 6.7e-8, 7.0e-8)
       C o = hs[r], vd = v[0];
       T d = 0;
 #pragma unroll
@@ -732,7 +732,7 @@ template <typename T, int OP> __global__ __launch_bounds__(8 * SB) void k_split(
          else
             o = cadd(o, i < j ? cmul(m[r][j], v[j]) : cmulc(m[r][j], v[j]));
       }
-      out[r] = cadd(o, cmk<C>(d * vd.x - mu * vd.y, d * vd.y + mu * vd.x));
+      out[r] = cmk<C>(fma(d, vd.x, fma(-mu, vd.y, o.x)), fma(d, vd.y, fma(mu, vd.x, o.y)));
    }
    // boundary points of open bc are zeroed in output and (Dw) input
    if (bp) out[0] = out[1] = cmk<C>(0, 0);
